@@ -259,21 +259,22 @@ __device__ inline void dp_project(float *state, const float4 hp, float lambda, f
 // Refined variants of the SVD-dependent steps. In FP32, F - R and log(sigma)
 // near sigma = 1 lose ~5 digits to cancellation, which is the size of the parity
 // tolerance. Here the quantities that cancel are computed to FP64 accuracy: the
-// polar rotation R by FP64 Newton iterations from F; the singular values as
-// |F v_i| / |v_i| in FP64 from the FP32 SVD's right singular vectors (the error
-// is second order in theirs); log(sigma) and exp of the small log-strain
-// corrections through log1p / expm1 of FP64 differences from 1.
+// polar rotation R by FP64 Newton iterations from F; the log strains and the
+// principal directions from the eigen-decomposition of F^T F - I.
+
 // Orthogonal polar factor r of a (a = r s, s symmetric positive definite) by
 // Newton's iteration x <- (g x + x^-T / g) / 2 with determinant scaling
 // g = det(x)^(-1/3) while det(x) is far from 1 (N. J. Higham, "Computing the
 // polar decomposition -- with applications", SIAM J. Sci. Stat. Comput. 7(4),
 // 1986). For det(a) > 0 this is U V^T of the SVD a = U diag(sig) V^T. Returns
 // false (r undefined) if det(a) <= 0 or it does not converge.
-__device__ inline bool polar_f64(const double *a, double *r) {
-    double x[9];
+//
+// Convergence is quadratic: a step of size d leaves an error of about d^2 / 2
+// (d per entry: at most 9/2 d^2 in norm), so the step that is below 3e-8 is the
+// last one (4e-15). Strains of 1e-4 to 1e-2 take 2 to 3 iterations.
+__device__ inline bool polar_f64(const float *a, double *x) {
 #pragma unroll
     for (int k = 0; k < 9; k++) x[k] = a[k];
-    bool close = false;
 #pragma unroll 1
     for (int it = 0; it < 24; it++) {
         double c[9];
@@ -289,7 +290,7 @@ __device__ inline bool polar_f64(const double *a, double *r) {
         const double det = x[0] * c[0] + x[1] * c[1] + x[2] * c[2];
         if (!(det > 0.0)) return false;
         // Any positive scale keeps the iteration convergent; FP32 is enough for it.
-        const double g = fabs(det - 1.0) > 1.0e-3 ? (double)(1.0f / cbrtf((float)det)) : 1.0;
+        const double g = fabs(det - 1.0) > 0.05 ? (double)(1.0f / cbrtf((float)det)) : 1.0;
         const double h = 0.5 / (g * det);
         double diff = 0.0, norm = 0.0;
 #pragma unroll
@@ -299,224 +300,227 @@ __device__ inline bool polar_f64(const double *a, double *r) {
             norm = fmax(norm, fabs(nx));
             x[k] = nx;
         }
-        // Quadratic convergence: once a step is below 1e-9 the next one is at round-off.
-        if (close) {
-#pragma unroll
-            for (int k = 0; k < 9; k++) r[k] = x[k];
-            return true;
-        }
-        close = diff <= 1.0e-9 * norm;
+        if (diff <= 3.0e-8 * norm) return true;
     }
     return false;
 }
 
-__device__ inline double det3d(const double *a) {
-    return a[0] * (a[4] * a[8] - a[5] * a[7]) - a[1] * (a[3] * a[8] - a[5] * a[6]) + a[2] * (a[3] * a[7] - a[4] * a[6]);
+// One Jacobi rotation in the (p, q) plane of a symmetric 3x3 matrix (its entries
+// pp, qq, pq and the third row's rp, rq) and of the columns p, q of v. The angle
+// only has to be near the one that annihilates pq (the sweeps converge all the
+// same), so its tangent comes from FP32 approximations; the cosine is then
+// corrected to FP64 by a Newton step, which keeps the rotation orthonormal.
+__device__ inline void jacobi_rotate(double &pp, double &qq, double &pq, double &rp, double &rq, double *v, int p, int q) {
+    const float d = (float)(qq - pp), b = 2.0f * (float)pq;
+    const float den = fabsf(d) + __builtin_amdgcn_sqrtf(d * d + b * b);
+    const float tf = den > 0.0f ? (d < 0.0f ? -b : b) * __builtin_amdgcn_rcpf(den) : 0.0f;
+    const double t = tf, w = 1.0 + t * t;
+    const double c0 = __builtin_amdgcn_rsqf((float)w);
+    const double c = c0 * (1.5 - 0.5 * w * c0 * c0), s = t * c;
+    const double cc = c * c, ss = s * s, cs = c * s, x = 2.0 * cs * pq, npp = cc * pp - x + ss * qq, nqq = ss * pp + x + cc * qq;
+    pq = (cc - ss) * pq + cs * (pp - qq);
+    pp = npp;
+    qq = nqq;
+    const double nrp = c * rp - s * rq;
+    rq = s * rp + c * rq;
+    rp = nrp;
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        const double a = v[k * 3 + p], z = v[k * 3 + q];
+        v[k * 3 + p] = c * a - s * z;
+        v[k * 3 + q] = s * a + c * z;
+    }
+}
+
+// Eigenvalues (less 1, in e) and eigenvectors (the columns of v, a rotation) of
+// F^T F by cyclic Jacobi sweeps.
+__device__ inline void eigen_f64(const float *f32, double *e, double *v) {
+    double e00, e11, e22, e01, e02, e12;
+    {
+        // The products are exact in FP64, the sums lose only FP64 round-off.
+        double f[9];
+#pragma unroll
+        for (int k = 0; k < 9; k++) f[k] = f32[k];
+        e00 = f[0] * f[0] + f[3] * f[3] + f[6] * f[6] - 1.0;
+        e11 = f[1] * f[1] + f[4] * f[4] + f[7] * f[7] - 1.0;
+        e22 = f[2] * f[2] + f[5] * f[5] + f[8] * f[8] - 1.0;
+        e01 = f[0] * f[1] + f[3] * f[4] + f[6] * f[7];
+        e02 = f[0] * f[2] + f[3] * f[5] + f[6] * f[8];
+        e12 = f[1] * f[2] + f[4] * f[5] + f[7] * f[8];
+    }
+#pragma unroll
+    for (int k = 0; k < 9; k++) v[k] = k % 4 == 0 ? 1.0 : 0.0;
+#pragma unroll 1
+    for (int sweep = 0; sweep < 12; sweep++) {
+        const double off = e01 * e01 + e02 * e02 + e12 * e12;
+        const double dg = (1.0 + e00) * (1.0 + e00) + (1.0 + e11) * (1.0 + e11) + (1.0 + e22) * (1.0 + e22);
+        if (!(off > 1.0e-30 * dg)) break;
+        jacobi_rotate(e00, e11, e01, e02, e12, v, 0, 1);
+        jacobi_rotate(e00, e22, e02, e01, e12, v, 0, 2);
+        jacobi_rotate(e11, e22, e12, e01, e02, v, 1, 2);
+    }
+    e[0] = e00;
+    e[1] = e11;
+    e[2] = e22;
+}
+
+__device__ inline double det3d(const float *a) {
+    const double x[9] = {a[0], a[1], a[2], a[3], a[4], a[5], a[6], a[7], a[8]};
+    return x[0] * (x[4] * x[8] - x[5] * x[7]) - x[1] * (x[3] * x[8] - x[5] * x[6]) + x[2] * (x[3] * x[7] - x[4] * x[6]);
+}
+
+// U V^T of the SVD with U and V rotations, for an F with det F <= 0 or so close
+// to singular that polar_f64 fails (such a particle is disabled unless its FP32
+// determinant rounds to a positive value): the two larger singular values give
+// their left vectors, the third is their cross product.
+__device__ inline void rotation_by_eigen(const float *f, double *r) {
+    double e[3], v[9];
+    eigen_f64(f, e, v);
+    // The column of the smallest eigenvalue goes last (cyclically: v stays a rotation).
+#pragma unroll 1
+    for (int turn = 0; turn < 2 && (e[0] < e[2] || e[1] < e[2]); turn++) {
+        const double t = e[0];
+        e[0] = e[1];
+        e[1] = e[2];
+        e[2] = t;
+#pragma unroll
+        for (int k = 0; k < 3; k++) {
+            const double w = v[3 * k];
+            v[3 * k] = v[3 * k + 1];
+            v[3 * k + 1] = v[3 * k + 2];
+            v[3 * k + 2] = w;
+        }
+    }
+    double u[2][3];
+#pragma unroll
+    for (int j = 0; j < 2; j++) {
+        const double w = 1.0 / sqrt(1.0 + e[j]);
+#pragma unroll
+        for (int i = 0; i < 3; i++) u[j][i] = w * ((double)f[3 * i] * v[j] + (double)f[3 * i + 1] * v[3 + j] + (double)f[3 * i + 2] * v[6 + j]);
+    }
+    const double c[3] = {u[0][1] * u[1][2] - u[0][2] * u[1][1], u[0][2] * u[1][0] - u[0][0] * u[1][2],
+                         u[0][0] * u[1][1] - u[0][1] * u[1][0]};
+#pragma unroll
+    for (int i = 0; i < 3; i++)
+#pragma unroll
+        for (int j = 0; j < 3; j++) r[3 * i + j] = u[0][i] * v[3 * j] + u[1][i] * v[3 * j + 1] + c[i] * v[3 * j + 2];
 }
 
 // linear_elasticity.slang:135-148 in FP64: tau = 2 mu (F - R) F^T + lambda (J - 1) J I
-// with R the polar rotation (U V^T of the SVD), J = det F.
+// with R the polar rotation (U V^T of the SVD), J = det F. tau is symmetric: six entries.
 __device__ inline void fc_stress_f64(float lambda, float mu, const float *f32, float *st) {
-    double f[9], rc[9], j;
-#pragma unroll
-    for (int k = 0; k < 9; k++) f[k] = f32[k];
     double r[9];
-    if (!polar_f64(f, r)) {
-        // det F <= 0 (the particle is disabled by the update) or no convergence.
-        fc_stress(lambda, mu, f32, st);
-        return;
-    }
+    if (!polar_f64(f32, r)) rotation_by_eigen(f32, r);
+    double f[9];
 #pragma unroll
-    for (int k = 0; k < 9; k++) rc[k] = f[k] - r[k];
-    j = det3d(f);
-    const double mu2 = 2.0 * (double)mu;
+    for (int k = 0; k < 9; k++) {
+        f[k] = f32[k];
+        r[k] = f[k] - r[k];
+    }
+    const double j = f[0] * (f[4] * f[8] - f[5] * f[7]) - f[1] * (f[3] * f[8] - f[5] * f[6]) + f[2] * (f[3] * f[7] - f[4] * f[6]);
+    const double mu2 = 2.0 * (double)mu, vol = (double)lambda * (j - 1.0) * j;
 #pragma unroll
     for (int i = 0; i < 3; i++)
 #pragma unroll
-        for (int k = 0; k < 3; k++) {
-            double r2 = mu2 * (f[0 * 3 + i] * rc[0 * 3 + k] + f[1 * 3 + i] * rc[1 * 3 + k] + f[2 * 3 + i] * rc[2 * 3 + k]);
-            if (i == k) r2 += (double)lambda * (j - 1.0) * j;
+        for (int k = i; k < 3; k++) {
+            double r2 = mu2 * (f[0 * 3 + i] * r[0 * 3 + k] + f[1 * 3 + i] * r[1 * 3 + k] + f[2 * 3 + i] * r[2 * 3 + k]);
+            if (i == k) r2 += vol;
             st[i * 3 + k] = (float)r2;
+            if (i != k) st[k * 3 + i] = (float)r2;
         }
 }
 
-// log(x) for x near 1 from the FP64 difference x - 1.
-__device__ inline double log_near1(double x) { return (double)log1pf((float)(x - 1.0)); }
-
-// Right singular vectors of f (the columns of v) to FP64 accuracy from FP32 ones
-// (the columns of v32): one Newton-Schulz step v = w (3 I - w^T w) / 2 makes them
-// orthonormal to FP64 round-off, then cyclic Jacobi sweeps on v^T f^T f v, whose
-// off-diagonal part starts at FP32 round-off, converge quadratically (at most 4
-// sweeps, also for repeated singular values). With FP32 vectors U diag(s') V^T
-// carries ~1e-7 absolute error, which is the size of a plastic F - I step.
-__device__ inline void refine_right_vectors(const double *f, const float *v32, double *v) {
-    double w[9], g[9];
-#pragma unroll
-    for (int k = 0; k < 9; k++) w[k] = v32[k];
-#pragma unroll
-    for (int i = 0; i < 3; i++)
-#pragma unroll
-        for (int j = 0; j < 3; j++) g[i * 3 + j] = w[0 * 3 + i] * w[0 * 3 + j] + w[1 * 3 + i] * w[1 * 3 + j] + w[2 * 3 + i] * w[2 * 3 + j];
-#pragma unroll
-    for (int i = 0; i < 3; i++)
-#pragma unroll
-        for (int j = 0; j < 3; j++)
-            v[i * 3 + j] = 0.5 * (w[i * 3 + 0] * ((j == 0 ? 3.0 : 0.0) - g[0 * 3 + j]) +
-                                  w[i * 3 + 1] * ((j == 1 ? 3.0 : 0.0) - g[1 * 3 + j]) +
-                                  w[i * 3 + 2] * ((j == 2 ? 3.0 : 0.0) - g[2 * 3 + j]));
-    double b[9], a[3][3];
-#pragma unroll
-    for (int i = 0; i < 3; i++)
-#pragma unroll
-        for (int j = 0; j < 3; j++) b[i * 3 + j] = f[i * 3 + 0] * v[0 * 3 + j] + f[i * 3 + 1] * v[1 * 3 + j] + f[i * 3 + 2] * v[2 * 3 + j];
-#pragma unroll
-    for (int i = 0; i < 3; i++)
-#pragma unroll
-        for (int j = 0; j < 3; j++) a[i][j] = b[0 * 3 + i] * b[0 * 3 + j] + b[1 * 3 + i] * b[1 * 3 + j] + b[2 * 3 + i] * b[2 * 3 + j];
-#pragma unroll 1
-    for (int sweep = 0; sweep < 4; sweep++) {
-        const double off = a[0][1] * a[0][1] + a[0][2] * a[0][2] + a[1][2] * a[1][2];
-        const double dg = a[0][0] * a[0][0] + a[1][1] * a[1][1] + a[2][2] * a[2][2];
-        if (!(off > 1.0e-30 * dg)) break;
-#pragma unroll
-        for (int e = 0; e < 3; e++) {
-            const int p = e == 2 ? 1 : 0;
-            const int q = e == 0 ? 1 : 2;
-            const double apq = a[p][q];
-            if (apq == 0.0) continue;
-            const double theta = (a[q][q] - a[p][p]) / (2.0 * apq);
-            const double t = (theta >= 0.0 ? 1.0 : -1.0) / (fabs(theta) + sqrt(theta * theta + 1.0));
-            const double c = 1.0 / sqrt(t * t + 1.0), sn = t * c;
-#pragma unroll
-            for (int k = 0; k < 3; k++) {
-                const double x = a[k][p], y = a[k][q];
-                a[k][p] = c * x - sn * y;
-                a[k][q] = sn * x + c * y;
-            }
-#pragma unroll
-            for (int k = 0; k < 3; k++) {
-                const double x = a[p][k], y = a[q][k];
-                a[p][k] = c * x - sn * y;
-                a[q][k] = sn * x + c * y;
-            }
-#pragma unroll
-            for (int k = 0; k < 3; k++) {
-                const double x = v[k * 3 + p], y = v[k * 3 + q];
-                v[k * 3 + p] = c * x - sn * y;
-                v[k * 3 + q] = sn * x + c * y;
-            }
-        }
+// log(1 + e) / 2, the log of a singular value from the eigenvalue 1 + e of
+// F^T F: atanh(e / (2 + e)) by its series for |e| <= 1/4 (relative error below
+// 1e-10), the library's FP64 function beyond.
+__device__ inline double half_log1p(double e) {
+    if (fabs(e) <= 0.25) {
+        const double r = e / (2.0 + e), q = r * r;
+        return r + r * q * (1.0 / 3.0 + q * (1.0 / 5.0 + q * (1.0 / 7.0 + q * (1.0 / 9.0 + q * (1.0 / 11.0)))));
     }
+    return 0.5 * log1p(e);
+}
+
+// exp(x) - 1: its Taylor series for |x| <= 1/4 (relative error below 1e-11), the
+// library's function beyond.
+__device__ inline double exp_m1(double x) {
+    if (fabs(x) <= 0.25) {
+        double p = 1.0 / 40320.0;
+        p = 1.0 / 5040.0 + x * p;
+        p = 1.0 / 720.0 + x * p;
+        p = 1.0 / 120.0 + x * p;
+        p = 1.0 / 24.0 + x * p;
+        p = 1.0 / 6.0 + x * p;
+        p = 0.5 + x * p;
+        return x + x * x * p;
+    }
+    return expm1(x);
 }
 
 // drucker_prager.slang:144-200 (Klar et al. 2016 return mapping in log-strain
-// space on the singular values), refined as described above.
+// space on the singular values), refined as described above. The projected
+// gradient is U diag(s') V^T = F V diag(s' / s) V^T, so only V and the ratios
+// s' / s - 1 = exp(log s' - log s) - 1 are needed, and F changes by the small
+// product F V diag(s' / s - 1) V^T.
+//
+// VALU-bound: 4 sweeps of 3 rotations (~50 FP64 operations each) take the place
+// of an FP32 SVD, its FP64 refinement and FP32 logarithms (~3000 operations).
 __device__ inline void dp_project_f64(float *state, const float4 hp, float lambda_f, float mu_f, float *f32) {
     if (lambda_f == 0.0f) return;
-    const double lambda = lambda_f, mu = mu_f;
-    float u[9], s32[3], v[9];
-    svd3<float>(f32, u, s32, v);
-    double s[3];
+    if (!(det3d(f32) > 0.0)) {
+        // The log of a singular value that is not positive is NaN, as in the shader;
+        // the particle is disabled by the update.
+        const float nan = __uint_as_float(0x7fc00000u);
+        state[0] = state[1] = state[2] = nan;
 #pragma unroll
-    for (int i = 0; i < 3; i++) {
-        const double v0 = v[0 * 3 + i], v1 = v[1 * 3 + i], v2 = v[2 * 3 + i];
-        const double w0 = (double)f32[0] * v0 + (double)f32[1] * v1 + (double)f32[2] * v2;
-        const double w1 = (double)f32[3] * v0 + (double)f32[4] * v1 + (double)f32[5] * v2;
-        const double w2 = (double)f32[6] * v0 + (double)f32[7] * v1 + (double)f32[8] * v2;
-        s[i] = sqrt((w0 * w0 + w1 * w1 + w2 * w2) / (v0 * v0 + v1 * v1 + v2 * v2));
+        for (int k = 0; k < 9; k++) f32[k] = nan;
+        return;
     }
-    if (s32[2] < 0.0f) s[2] = -s[2];  // svd3 gives sig[2] the sign of det F
+    double e[3], v[9];
+    eigen_f64(f32, e, v);
     const float q = state[1];
     const float angle = hp.x + (hp.y * q - hp.w) * expf(-hp.z * q);
     const float sa = sinf(angle);
     const double alpha = (double)(sqrtf(2.0f / 3.0f) * (2.0f * sa) / (3.0f - sa));
-    const double d = 3.0;
-    double strain[3], dev[3], ns[3], hard;
+    const double lambda = lambda_f, mu = mu_f, third = (double)state[2] / 3.0;
+    const double raw[3] = {half_log1p(e[0]), half_log1p(e[1]), half_log1p(e[2])};
+    double dev[3];
+    const double tr = raw[0] + raw[1] + raw[2] + 3.0 * third;
 #pragma unroll
-    for (int i = 0; i < 3; i++) strain[i] = log_near1(s[i]) + (double)state[2] / d;
-    double tr = strain[0] + strain[1] + strain[2];
+    for (int i = 0; i < 3; i++) dev[i] = raw[i] + third - tr / 3.0;
+    // Tension (s' = 1: F becomes its polar rotation) or the projection onto the cone,
+    // selected without branches: one gave a wrong register to the lanes that reach
+    // the first case through its second condition.
+    const bool tension = (tr > 0.0) | ((dev[0] == 0.0) & (dev[1] == 0.0) & (dev[2] == 0.0));
+    const double dn = sqrt(dev[0] * dev[0] + dev[1] * dev[1] + dev[2] * dev[2]);
+    const double gamma = dn + (3.0 * lambda + 2.0 * mu) / (2.0 * mu) * tr * alpha;
+    if (!tension & (gamma <= 0.0)) return;
+    const double k = gamma / (tension ? 1.0 : dn);
+    // log s' - log s per direction
+    double dl[3], n2 = 0.0;
 #pragma unroll
-    for (int i = 0; i < 3; i++) dev[i] = strain[i] - tr / d;
-    const double prev_det = s[0] * s[1] * s[2];
-    if (tr > 0.0 || (dev[0] == 0.0 && dev[1] == 0.0 && dev[2] == 0.0)) {
-        // Tension: sigma -> 1, so F becomes its polar rotation U V^T.
-        hard = sqrt(strain[0] * strain[0] + strain[1] * strain[1] + strain[2] * strain[2]);
-        double fd[9], r[9];
-#pragma unroll
-        for (int k = 0; k < 9; k++) fd[k] = f32[k];
-        if (polar_f64(fd, r)) {
-#pragma unroll
-            for (int k = 0; k < 9; k++) f32[k] = (float)r[k];
-        } else {
-            const float one[3] = {1.0f, 1.0f, 1.0f};
-            svd_recompose(u, one, v, f32);
-        }
-        state[0] = (float)((double)state[0] * prev_det);
-        state[2] = (float)((double)state[2] + log_near1(prev_det));
-        state[1] = (float)((double)state[1] + hard);
-        return;
+    for (int i = 0; i < 3; i++) {
+        n2 += (raw[i] + third) * (raw[i] + third);
+        dl[i] = tension ? -raw[i] : third - dev[i] * k;
     }
-    double dn = sqrt(dev[0] * dev[0] + dev[1] * dev[1] + dev[2] * dev[2]);
-    double gamma = dn + (d * lambda + 2.0 * mu) / (2.0 * mu) * tr * alpha;
-    if (gamma <= 0.0) return;
-    if (!(s32[2] > 0.0f)) {
-        // det F <= 0 (or NaN): log of the signed singular value is NaN, as in the
-        // shader; the particle is disabled by the update.
-#pragma unroll
-        for (int i = 0; i < 3; i++) ns[i] = 1.0 + (double)expm1f((float)(strain[i] - dev[i] * (gamma / dn)));
-        const double new_det = ns[0] * ns[1] * ns[2];
-        state[0] = (float)((double)state[0] * prev_det / new_det);
-        state[2] = (float)((double)state[2] + log_near1(prev_det) - log_near1(new_det));
-        state[1] = (float)((double)state[1] + gamma);
-#pragma unroll
-        for (int i = 0; i < 3; i++)
-#pragma unroll
-            for (int j = 0; j < 3; j++)
-                f32[i * 3 + j] = (float)((double)u[i * 3 + 0] * ns[0] * (double)v[j * 3 + 0] +
-                                         (double)u[i * 3 + 1] * ns[1] * (double)v[j * 3 + 1] +
-                                         (double)u[i * 3 + 2] * ns[2] * (double)v[j * 3 + 2]);
-        return;
-    }
-    // Projection onto the cone: F' = U diag(s') V^T needs FP64-accurate singular
-    // vectors. Refine V, take the singular values |F v_i| from it and redo the
-    // return mapping with them (the decision above used the same values to second
-    // order), then F' = sum_i s'_i / |F v_i| (F v_i) v_i^T.
-    double fd[9], vd[9], bd[9];
-#pragma unroll
-    for (int k = 0; k < 9; k++) fd[k] = f32[k];
-    refine_right_vectors(fd, v, vd);
-#pragma unroll
-    for (int i = 0; i < 3; i++)
-#pragma unroll
-        for (int j = 0; j < 3; j++) bd[i * 3 + j] = fd[i * 3 + 0] * vd[0 * 3 + j] + fd[i * 3 + 1] * vd[1 * 3 + j] + fd[i * 3 + 2] * vd[2 * 3 + j];
-    double sr[3];
-#pragma unroll
-    for (int j = 0; j < 3; j++) sr[j] = sqrt(bd[0 * 3 + j] * bd[0 * 3 + j] + bd[1 * 3 + j] * bd[1 * 3 + j] + bd[2 * 3 + j] * bd[2 * 3 + j]);
-#pragma unroll
-    for (int i = 0; i < 3; i++) strain[i] = log_near1(sr[i]) + (double)state[2] / d;
-    tr = strain[0] + strain[1] + strain[2];
-#pragma unroll
-    for (int i = 0; i < 3; i++) dev[i] = strain[i] - tr / d;
-    dn = sqrt(dev[0] * dev[0] + dev[1] * dev[1] + dev[2] * dev[2]);
-    gamma = dn + (d * lambda + 2.0 * mu) / (2.0 * mu) * tr * alpha;
-    if (gamma <= 0.0) return;
-#pragma unroll
-    for (int i = 0; i < 3; i++) ns[i] = 1.0 + (double)expm1f((float)(strain[i] - dev[i] * (gamma / dn)));
-    hard = gamma;
-    const double det_r = sr[0] * sr[1] * sr[2];
-    const double new_det = ns[0] * ns[1] * ns[2];
-    state[0] = (float)((double)state[0] * det_r / new_det);
-    state[2] = (float)((double)state[2] + log_near1(det_r) - log_near1(new_det));
+    const double hard = tension ? sqrt(n2) : gamma;
+    const double r0 = exp_m1(dl[0]), r1 = exp_m1(dl[1]), r2 = exp_m1(dl[2]);
+    state[0] = (float)((double)state[0] / ((1.0 + r0) * (1.0 + r1) * (1.0 + r2)));
+    state[2] = (float)((double)state[2] - (dl[0] + dl[1] + dl[2]));
     state[1] = (float)((double)state[1] + hard);
-    double rs[3];
-#pragma unroll
-    for (int j = 0; j < 3; j++) rs[j] = ns[j] / sr[j];
+    double m[9];
 #pragma unroll
     for (int i = 0; i < 3; i++)
+#pragma unroll
+        for (int j = i; j < 3; j++)
+            m[i * 3 + j] = m[j * 3 + i] = r0 * v[i * 3] * v[j * 3] + r1 * v[i * 3 + 1] * v[j * 3 + 1] + r2 * v[i * 3 + 2] * v[j * 3 + 2];
+#pragma unroll
+    for (int i = 0; i < 3; i++) {
+        const double row[3] = {f32[i * 3], f32[i * 3 + 1], f32[i * 3 + 2]};
 #pragma unroll
         for (int j = 0; j < 3; j++)
-            f32[i * 3 + j] = (float)(bd[i * 3 + 0] * rs[0] * vd[j * 3 + 0] + bd[i * 3 + 1] * rs[1] * vd[j * 3 + 1] +
-                                     bd[i * 3 + 2] * rs[2] * vd[j * 3 + 2]);
+            f32[i * 3 + j] = (float)(row[j] + (row[0] * m[j] + row[1] * m[3 + j] + row[2] * m[6 + j]));
+    }
 }
 
 // ---------------------------------------------------------------------------
