@@ -21,6 +21,10 @@ HIPCC_FLAGS = [
     # Packed FP32 instructions stay off: keep float code on scalar VALU ops.
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     "-munsafe-fp-atomics",
+    # Hoisting constants and addresses out of the per-block loops, which run once or
+    # twice per wave, only holds (and spills) registers: P2G 156 -> 132 VGPRs, the
+    # neo-Hookean G2P 117 -> 102.
+    "-mllvm", "-disable-machine-licm",
 ]
 
 

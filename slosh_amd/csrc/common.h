@@ -43,6 +43,7 @@ __device__ __host__ inline uint32_t tile_index(uint32_t x, uint32_t y, uint32_t 
 #define CTR_ERRORS 2
 #define CTR_MOVERS 3     // entries of the mover list destined for this table
 #define CTR_OVERFLOW 4   // movers beyond a block's MOVER_CAP list slots
+#define CTR_ITEMS 5      // items of the fused G2P kernel
 #define ERR_HASH_FULL 1u
 #define ERR_LOOKUP 2u
 #define ERR_KEY_RANGE 4u
@@ -159,33 +160,77 @@ __device__ __host__ inline uint32_t hash_key(uint32_t k) {
     return k;
 }
 
-// Associated cell (round(x / h) - 1, half-to-even as WGSL round) and the block
-// it belongs to: block_associated_to_point (grid.slang:346-355) and
-// associated_cell_index_in_block_off_by_one (particle.slang:79-87).
-// x / h. For a power-of-two h (normal, with a normal reciprocal) the product
-// with the exact reciprocal 2^-e is the same number as the quotient: both are
-// exact scalings, or round the same exact value. The test is uniform (h is a
-// kernel argument), so the other path costs one scalar branch.
-__device__ inline float div_h(float x, float h) {
+// Whether h is a power of two with a normal reciprocal (2^-e in *inv).
+__device__ inline bool pow2_reciprocal(float h, float *inv) {
     const uint32_t hb = __float_as_uint(h);
-    if ((hb & 0x807fffffu) == 0u && hb - 0x00800000u < 0x7e000000u)
-        return x * __uint_as_float(0x7f000000u - (hb & 0x7f800000u));
-    return x / h;
+    *inv = __uint_as_float(0x7f000000u - (hb & 0x7f800000u));
+    return (hb & 0x807fffffu) == 0u && hb - 0x00800000u < 0x7e000000u;
+}
+
+// A point's quadratic stencil: per axis its associated cell (round(x / h) - 1,
+// half-to-even as WGSL round; node 0 of the stencil), that node's offset from
+// the point, and the point's offset from it in cells (the kernel's argument).
+// For a power-of-two h the products with the exact reciprocal are the same
+// numbers as the quotients: both are exact scalings, or round the same exact
+// value. The test is uniform (h is a kernel argument): one scalar branch for
+// all six quotients instead of a division sequence each.
+struct Stencil {
+    float cell[3], ref[3], f[3];
+};
+
+__device__ inline Stencil stencil_of(float h, float x, float y, float z) {
+    Stencil s;
+    const float p[3] = {x, y, z};
+    float r;
+    if (pow2_reciprocal(h, &r)) {
+#pragma unroll
+        for (int i = 0; i < 3; i++) {
+            s.cell[i] = rintf(p[i] * r) - 1.0f;
+            s.ref[i] = s.cell[i] * h - p[i];
+            s.f[i] = -s.ref[i] * r;
+        }
+    } else {
+#pragma unroll
+        for (int i = 0; i < 3; i++) {
+            s.cell[i] = rintf(p[i] / h) - 1.0f;
+            s.ref[i] = s.cell[i] * h - p[i];
+            s.f[i] = -s.ref[i] / h;
+        }
+    }
+    return s;
+}
+
+// The block a cell belongs to and its place there: block_associated_to_point
+// (grid.slang:346-355) and associated_cell_index_in_block_off_by_one
+// (particle.slang:79-87).
+__device__ inline void block_of_cell(const float *cell, int *b, uint32_t *l) {
+#pragma unroll
+    for (int i = 0; i < 3; i++) {
+        const float f = floorf(cell[i] / 4.0f);
+        b[i] = (int)f;
+        l[i] = (uint32_t)(cell[i] - f * 4.0f);
+    }
 }
 
 __device__ inline void assoc_block_cell(float h, float px, float py, float pz, int *bx, int *by, int *bz,
                                         uint32_t *cell) {
-    float ax = rintf(div_h(px, h)) - 1.0f;
-    float ay = rintf(div_h(py, h)) - 1.0f;
-    float az = rintf(div_h(pz, h)) - 1.0f;
-    float fx = floorf(ax / 4.0f), fy = floorf(ay / 4.0f), fz = floorf(az / 4.0f);
-    *bx = (int)fx;
-    *by = (int)fy;
-    *bz = (int)fz;
-    uint32_t lx = (uint32_t)(ax - fx * 4.0f);
-    uint32_t ly = (uint32_t)(ay - fy * 4.0f);
-    uint32_t lz = (uint32_t)(az - fz * 4.0f);
-    *cell = lx + 4u * ly + 16u * lz;
+    float r, c[3];
+    if (pow2_reciprocal(h, &r)) {
+        c[0] = rintf(px * r) - 1.0f;
+        c[1] = rintf(py * r) - 1.0f;
+        c[2] = rintf(pz * r) - 1.0f;
+    } else {
+        c[0] = rintf(px / h) - 1.0f;
+        c[1] = rintf(py / h) - 1.0f;
+        c[2] = rintf(pz / h) - 1.0f;
+    }
+    int b[3];
+    uint32_t l[3];
+    block_of_cell(c, b, l);
+    *bx = b[0];
+    *by = b[1];
+    *bz = b[2];
+    *cell = l[0] + 4u * l[1] + 16u * l[2];
 }
 
 // Bounded open-addressing lookup (find_block_header_id, grid.slang:176-198);

@@ -12,16 +12,14 @@
 //                    parts of the 7 "-1" neighbours' tiles, then
 //                    grid_update.slang:38-163 (gravity, clamp, collision
 //                    cache / collide(), boundary projection).
-//   k_g2p_update     one workgroup per block: 6x6x6 node halo in LDS, then per
-//                    primary particle g2p.slang:150-265 fused with
-//                    particle_update.slang:32-160. Outputs go to the other
+//   k_g2p_update     one wave per 64 entries of a block: 6x6x6 node halo in the
+//                    wave's LDS tile, then per primary particle g2p.slang:150-265
+//                    fused with particle_update.slang:32-160. Outputs go to the other
 //                    particle buffer at the particle's sorted slot, so particle
 //                    storage follows the block order of the last substep.
 //   k_g2p / k_particle_update  the same two stages as separate in-place
 //                    kernels, used when a hook replaces or observes G2P.
 //   k_rigid_update   rigid_impulses.slang:70-121.
-#include <type_traits>
-
 #include "launch.h"
 #include "../../include/slosh_hip.h"
 
@@ -1027,21 +1025,17 @@ __device__ inline void plastic_records(const StepParams &P, const PStatic &st, u
 // With dpt_i = ref + s_i h (s_i in {0,1,2}^3 the node's stencil shift), the sums
 // are formed from V = sum w v_i and S_a = sum w s_i,a v_i (a = x, y, z):
 // sum w v_i dpt_i,a = V ref_a + h S_a.
-__device__ inline void g2p_particle(const float4 *__restrict__ sh, float h, float inv_d, float3 p, bool enabled,
-                                    float3 *vel, float *vg, float *vgd_out) {
+// `at`: the particle's stencil; lc: its associated cell's place in the block.
+__device__ inline void g2p_particle(const float4 *__restrict__ sh, float h, float inv_d, const Stencil &at,
+                                    const uint32_t *lc, bool enabled, float3 *vel, float *vg, float *vgd_out) {
     float V[3] = {0.0f, 0.0f, 0.0f}, S[3][3] = {{0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f}};
     float ref[3] = {0.0f, 0.0f, 0.0f};
     if (enabled) {
         float w[3][3];
-        float pp[3] = {p.x, p.y, p.z};
-        uint32_t lc[3];
 #pragma unroll
         for (int i = 0; i < 3; i++) {
-            float ac = rintf(div_h(pp[i], h)) - 1.0f;
-            ref[i] = ac * h - pp[i];
-            k_eval_all(div_h(-ref[i], h), w[i]);
-            float ab = floorf(ac / 4.0f) * 4.0f;
-            lc[i] = (uint32_t)(ac - ab);
+            ref[i] = at.ref[i];
+            k_eval_all(at.f[i], w[i]);
         }
         const uint32_t packed = lc[0] + lc[1] * 6u + lc[2] * 36u;
         // V = sum_n w_n v_n and S[d] = sum_n s_d(n) w_n v_n (s_d = the node's stencil
@@ -1091,17 +1085,15 @@ __device__ inline void g2p_particle(const float4 *__restrict__ sh, float h, floa
     *vgd_out = inv_d * vgd;
 }
 
-// particle_update.slang:32-160 for one particle. `aff` holds the velocity
-// gradient on entry and the APIC affine matrix on exit. No multiply-add
+// particle_update.slang:32-160 for one particle, in three parts. No multiply-add
 // contraction here or in the stress helpers: F - I and mu (F F^T - I) are small
 // differences of O(1) values, so each rounding step shows in them; unfused
-// products and sums round like the shader source's separate operations. MODELS is the set of
-// material tags the kernel instance handles (bit t = tag t), so scenes without
-// SVD-based models do not carry that code's register footprint.
-template <uint32_t MODELS, bool F64>
-__device__ inline void update_particle(const StepParams &P, float3 &pos, float3 &v, float &mass, uint32_t &enabled,
-                                       float *aff, float *F, float4 prop, float4 model, const PStatic &st,
-                                       uint32_t oid, uint32_t scene, float *dps) {
+// products and sums round like the shader source's separate operations.
+
+// The first part: velocity clamp, damping and fixing, the new position, F += F
+// (dt aff) (`aff` is the velocity gradient, zeroed for a fixed particle).
+__device__ inline void advance_particle(const StepParams &P, float3 pos, float3 &v, float *aff, float *F, float4 prop,
+                                        float3 *np) {
 #pragma clang fp contract(off)
     const float dt = P.dt, h = P.h;
     float vl = sqrtf(v.x * v.x + v.y * v.y + v.z * v.z);
@@ -1113,7 +1105,7 @@ __device__ inline void update_particle(const StepParams &P, float3 &pos, float3 
     if (damp != 1.0f) v = make_float3(v.x / damp, v.y / damp, v.z / damp);
     bool fixed = __float_as_uint(prop.z) != 0u;
     if (fixed) v = make_float3(0.0f, 0.0f, 0.0f);
-    float3 np = make_float3(pos.x + v.x * dt, pos.y + v.y * dt, pos.z + v.z * dt);
+    *np = make_float3(pos.x + v.x * dt, pos.y + v.y * dt, pos.z + v.z * dt);
     // F += mul(F, affine * dt)
     float adt[9], fa[9];
 #pragma unroll
@@ -1125,9 +1117,16 @@ __device__ inline void update_particle(const StepParams &P, float3 &pos, float3 
 #pragma unroll
         for (int k = 0; k < 9; k++) aff[k] = 0.0f;
     }
-    // DefaultParticleModel::update, default.slang:51-92
+}
+
+// The second part, DefaultParticleModel::update (default.slang:51-92): the plastic
+// projection of F and the stress. MODELS is the set of material tags the kernel
+// instance handles (bit t = tag t), so scenes without SVD-based models do not
+// carry that code's register footprint.
+template <uint32_t MODELS, bool F64>
+__device__ inline void material_update(const StepParams &P, float *F, float4 model, const PStatic &st, uint32_t oid,
+                                       uint32_t scene, float *dps, float *stress) {
     uint32_t tag = __float_as_uint(model.x);
-    float stress[9];
     if ((MODELS & 2u) && tag == 1u) {
         nh_stress(model.y, model.z, F, stress);
     } else if ((MODELS & 1u) && tag == 0u) {
@@ -1145,21 +1144,27 @@ __device__ inline void update_particle(const StepParams &P, float3 &pos, float3 
 #pragma unroll
         for (int k = 0; k < 9; k++) stress[k] = 0.0f;
     }
-    float sk = prop.x * P.inv_d * dt;
-    bool ok = np.x == np.x && np.y == np.y && np.z == np.z && det3(F) > 0.0f;
-    if (ok) {
-        pos = np;
+}
+
+// The third part: whether the particle stays enabled (a finite position and
+// det F > 0), and its APIC affine matrix (from the velocity gradient, in `aff`);
+// a particle that is disabled gets zeros and F = I.
+__device__ inline bool stays_enabled(float3 np, const float *F) {
+    return np.x == np.x && np.y == np.y && np.z == np.z && det3(F) > 0.0f;
+}
+
+__device__ inline void finish_particle(const StepParams &P, bool ok, float mass, float init_volume, const float *stress,
+                                       float *aff, float *F) {
+#pragma clang fp contract(off)
+    const float sk = init_volume * P.inv_d * P.dt;
 #pragma unroll
-        for (int k = 0; k < 9; k++) aff[k] = aff[k] * mass - stress[k] * sk;
-    } else {
-        enabled = 0u;
-        v = make_float3(0.0f, 0.0f, 0.0f);
-#pragma unroll
-        for (int k = 0; k < 9; k++) {
+    for (int k = 0; k < 9; k++) {
+        if (ok) {
+            aff[k] = aff[k] * mass - stress[k] * sk;
+        } else {
             F[k] = (k == 0 || k == 4 || k == 8) ? 1.0f : 0.0f;
             aff[k] = 0.0f;
         }
-        mass = 0.0f;
     }
 }
 
@@ -1221,16 +1226,6 @@ __device__ inline uint32_t entry_slot(const BlockRange &r, uint32_t m) {
     return m < r.cand_n ? r.cand_lo + m : r.list[m - r.cand_n];
 }
 
-// Block key of the particle at x (w = scene << 1 | enabled bits): the key the
-// sort files it under (a block outside the key space aliases another block of
-// its key space, and is filed, counted and processed under that key).
-__device__ inline uint32_t key_at(float h, uint32_t batched, float4 x) {
-    int bx, by, bz;
-    uint32_t cell;
-    assoc_block_cell(h, x.x, x.y, x.z, &bx, &by, &bz, &cell);
-    return pack_key(batched, __float_as_uint(x.w) >> 1, bx, by, bz);
-}
-
 // ---------------------------------------------------------------------------
 // Kernels.
 
@@ -1266,51 +1261,78 @@ struct NextTable {
     uint32_t prime;
 };
 
-// Block totals and starts of a steady-state substep, in block-list order, by
-// one workgroup of 192 threads: total = stayers of the block's previous range +
-// movers received. Runs beside the per-block work of the same launch (nothing
-// in it reads them).
+// Per block, in block-list order, by one workgroup of 192 threads: in the steady
+// state its total (stayers of its previous range + movers received) and storage
+// start; in both modes the start of its G2P items (one per 64 entries of its
+// sequence) and, into `counters`, the number of items. Runs beside the per-block
+// work of the same launch (nothing in it reads them).
+template <bool FAST>
 __device__ void p2g_block_scan(const Members &M, uint32_t *__restrict__ blk_start, uint32_t *__restrict__ blk_cnt,
-                               uint32_t *wsum) {
+                               uint32_t *__restrict__ item_start, uint32_t *__restrict__ n_items, uint32_t *wsum) {
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
     const uint32_t B = M.counters[CTR_NUM_BLOCKS];
     // 24 entries per thread: up to 4608 blocks in one pass of two dependent loads.
     constexpr uint32_t PER = 24u, TILE = 192u * PER;
-    uint32_t carry = 0u;
+    uint32_t carry = 0u, icarry = 0u;
     for (uint32_t base = 0; base < B; base += TILE) {
-        uint32_t hid[PER], c[PER];
+        uint32_t hid[PER], c[PER], it[PER];
 #pragma unroll
         for (uint32_t j = 0; j < PER; j++) {
             const uint32_t k = base + tid * PER + j;
             hid[j] = k < B ? M.blist[k] : SLOSH_NONE;
         }
-        uint32_t t = 0u;
+        uint32_t t = 0u, ti = 0u;
 #pragma unroll
         for (uint32_t j = 0; j < PER; j++) {
-            c[j] = hid[j] != SLOSH_NONE ? M.bin[hid[j]].z + M.mcount[hid[j]] : 0u;
+            c[j] = 0u;
+            it[j] = 0u;
+            if (hid[j] != SLOSH_NONE) {
+                const BlockRange br = block_range<FAST>(M, hid[j]);
+                c[j] = br.total;
+                it[j] = br.total ? (br.cand_n + br.list_n + 63u) >> 6 : 0u;
+            }
             t += c[j];
+            ti += it[j];
         }
-        uint32_t x = t;
+        uint32_t x = t, xi = ti;
 #pragma unroll
         for (int d = 1; d < 64; d <<= 1) {
-            const uint32_t y = __shfl_up(x, d);
-            if ((int)lane >= d) x += y;
+            const uint32_t y = __shfl_up(x, d), yi = __shfl_up(xi, d);
+            if ((int)lane >= d) {
+                x += y;
+                xi += yi;
+            }
         }
-        if (lane == 63) wsum[wave] = x;
+        if (lane == 63) {
+            wsum[wave] = x;
+            wsum[4 + wave] = xi;
+        }
         __syncthreads();
-        const uint32_t w0 = wsum[0], w1 = wsum[1], w2 = wsum[2];
-        uint32_t e = carry + (wave > 0 ? w0 : 0u) + (wave > 1 ? w1 : 0u) + x - t;
+        uint32_t e = carry + x - t, ei = icarry + xi - ti;
+#pragma unroll
+        for (uint32_t w = 0; w < 3; w++) {
+            if (w < wave) {
+                e += wsum[w];
+                ei += wsum[4 + w];
+            }
+            carry += wsum[w];
+            icarry += wsum[4 + w];
+        }
 #pragma unroll
         for (uint32_t j = 0; j < PER; j++) {
             if (hid[j] != SLOSH_NONE) {
-                blk_start[hid[j]] = e;
-                blk_cnt[hid[j]] = c[j];
+                if (FAST) {
+                    blk_start[hid[j]] = e;
+                    blk_cnt[hid[j]] = c[j];
+                }
+                item_start[hid[j]] = ei;
             }
             e += c[j];
+            ei += it[j];
         }
-        carry += w0 + w1 + w2;
         __syncthreads();  // wsum is reused by the next tile
     }
+    if (tid == 0) *n_items = icarry;
 }
 
 // LDS element of node (x, y, z) of a P2G slab tile (z = 0..3), 16-byte elements.
@@ -1339,7 +1361,7 @@ struct P2GShared {
                               // p2g_chunk before it stages anything
     };
     uint32_t lcnt[64];
-    uint32_t wsum[4];
+    uint32_t wsum[8];
 };
 static_assert(sizeof(float4) * 3 * P2G_SLAB_LDS <= sizeof(P2GShared<192>::sp4),
               "the slab tiles take no LDS beyond the staging of the smallest chunk");
@@ -1396,18 +1418,13 @@ __device__ inline void p2g_chunk(const StepParams &P, P2GShared<P2G_CHUNK> &S, u
         }
         // The associated cell: node 0 of the stencil sits at d0 = x_0 - x_p; its
         // block (floor of the cell / 4) and its place in that block.
-        const float xp[3] = {ps[r].x, ps[r].y, ps[r].z};
-        float d0[3];
-        int blk[3], lc[3];
+        const Stencil at = stencil_of(h, ps[r].x, ps[r].y, ps[r].z);
+        int blk[3];
+        uint32_t lc[3];
+        block_of_cell(at.cell, blk, lc);
+        const float *d0 = at.ref;
 #pragma unroll
-        for (int i = 0; i < 3; i++) {
-            const float ac = rintf(div_h(xp[i], h)) - 1.0f;
-            d0[i] = ac * h - xp[i];
-            fo[r][i] = div_h(-d0[i], h);
-            const float fb = floorf(ac / 4.0f);
-            blk[i] = (int)fb;
-            lc[i] = (int)(ac - fb * 4.0f);
-        }
+        for (int i = 0; i < 3; i++) fo[r][i] = at.f[i];
         // A candidate that moved to another block is that block's member.
         if (pack_key(P.batched, __float_as_uint(ps[r].w) >> 1, blk[0], blk[1], blk[2]) != block_key) {
             pp[r] = SLOSH_NONE;
@@ -1416,7 +1433,7 @@ __device__ inline void p2g_chunk(const StepParams &P, P2GShared<P2G_CHUNK> &S, u
         const float *c = cc[r];
 #pragma unroll
         for (int i = 0; i < 3; i++) a0[r][i] = mom[i] + (d0[0] * c[i] + d0[1] * c[3 + i] + d0[2] * c[6 + i]);
-        cl[r] = (uint32_t)(lc[0] + 4 * lc[1] + 16 * lc[2]);
+        cl[r] = lc[0] + 4u * lc[1] + 16u * lc[2];
         rk[r] = atomicAdd(&S.lcnt[cl[r]], 1u);
     }
     __syncthreads();
@@ -1485,14 +1502,15 @@ __device__ inline void p2g_chunk(const StepParams &P, P2GShared<P2G_CHUNK> &S, u
 }
 
 // Chunks of up to 384 members fit in 128 VGPRs (4 waves/SIMD; their LDS allows 5
-// workgroups per CU); 512 needs ~156 (3 waves/SIMD, as its 35 KB of LDS allow).
+// workgroups per CU); 512 needs 132 (3 waves/SIMD, as its 35 KB of LDS allow).
 template <int P2G_CHUNK, bool FAST>
 __global__ __launch_bounds__(192, P2G_CHUNK <= 384 ? 4 : 1) void k_p2g(StepParams P, NextTable nt, const float4 *__restrict__ pos,
                                              const float4 *__restrict__ vm, const float *__restrict__ C,
                                              const float *__restrict__ fdt, uint32_t pcap, Members M,
                                              const uint32_t *__restrict__ keys, float4 *__restrict__ tiles,
                                              uint32_t *__restrict__ cell_cnt, uint32_t *__restrict__ blk_start_out,
-                                             uint32_t *__restrict__ blk_cnt_out) {
+                                             uint32_t *__restrict__ blk_cnt_out, uint32_t *__restrict__ item_start,
+                                             uint32_t *__restrict__ n_items) {
     __shared__ P2GShared<P2G_CHUNK> S;
     if (nt.prime) {
         for (uint32_t s = blockIdx.x * blockDim.x + threadIdx.x; s < P.cap; s += gridDim.x * blockDim.x)
@@ -1504,10 +1522,9 @@ __global__ __launch_bounds__(192, P2G_CHUNK <= 384 ? 4 : 1) void k_p2g(StepParam
             nt.counters[CTR_OVERFLOW] = 0u;
         }
     }
-    // Steady state: workgroup 0 computes the block totals and starts.
-    const uint32_t first = FAST ? 1u : 0u;
-    if (FAST && blockIdx.x == 0) {
-        p2g_block_scan(M, blk_start_out, blk_cnt_out, S.wsum);
+    // Workgroup 0 computes the block totals and starts (steady state) and the item starts.
+    if (blockIdx.x == 0) {
+        p2g_block_scan<FAST>(M, blk_start_out, blk_cnt_out, item_start, n_items, S.wsum);
         return;
     }
     const uint32_t B = M.counters[CTR_NUM_BLOCKS];
@@ -1516,7 +1533,7 @@ __global__ __launch_bounds__(192, P2G_CHUNK <= 384 ? 4 : 1) void k_p2g(StepParam
     const int lx = lane & 3, ly = (lane >> 2) & 3, lz = lane >> 4;
 
     if (threadIdx.x < 64) S.lcnt[threadIdx.x] = 0u;
-    for (uint32_t k = blockIdx.x - first; k < B; k += gridDim.x - first) {
+    for (uint32_t k = blockIdx.x - 1u; k < B; k += gridDim.x - 1u) {
         const uint32_t hid = M.blist[k];
         const BlockRange br = block_range<FAST>(M, hid);
         // A block without particles (a "+1" neighbour only) has an all-zero tile:
@@ -1596,6 +1613,33 @@ __global__ __launch_bounds__(192, P2G_CHUNK <= 384 ? 4 : 1) void k_p2g(StepParam
     }
 }
 
+// The work list of the fused G2P kernel: an item is 64 consecutive entries of a
+// block's sequence (header id, index of the 64).
+struct ItemLists {
+    uint2 *items;
+    const uint32_t *item_start;  // per block: its first item
+    uint32_t *taken, *stay;      // per block, counted by G2P: output slots taken, stayers
+    uint32_t fast;
+};
+
+// Writes a block's items and clears its counters; the lanes of one wave.
+__device__ inline void write_items(const Members &M, const ItemLists &L, uint32_t hid, uint32_t lane) {
+    uint32_t entries, total;
+    if (L.fast) {
+        const BlockRange br = block_range<true>(M, hid);
+        entries = br.cand_n + br.list_n;
+        total = br.total;
+    } else {
+        entries = total = M.blk_cnt[hid];
+    }
+    const uint32_t n = total ? (entries + 63u) >> 6 : 0u;
+    for (uint32_t c = lane; c < n; c += 64u) L.items[L.item_start[hid] + c] = make_uint2(hid, c);
+    if (lane == 0) {
+        L.taken[hid] = 0u;
+        L.stay[hid] = 0u;
+    }
+}
+
 // mode 0: node momentum from tiles; mode 1: nodes already hold momentum (P2G hook).
 // do_update 0: only combine tiles (grid update disabled).
 template <bool MESH>
@@ -1605,8 +1649,9 @@ __global__ __launch_bounds__(256) void k_grid_update(StepParams P, const float4 
                                                      const uint32_t *__restrict__ keys, Colliders cs,
                                                      const NodeColl *__restrict__ coll_prev, NodeColl *__restrict__ coll_cur,
                                                      const uint32_t *__restrict__ counters,
-                                                     const uint32_t *__restrict__ blk_cnt, uint32_t mode,
+                                                     Members M, ItemLists L, uint32_t mode,
                                                      uint32_t do_update) {
+    const uint32_t *__restrict__ blk_cnt = M.blk_cnt;
     __shared__ float4 cbox[2 * SLOSH_MAX_COLLIDERS];
     if (threadIdx.x < cs.count) collider_box<MESH>(cs, threadIdx.x, 1.5f * P.h, &cbox[2 * threadIdx.x], &cbox[2 * threadIdx.x + 1]);
     __syncthreads();
@@ -1618,6 +1663,7 @@ __global__ __launch_bounds__(256) void k_grid_update(StepParams P, const float4 
         const uint32_t hid = blist[k];
         float4 acc;
         if (mode == 0) {
+            write_items(M, L, hid, lane);
             // Tiles of blocks without particles were not written (they count as
             // zero). Each tile value is loaded together with its block's particle
             // count and then selected by it, so the tile loads wait only for the
@@ -1789,12 +1835,38 @@ __device__ inline void load_halo(float4 *__restrict__ sh, const float4 *__restri
     }
 }
 
+// The same by one wave into its own LDS tile: lanes 0..6 load the neighbour ids,
+// each lane takes its nodes' from them.
+__device__ inline void load_halo_wave(float4 *__restrict__ sh, const float4 *__restrict__ nodes,
+                                      const uint32_t *__restrict__ nbr, uint32_t hid, uint32_t lane) {
+    const uint32_t nb = lane < 7u ? nbr[(size_t)hid * NBR_STRIDE + lane] : hid;
+    constexpr uint32_t R = (TILE_NODES + 63u) / 64u;
+    float4 v[R];
+#pragma unroll
+    for (uint32_t r = 0; r < R; r++) {
+        const uint32_t j = lane + 64u * r;
+        const uint32_t sx = j % 6u, sy = (j / 6u) % 6u, sz = j / 36u;
+        const uint32_t ox = sx >= 4u, oy = sy >= 4u, oz = sz >= 4u;
+        const uint32_t oi = ox * 4u + oy * 2u + oz;
+        const uint32_t src = (uint32_t)__shfl((int)nb, oi == 0u ? 7 : (int)oi - 1);
+        const uint32_t node = (sx - 4u * ox) + 4u * (sy - 4u * oy) + 16u * (sz - 4u * oz);
+        v[r] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        if (j < TILE_NODES && src != SLOSH_NONE) v[r] = nodes[(size_t)src * NODES_PER_BLOCK + node];
+    }
+#pragma unroll
+    for (uint32_t r = 0; r < R; r++) {
+        const uint32_t j = lane + 64u * r;
+        if (j < TILE_NODES) sh[j] = v[r];
+    }
+}
+
 // What the fused G2P kernel prepares for the next substep: its table (keys
 // inserted, a new block's mover count cleared), the list of particles that
 // leave their block, and every block's stayer count.
 struct NextSort {
     uint32_t *mcount;         // next table: movers per block (cleared at insertion)
     uint32_t *mv_key, *mv_slot;  // movers: new block key, output slot
+    uint32_t *taken;          // this table: output slots each block has handed out
     uint32_t *stay;           // this table: particles of each block that stay in it
     uint32_t *errors;         // this substep's error word (ERR_KEY_RANGE)
 };
@@ -1802,79 +1874,78 @@ struct NextSort {
 // F64: the SVD-based steps refined to FP64 accuracy. The bound keeps that
 // variant at three waves per SIMD (168 VGPRs).
 //
+// One wave per item: 64 consecutive entries of a block's sequence, with the
+// block's node halo in an LDS tile of the wave's own, so that waves share no
+// barrier and a block's last, partly filled round holds one wave instead of a
+// workgroup. With one workgroup per block a second round of 256 entries cost a
+// block 3.8 us of serial latency, and a block of 50 particles kept four waves;
+// per wave (medians of the kernel, before and after): 2.1M sand and spheres (42k
+// blocks) 643 -> 282 us, 48 scenes of three materials (2.0M) 320 -> 172 us, sand on
+// a heightfield (85k) 43 -> 21 us, dam break of 131k 15.7 -> 13.6 us and of 1M
+// 52 us both at its start, 66 -> 52 us once it moves. The small scenes are bound by
+// the chain of dependent loads and the ~1000 instructions of one particle, the
+// large ones by memory (188 MB per launch at 1M) and issue.
+//
 // Output order: a block's members take the output slots [start, start + total)
-// of the block in order of arrival of their wavefronts (one LDS atomic per
-// wavefront), so a block's particles stay together in storage. The particles
-// whose updated position leaves the block are listed, with their new block key,
-// for the next substep's sort; the others are counted (the block's stayers).
-template <uint32_t MODELS, int NT, bool F64, bool FAST>
-__global__ __launch_bounds__(NT, F64 ? (MODELS == 3u ? 4 : 3) : 1) void k_g2p_update(StepParams P, PBuf in, PBuf out, PStatic st, uint32_t pcap,
+// of the block in order of arrival of their waves (one atomic per wave, issued
+// before the sums that hide it), so a block's particles stay together in
+// storage. The particles whose updated position leaves the block are listed,
+// with their new block key, for the next substep's sort; the others are counted
+// (the block's stayers).
+template <uint32_t MODELS, bool F64>
+__global__ __launch_bounds__(256, F64 ? (MODELS == 3u ? 4 : 3) : 1) void k_g2p_update(StepParams P, PBuf in, PBuf out, PStatic st, uint32_t pcap_arg,
                                                     float *__restrict__ fdt, Members M,
+                                                    const uint2 *__restrict__ items,
                                                     const uint32_t *__restrict__ blk_start,
                                                     const float4 *__restrict__ nodes,
                                                     const uint32_t *__restrict__ keys, NextTable nt, NextSort ns,
                                                     Bodies bodies) {
-    __shared__ float4 sh[TILE_NODES];
-    __shared__ uint32_t n_out, n_stay;
+    extern __shared__ float4 halo[];  // TILE_NODES per wave
     // integrate_bodies: reads no particle or grid state (the impulses it applies
-    // are only written by the host), so it runs alongside the particle update.
-    if (blockIdx.x == 0 && threadIdx.x < bodies.count) integrate_body(P, bodies, threadIdx.x);
-    const uint32_t B = M.counters[CTR_NUM_BLOCKS];
-    const uint32_t n_ovf = M.counters[CTR_OVERFLOW];
-    const uint32_t lane = threadIdx.x & 63u;
-    BlockInit init;
-    init.mcount = ns.mcount;
-    init.blk_cnt = nullptr;
-    init.cell_cnt = nullptr;
-    // A block with stayers inserts its 8 blocks into the next table while the
-    // workgroup works on its next block (threads 0-7, key in `pk`): the first
-    // probe's load is issued with the next block's halo loads.
-    uint32_t pk = SLOSH_NONE;
-    for (uint32_t k = blockIdx.x; k < B; k += gridDim.x) {
-        uint32_t probe = SLOSH_NONE;
-        if (pk != SLOSH_NONE) probe = nt.keys[hash_key(pk) & (P.cap - 1u)];
-        const uint32_t hid = M.blist[k];
-        const BlockRange br = block_range<FAST>(M, hid);
-        const uint32_t cnt = br.total;
-        if (cnt == 0) {
-            if (threadIdx.x == 0) ns.stay[hid] = 0u;
-            if (pk != SLOSH_NONE && probe != pk) hash_insert(nt.keys, P.cap, pk, nt.counters, init);
-            pk = SLOSH_NONE;
-            continue;
-        }
+    // are only written by the host), so the last workgroup runs it alongside the
+    // particle update.
+    if (blockIdx.x == gridDim.x - 1u) {
+        if (threadIdx.x < bodies.count) integrate_body(P, bodies, threadIdx.x);
+        return;
+    }
+    const uint32_t n_items = M.counters[CTR_ITEMS];
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), waves = blockDim.x >> 6;
+    float4 *sh = halo + wave * TILE_NODES;
+    for (uint32_t i = blockIdx.x * waves + wave; i < n_items; i += (gridDim.x - 1u) * waves) {
+        // Opaque copies: most waves take one item, so nothing is worth computing
+        // ahead of the loop and holding in (spilled) registers.
+        uint32_t lane = threadIdx.x & 63u, pcap = pcap_arg;
+        asm volatile("" : "+v"(lane), "+s"(pcap));
+        BlockInit init;
+        init.mcount = ns.mcount;
+        init.blk_cnt = nullptr;
+        init.cell_cnt = nullptr;
+        const uint2 item = items[i];
+        const uint32_t hid = __builtin_amdgcn_readfirstlane(item.x);
+        const uint32_t first = __builtin_amdgcn_readfirstlane(item.y) * 64u;
+        const BlockRange br = M.fast ? block_range<true>(M, hid) : block_range<false>(M, hid);
         const uint32_t s0 = blk_start[hid];
         const uint32_t block_key = keys[hid];
-        int bx, by, bz;
-        uint32_t scene;
-        unpack_key(P.batched, block_key, &bx, &by, &bz, &scene);
-        bool stays = false;
-        load_halo(sh, nodes, M.nbr, hid);
-        if (threadIdx.x == 0) {
-            n_out = 0u;
-            n_stay = 0u;
-        }
-        __syncthreads();
-        if (pk != SLOSH_NONE && probe != pk) hash_insert(nt.keys, P.cap, pk, nt.counters, init);
-        pk = SLOSH_NONE;
-        // The block's entries (a candidate is a member only if it is still in the
-        // block), then, only if some of its movers overflowed their list, the
-        // overflow list, whose entries of other blocks are skipped. Per member:
-        // G2P, update, output at the next free slot of the block's range (one LDS
-        // atomic per wavefront), listed if it leaves the block, its blocks
-        // inserted into the next table. Every lane of the workgroup runs the same
-        // number of iterations (the wave-level counting and run detection see all
-        // lanes).
+        // The item's entries (a candidate is a member only if it is still in the
+        // block); the block's first item then takes the overflow list, only if some
+        // of the block's movers overflowed theirs (entries of other blocks are
+        // skipped). Per member: G2P, update, output at the next free slot of the
+        // block's range, listed if it leaves the block, its blocks inserted into the
+        // next table. Every lane runs the same number of iterations (the wave-level
+        // counting and run detection see all lanes).
         const uint32_t n_main = br.cand_n + br.list_n;
-        const uint32_t n_all = n_main + (br.overflow ? n_ovf : 0u);
-        for (uint32_t jb = 0; jb < n_all; jb += blockDim.x) {
-            const uint32_t m = jb + threadIdx.x;
-            bool entry = m < n_all;
+        const uint32_t n_ovf = first == 0u && br.overflow ? M.counters[CTR_OVERFLOW] : 0u;
+        for (uint32_t o = 0; o < 64u + n_ovf; o += 64u) {
+            bool entry;
             uint32_t p = 0u;
-            if (m < n_main) {
-                p = entry_slot(br, m);
-            } else if (entry) {
-                entry = M.ovf_hid[m - n_main] == hid;
-                p = M.ovf_slot[m - n_main];
+            if (o == 0u) {
+                const uint32_t m = first + lane;
+                entry = m < n_main;
+                if (entry) p = entry_slot(br, m);
+            } else {
+                const uint32_t q = o - 64u + lane;
+                entry = q < n_ovf && M.ovf_hid[q] == hid;
+                if (entry) p = M.ovf_slot[q];
             }
             float4 ps = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
             // The neo-Hookean-only instance has registers to spare: it issues the
@@ -1891,28 +1962,33 @@ __global__ __launch_bounds__(NT, F64 ? (MODELS == 3u ? 4 : 3) : 1) void k_g2p_up
                     oid = in.ids[p];
                 }
             }
-            const bool valid = entry && key_at(P.h, P.batched, ps) == block_key;
+            load_halo_wave(sh, nodes, M.nbr, hid, lane);  // (the last iteration may have reused the tile)
+            const uint32_t wbits = __float_as_uint(ps.w);
+            const uint32_t scene = wbits >> 1;
+            const Stencil at = stencil_of(P.h, ps.x, ps.y, ps.z);
+            int blk[3];
+            uint32_t lc[3];
+            block_of_cell(at.cell, blk, lc);
+            const bool valid = entry && pack_key(P.batched, scene, blk[0], blk[1], blk[2]) == block_key;
             const uint64_t vmask = __ballot(valid);
+            if (vmask == 0ull) continue;
             uint32_t ob = 0u;
-            if (lane == 0 && vmask) ob = atomicAdd(&n_out, (uint32_t)__popcll(vmask));
-            const uint32_t j = __shfl(ob, 0) + (uint32_t)__popcll(vmask & lanemask_lt());
-            const uint32_t slot = s0 + j;
+            if (lane == 0) ob = atomicAdd(&ns.taken[hid], (uint32_t)__popcll(vmask));
+            const float3 pos = make_float3(ps.x, ps.y, ps.z);
+            float3 v;
+            float aff[9], vgd;
+            if (valid) g2p_particle(sh, P.h, P.inv_d, at, lc, (wbits & 1u) != 0u, &v, aff, &vgd);
+            // The wave's first slot, from lane 0 (every lane is active here).
+            const uint32_t slot = s0 + __builtin_amdgcn_readfirstlane(ob) + (uint32_t)__popcll(vmask & lanemask_lt());
             uint32_t next_key = 0u;
+            bool in_range = true;
             if (valid) {
-                const uint32_t wbits = __float_as_uint(ps.w);
-                uint32_t enabled = wbits & 1u;
-                float3 pos = make_float3(ps.x, ps.y, ps.z);
-                float3 v;
-                float aff[9];
-                float vgd;
-                g2p_particle(sh, P.h, P.inv_d, pos, enabled != 0u, &v, aff, &vgd);
-                const uint32_t scene = wbits >> 1;
                 // Uniform masses (one for all, or one per scene) skip the 16-byte
                 // velocity / mass load (the velocity comes from the grid): only the
                 // update disables, and it zeroes the mass.
-                float mass = P.mass_uniform ? (enabled ? P.u_mass : 0.0f)
-                             : P.scene_mass  ? (enabled ? st.scene_rec[4 * (size_t)scene + 3].z : 0.0f)
-                                             : in.vm[p].w;
+                const float mass = P.mass_uniform ? ((wbits & 1u) ? P.u_mass : 0.0f)
+                                   : P.scene_mass  ? ((wbits & 1u) ? st.scene_rec[4 * (size_t)scene + 3].z : 0.0f)
+                                                   : in.vm[p].w;
                 if (!EARLY) {
 #pragma unroll
                     for (int q = 0; q < 9; q++) F[q] = in.F[(size_t)q * pcap + p];
@@ -1920,54 +1996,74 @@ __global__ __launch_bounds__(NT, F64 ? (MODELS == 3u ? 4 : 3) : 1) void k_g2p_up
                 }
                 float4 prop, model;
                 static_records(P, st, oid, scene, &prop, &model);
-                // Only Drucker-Prager particles read or write their plastic state
-                // (the other particles' state slots are never read).
-                const uint32_t tag = __float_as_uint(model.x);
-                const bool plastic = P.has_sand && (tag == 2u || tag == 3u);
-                float dps[3] = {0.0f, 0.0f, 0.0f};
-                if (plastic) {
-#pragma unroll
-                    for (int q = 0; q < 3; q++) dps[q] = in.dps[(size_t)q * pcap + p];
-                }
-                update_particle<MODELS, F64>(P, pos, v, mass, enabled, aff, F, prop, model, st, oid, scene, dps);
-                out.pos[slot] = make_float4(pos.x, pos.y, pos.z, __uint_as_float((wbits & ~1u) | enabled));
+                float3 np;
+                advance_particle(P, pos, v, aff, F, prop, &np);
+                // What is known before the stress leaves the registers: stored for a
+                // particle that stays enabled (rewritten below if it does not).
+                out.pos[slot] = make_float4(np.x, np.y, np.z, ps.w);
                 out.vm[slot] = make_float4(v.x, v.y, v.z, mass);
-#pragma unroll
-                for (int q = 0; q < 9; q++) {
-                    out.C[(size_t)q * pcap + slot] = aff[q];
-                    out.F[(size_t)q * pcap + slot] = F[q];
-                }
                 out.vgd[slot] = vgd;
                 out.ids[slot] = oid;
-                if (plastic) {
-#pragma unroll
-                    for (int q = 0; q < 3; q++) out.dps[(size_t)q * pcap + slot] = dps[q];
-                }
                 if (P.has_force) {
                     fdt[slot] = 0.0f;
                     fdt[(size_t)pcap + slot] = 0.0f;
                     fdt[2 * (size_t)pcap + slot] = 0.0f;
                 }
-                next_key = key_at(P.h, P.batched, make_float4(pos.x, pos.y, pos.z, __uint_as_float(wbits)));
+                bool ok = np.x == np.x && np.y == np.y && np.z == np.z;
+                int nx, ny, nz;
+                uint32_t cell;
+                assoc_block_cell(P.h, np.x, np.y, np.z, &nx, &ny, &nz, &cell);
+                next_key = pack_key(P.batched, scene, nx, ny, nz);
+                in_range = block_in_key_range(P.batched, nx, ny, nz);
+                // The FP64 steps need the registers: the velocity gradient waits in
+                // the wave's LDS tile, which the sums above no longer need.
+                float *keep = reinterpret_cast<float *>(sh) + lane;
+                if (F64) {
+#pragma unroll
+                    for (int q = 0; q < 9; q++) keep[64 * q] = aff[q];
+                }
+                // Only Drucker-Prager particles read or write their plastic state
+                // (the other particles' state slots are never read).
+                const uint32_t tag = __float_as_uint(model.x);
+                const bool plastic = P.has_sand && (tag == 2u || tag == 3u);
+                float dps[3] = {0.0f, 0.0f, 0.0f}, stress[9];
+                if (plastic) {
+#pragma unroll
+                    for (int q = 0; q < 3; q++) dps[q] = in.dps[(size_t)q * pcap + p];
+                }
+                material_update<MODELS, F64>(P, F, model, st, oid, scene, dps, stress);
+                if (plastic) {
+#pragma unroll
+                    for (int q = 0; q < 3; q++) out.dps[(size_t)q * pcap + slot] = dps[q];
+                }
+                ok = ok && det3(F) > 0.0f;
+                if (F64) {
+#pragma unroll
+                    for (int q = 0; q < 9; q++) aff[q] = keep[64 * q];
+                }
+                finish_particle(P, ok, mass, prop.x, stress, aff, F);
+#pragma unroll
+                for (int q = 0; q < 9; q++) {
+                    out.C[(size_t)q * pcap + slot] = aff[q];
+                    out.F[(size_t)q * pcap + slot] = F[q];
+                }
+                if (!ok) {
+                    const float4 old = in.pos[p];
+                    out.pos[slot] = make_float4(old.x, old.y, old.z, __uint_as_float(wbits & ~1u));
+                    out.vm[slot] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+                    next_key = block_key;
+                }
             }
             const bool mover = valid && next_key != block_key;
-            stays |= valid && !mover;
             const uint64_t sm = __ballot(valid && !mover);
-            if (lane == 0 && sm) atomicAdd(&n_stay, (uint32_t)__popcll(sm));
+            uint32_t before = 1u;
+            if (sm && lane == 0) before = atomicAdd(&ns.stay[hid], (uint32_t)__popcll(sm));
             const uint64_t mv = __ballot(mover);
             if (mv) {
                 // Only a particle that leaves its block can leave the key space (a
-                // block outside it would alias another one): reported, once per
-                // wavefront.
-                bool out_of_range = false;
-                if (mover) {
-                    const float4 np = out.pos[slot];
-                    int nx, ny, nz;
-                    uint32_t cell;
-                    assoc_block_cell(P.h, np.x, np.y, np.z, &nx, &ny, &nz, &cell);
-                    out_of_range = !block_in_key_range(P.batched, nx, ny, nz);
-                }
-                if (lane == 0 && __ballot(out_of_range)) atomicOr(ns.errors, ERR_KEY_RANGE);
+                // block outside it would alias another one): reported, once per wave.
+                const uint64_t bad = __ballot(mover && !in_range);
+                if (bad && lane == 0) atomicOr(ns.errors, ERR_KEY_RANGE);
                 if (nt.prime) {
                     // The movers, listed for the next substep's sort.
                     uint32_t lb = 0u;
@@ -1987,16 +2083,12 @@ __global__ __launch_bounds__(NT, F64 ? (MODELS == 3u ? 4 : 3) : 1) void k_g2p_up
                 // insert theirs, one round per run of equal keys.
                 const uint64_t heads = run_heads(next_key, mover) & mv;
                 insert_blocks(nt.keys, P.cap, P.batched, next_key, heads, nt.counters, init);
+                // The first wave with stayers inserts the block itself and its +1 neighbours.
+                if (__builtin_amdgcn_readfirstlane(before) == 0u)
+                    insert_blocks(nt.keys, P.cap, P.batched, block_key, 1ull, nt.counters, init);
             }
         }
-        // The barrier also ends this block's reads of `sh`, `n_out` and `n_stay`.
-        const bool any_stays = __syncthreads_or(stays);
-        if (threadIdx.x == 0) ns.stay[hid] = n_stay;
-        if (nt.prime && any_stays && threadIdx.x < 8)
-            pk = pack_key(P.batched, scene, bx + BLOCK_ASSOC[threadIdx.x][0], by + BLOCK_ASSOC[threadIdx.x][1],
-                          bz + BLOCK_ASSOC[threadIdx.x][2]);
     }
-    if (pk != SLOSH_NONE) hash_insert(nt.keys, P.cap, pk, nt.counters, init);
 }
 
 // WgTimestepBounds (timestep_bound.slang:18-92): per enabled particle, the
@@ -2104,8 +2196,11 @@ __global__ __launch_bounds__(256) void k_g2p(StepParams P, PBuf buf, uint32_t pc
             float3 v;
             float g[9];
             float vgd;
-            g2p_particle(sh, P.h, P.inv_d, make_float3(ps.x, ps.y, ps.z), (__float_as_uint(ps.w) & 1u) != 0u, &v, g,
-                         &vgd);
+            const Stencil at = stencil_of(P.h, ps.x, ps.y, ps.z);
+            int b[3];
+            uint32_t lc[3];
+            block_of_cell(at.cell, b, lc);
+            g2p_particle(sh, P.h, P.inv_d, at, lc, (__float_as_uint(ps.w) & 1u) != 0u, &v, g, &vgd);
             float4 o = buf.vm[p];
             buf.vm[p] = make_float4(v.x, v.y, v.z, o.w);
 #pragma unroll
@@ -2143,7 +2238,19 @@ __global__ __launch_bounds__(256, F64 ? 3 : 1) void k_particle_update(StepParams
     }
     float4 prop, model;
     static_records(P, st, oid, wbits >> 1, &prop, &model);
-    update_particle<MODELS, F64>(P, pos, v, mass, enabled, aff, F, prop, model, st, oid, wbits >> 1, dps);
+    float3 np;
+    float stress[9];
+    advance_particle(P, pos, v, aff, F, prop, &np);
+    material_update<MODELS, F64>(P, F, model, st, oid, wbits >> 1, dps, stress);
+    const bool ok = stays_enabled(np, F);
+    finish_particle(P, ok, mass, prop.x, stress, aff, F);
+    if (ok) {
+        pos = np;
+    } else {
+        enabled = 0u;
+        v = make_float3(0.0f, 0.0f, 0.0f);
+        mass = 0.0f;
+    }
     buf.pos[p] = make_float4(pos.x, pos.y, pos.z, __uint_as_float((wbits & ~1u) | enabled));
     buf.vm[p] = make_float4(v.x, v.y, v.z, mass);
 #pragma unroll
@@ -2188,6 +2295,14 @@ static uint32_t block_grid(const StepParams &P, uint32_t per_wg) {
     return min_t(div_up_t(P.cap, per_wg), P.block_wgs ? P.block_wgs : 8192u);
 }
 
+// Workgroups of `waves` items each: every entry sequence is at most its block's
+// candidates and listed movers (together at most 2 n entries), in 64s.
+static uint32_t item_grid(const StepParams &P, uint32_t waves) {
+    const uint64_t items = max_items(P.n, P.cap);
+    const uint32_t wgs = div_up_t(items, waves);
+    return wgs == 0u ? 1u : min_t(wgs, P.block_wgs ? P.block_wgs : 8192u);
+}
+
 static Members members_of(const TransferBuffers &t) {
     Members M;
     M.fast = t.fast;
@@ -2219,10 +2334,10 @@ hipError_t launch_p2g(const StepParams &P, const ParticleBuffers &pb, uint32_t p
                           : P.p2g_chunk == 256u ? k_p2g<256, false>
                           : P.p2g_chunk == 384u ? k_p2g<384, false>
                                                 : k_p2g<512, false>);
-    // Steady state: one more workgroup (the first) computes the block starts.
-    launch_kernel(ev, kern, dim3(block_grid(P, 1) + (t.fast ? 1u : 0u)), dim3(192), 0, stream, P, nt,
+    // One more workgroup (the first) computes the block and item starts.
+    launch_kernel(ev, kern, dim3(block_grid(P, 1) + 1u), dim3(192), 0, stream, P, nt,
                   (const float4 *)pb.pos, (const float4 *)pb.vm, (const float *)pb.C, (const float *)t.fdt, pcap,
-                  members_of(t), t.keys, t.tiles, t.cell_cnt, t.blk_start, t.blk_cnt);
+                  members_of(t), t.keys, t.tiles, t.cell_cnt, t.blk_start, t.blk_cnt, t.item_start, t.n_items);
     return hipGetLastError();
 }
 
@@ -2235,12 +2350,18 @@ hipError_t launch_grid_update(const StepParams &P, const TransferBuffers &t, con
     cs.count = c.count;
     cs.mesh_vtx = c.mesh_vtx;
     cs.mesh_idx = c.mesh_idx;
+    ItemLists items;
+    items.items = t.items;
+    items.item_start = t.item_start;
+    items.taken = t.taken;
+    items.stay = t.stay;
+    items.fast = t.fast;
     // Trimesh projection (a BVH walk) is compiled into its own instance so that
     // scenes without meshes keep the smaller kernel.
     launch_kernel(ev, c.mesh_vtx ? k_grid_update<true> : k_grid_update<false>, dim3(block_grid(P, 4)), dim3(256), 0,
                   stream, P,
                   (const float4 *)t.tiles, t.nodes, t.nbr, t.blist, t.keys, cs, (const NodeColl *)t.coll_prev,
-                  (NodeColl *)t.coll_cur, t.counters, (const uint32_t *)t.blk_cnt, mode, do_update);
+                  (NodeColl *)t.coll_cur, t.counters, members_of(t), items, mode, do_update);
     return hipGetLastError();
 }
 
@@ -2256,6 +2377,7 @@ hipError_t launch_g2p_update(const StepParams &P, const ParticleBuffers &in, con
     ns.mcount = next.mcount;
     ns.mv_key = next.mv_key;
     ns.mv_slot = next.mv_slot;
+    ns.taken = t.taken;
     ns.stay = t.stay;
     ns.errors = t.errors;
     Bodies b;
@@ -2275,19 +2397,14 @@ hipError_t launch_g2p_update(const StepParams &P, const ParticleBuffers &in, con
     // only (no SVD code), fixed-corotated and neo-Hookean, every material.
     const bool nh_only = (P.tag_mask & ~2u) == 0u;
     const bool elastic_only = (P.tag_mask & ~3u) == 0u;
-    const bool narrow = P.g2p_threads == 128u;
-    auto pick = [&](auto fast) {
-        constexpr bool F = decltype(fast)::value;
-        return nh_only ? (narrow ? k_g2p_update<2u, 128, false, F> : k_g2p_update<2u, 256, false, F>)
-               : elastic_only
-                   ? (P.svd_f64 ? (narrow ? k_g2p_update<3u, 128, true, F> : k_g2p_update<3u, 256, true, F>)
-                                : (narrow ? k_g2p_update<3u, 128, false, F> : k_g2p_update<3u, 256, false, F>))
-                   : (P.svd_f64 ? (narrow ? k_g2p_update<15u, 128, true, F> : k_g2p_update<15u, 256, true, F>)
-                                : (narrow ? k_g2p_update<15u, 128, false, F> : k_g2p_update<15u, 256, false, F>));
-    };
-    auto kern = t.fast ? pick(std::true_type{}) : pick(std::false_type{});
-    launch_kernel(ev, kern, dim3(block_grid(P, 1)), dim3(narrow ? 128 : 256), 0, stream, P, to_pbuf(in),
-                  to_pbuf(out), st, pcap, t.fdt, members_of(t), (const uint32_t *)t.blk_start,
+    auto kern = nh_only        ? k_g2p_update<2u, false>
+                : elastic_only ? (P.svd_f64 ? k_g2p_update<3u, true> : k_g2p_update<3u, false>)
+                               : (P.svd_f64 ? k_g2p_update<15u, true> : k_g2p_update<15u, false>);
+    const uint32_t waves = P.g2p_threads == 128u ? 2u : 4u;
+    // One more workgroup (the last) integrates the rigid bodies.
+    launch_kernel(ev, kern, dim3(item_grid(P, waves) + 1u), dim3(64u * waves),
+                  waves * TILE_NODES * (uint32_t)sizeof(float4), stream, P, to_pbuf(in),
+                  to_pbuf(out), st, pcap, t.fdt, members_of(t), (const uint2 *)t.items, (const uint32_t *)t.blk_start,
                   (const float4 *)t.nodes, t.keys, nt, ns, b);
     return hipGetLastError();
 }

@@ -33,6 +33,8 @@ struct TransferBuffers {
     const uint32_t *keys, *blist, *nbr, *counters;
     const uint32_t *perm;                             // full sort
     uint32_t *cell_cnt, *blk_start, *blk_cnt, *stay;  // this table
+    uint2 *items;  // the fused G2P kernel's items (max_items of them)
+    uint32_t *item_start, *n_items, *taken;
     const uint4 *bin;  // per block: range (start, count) and stayers of its previous-table block
     const uint32_t *mcount, *mlist, *ovf_slot, *ovf_hid;
     uint32_t *errors;  // this substep's error word
@@ -40,6 +42,10 @@ struct TransferBuffers {
     void *coll_prev, *coll_cur;
     float *fdt;
 };
+
+// Most items n particles in at most cap blocks can give: a block's entries are
+// its candidates and listed movers (at most n of each over all blocks), in 64s.
+inline size_t max_items(size_t n, size_t cap) { return 2 * n / 64 + (n < cap ? n : cap) + 1; }
 
 struct ParticleBuffers {
     float4 *pos, *vm;

@@ -186,6 +186,9 @@ struct slosh_data {
     uint32_t *stay[2] = {nullptr, nullptr}, *mcount[2] = {nullptr, nullptr};
     uint32_t *blist = nullptr, *nbr = nullptr, *cell_cnt = nullptr, *cell_start = nullptr;
     uint32_t *mlist = nullptr;  // MOVER_CAP movers per block
+    // The fused G2P kernel's items, and per block their start and the output slots taken.
+    uint2 *items = nullptr;
+    uint32_t *item_start = nullptr, *taken = nullptr;
     uint4 *bin = nullptr;       // per block: its previous-table block's range and stayers
     uint32_t *pslot = nullptr, *prank = nullptr, *perm = nullptr;
     // per particle: movers listed for the next substep, and movers beyond a
@@ -341,6 +344,7 @@ static int alloc_particle_buffers(slosh_data *d, size_t pcap, bool sand) {
     TRY(dalloc(&d->mv_slot, pcap));
     TRY(dalloc(&d->ovf_slot, pcap));
     TRY(dalloc(&d->ovf_hid, pcap));
+    TRY(dalloc(&d->items, max_items(pcap, d->cap)));
     // Every entry a kernel can read is a particle index even before the first sort.
     HIP_TRY(hipMemset(d->perm, 0, sizeof(uint32_t) * (pcap ? pcap : 1)));
     HIP_TRY(hipMemset(d->fdt, 0, sizeof(float) * 3 * (pcap ? pcap : 1)));
@@ -376,6 +380,7 @@ static void free_particle_buffers(slosh_data *d) {
     dfree(d->mv_slot);
     dfree(d->ovf_slot);
     dfree(d->ovf_hid);
+    dfree(d->items);
 }
 
 static bool model_is_sand(const slosh_particle_model &m) { return m.words[0] == 2u || m.words[0] == 3u; }
@@ -1105,6 +1110,10 @@ static int run_step(slosh_pipeline *pl, slosh_data *d, hipStream_t st, const slo
     t.blk_start = d->blk_start[cur_g];
     t.blk_cnt = d->blk_cnt[cur_g];
     t.stay = d->stay[cur_g];
+    t.items = d->items;
+    t.item_start = d->item_start;
+    t.n_items = ctr_set(d, cur_g) + CTR_ITEMS;
+    t.taken = d->taken;
     t.bin = d->bin;
     t.mcount = d->mcount[cur_g];
     t.mlist = d->mlist;
@@ -1143,7 +1152,6 @@ static int run_step(slosh_pipeline *pl, slosh_data *d, hipStream_t st, const slo
     if (hooks && hooks->after_grid_update && hooks->after_grid_update(d, st, hs) != 0)
         return fail(SLOSH_E_HOOK, "after_grid_update hook failed");
 
-    if (p2g_by_hook) next.prime = 0u;  // the table of the next substep was not reset
     BodyBuffers bb;
     bb.poses = d->poses;
     bb.vels = d->vels;
@@ -1155,7 +1163,8 @@ static int run_step(slosh_pipeline *pl, slosh_data *d, hipStream_t st, const slo
     if (hooks && hooks->run_g2p && hooks->run_g2p(d, st, hs, &handled) != 0)
         return fail(SLOSH_E_HOOK, "run_g2p hook failed");
     const bool g2p_by_hook = handled != 0;
-    const bool split = g2p_by_hook || (hooks && hooks->after_g2p) || !K.particles_update;
+    // (A P2G hook leaves the fused kernel's item starts unwritten.)
+    const bool split = g2p_by_hook || p2g_by_hook || (hooks && hooks->after_g2p) || !K.particles_update;
     if (!g2p_by_hook && !K.builtin_transfers)
         return fail(SLOSH_E_NO_KERNELS, "pipeline built without builtin transfer kernels; a hook must handle run_g2p");
     if (!split) {
@@ -1302,6 +1311,8 @@ static void free_data(slosh_data *d) {
     dfree(d->cell_start);
     dfree(d->mlist);
     dfree(d->bin);
+    dfree(d->item_start);
+    dfree(d->taken);
     dfree(d->blk_tile_sums);
     dfree(d->counters);
     dfree(d->tiles);
@@ -1476,6 +1487,8 @@ static int create_impl(slosh_pipeline *pipeline, const slosh_sim_params *params,
     TRY(dalloc(&d->cell_start, cap * NODES_PER_BLOCK));
     TRY(dalloc(&d->mlist, cap * MOVER_CAP));
     TRY(dalloc(&d->bin, cap));
+    TRY(dalloc(&d->item_start, cap));
+    TRY(dalloc(&d->taken, cap));
     TRY(dalloc(&d->blk_tile_sums, (cap + 4095) / 4096 + 1));
     TRY(dalloc(&d->counters, 16));
     HIP_TRY(hipMemset(d->counters, 0, 64));
