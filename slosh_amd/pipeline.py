@@ -311,17 +311,17 @@ class MpmData:
         _lib.check(_lib.load().slosh_check_errors(self.handle, self._s(stream)))
 
     def positions(self, stream=None):
-        out = np.zeros((self.n, 4), np.float32)
+        out = np.empty((self.n, 4), np.float32)
         _lib.check(_lib.load().slosh_read_positions(self.handle, self._s(stream), _p(out)))
         return out
 
     def kinematics(self, stream=None):
-        out = np.zeros(self.n, L.KINEMATICS)
+        out = np.empty(self.n, L.KINEMATICS)
         _lib.check(_lib.load().slosh_read_kinematics(self.handle, self._s(stream), _p(out)))
         return out
 
     def def_grad(self, stream=None):
-        out = np.zeros((self.n, 3, 4), np.float32)
+        out = np.empty((self.n, 3, 4), np.float32)
         _lib.check(_lib.load().slosh_read_def_grad(self.handle, self._s(stream), _p(out)))
         return out
 
