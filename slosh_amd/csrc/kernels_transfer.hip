@@ -20,6 +20,8 @@
 //   k_g2p / k_particle_update  the same two stages as separate in-place
 //                    kernels, used when a hook replaces or observes G2P.
 //   k_rigid_update   rigid_impulses.slang:70-121.
+#include <type_traits>
+
 #include "launch.h"
 #include "../../include/slosh_hip.h"
 
@@ -692,6 +694,10 @@ struct Colliders {
     uint32_t count;
     const float4 *mesh_vtx;   // trimesh collision vertices: BVH AABBs, vertices, pseudo-normals
     const uint32_t *mesh_idx; // trimesh collision indices: BVH topology, triangles
+    // The BVHs of the trimesh bodies as the walk reads them (see pack_meshes), and
+    // each body's first node.
+    const float4 *mesh_nodes, *mesh_leaves;
+    const uint32_t *mesh_base;
 };
 
 // triangle_project_local_point_and_get_location (trimesh.slang:304-377): closest
@@ -751,67 +757,162 @@ __device__ inline float3 triangle_project(float3 a, float3 b, float3 c, float3 p
     return p;
 }
 
-// TriMesh::project_local_point (trimesh.slang:111-154): the closest triangle within
-// max_dist by the stackless BVH walk (links point forward, checked on the host, so
-// the walk ends after at most `nodes` steps), inside by the pseudo-normal of the
-// feature the point projects on. Returns whether a triangle was found.
-__device__ inline bool trimesh_project(const Colliders &cs, float4 a, float4 b, float3 pt, float max_dist,
-                                       float3 *out, bool *inside) {
+// Distance of a point from a box (0 inside), in the operation order of the BVH walk.
+__device__ inline float box_distance(float4 mn, float4 mx, float3 pt) {
 #pragma clang fp contract(off)
-    const uint32_t vroot = __float_as_uint(a.x), iroot = __float_as_uint(a.y), nodes = __float_as_uint(a.z);
-    const uint32_t nvert = __float_as_uint(b.y);
-    const uint32_t *topo = cs.mesh_idx + iroot;
-    const uint32_t *tri_idx = topo + 3u * nodes;
-    const float4 *verts = cs.mesh_vtx + vroot + 2u * nodes;
+    const float qx = (pt.x + (fmaxf(mn.x - pt.x, 0.0f) - fmaxf(pt.x - mx.x, 0.0f))) - pt.x;
+    const float qy = (pt.y + (fmaxf(mn.y - pt.y, 0.0f) - fmaxf(pt.y - mx.y, 0.0f))) - pt.y;
+    const float qz = (pt.z + (fmaxf(mn.z - pt.z, 0.0f) - fmaxf(pt.z - mx.z, 0.0f))) - pt.z;
+    return sqrtf(qx * qx + qy * qy + qz * qz);
+}
+
+// The closest point of the triangle of BVH leaf `leaf` (3 vertices, the triangle
+// index in the first one's w), its distance and the feature it lies on.
+__device__ inline float leaf_distance(const float4 *__restrict__ leaf, float3 pt, float3 *p, uint32_t *tri,
+                                      uint32_t *feat, uint32_t *id) {
+#pragma clang fp contract(off)
+    const float4 va = leaf[0], vb = leaf[1], vc = leaf[2];
+    *tri = __float_as_uint(va.w);
+    *p = triangle_project(make_float3(va.x, va.y, va.z), make_float3(vb.x, vb.y, vb.z), make_float3(vc.x, vc.y, vc.z),
+                          pt, feat, id);
+    const float dx = p->x - pt.x, dy = p->y - pt.y, dz = p->z - pt.z;
+    return sqrtf(dx * dx + dy * dy + dz * dz);
+}
+
+// TriMesh::project_local_point (trimesh.slang:111-154): the leaf of the closest
+// triangle within max_dist by the stackless BVH walk (SLOSH_NONE: none; links point
+// forward, checked on the host, so the walk ends). The lanes of a wave hold
+// neighbouring nodes and visit mostly the same BVH nodes, so they walk together: each
+// step takes the first node any lane is at, which makes its record one scalar load,
+// and the lanes that are there test it. Every lane still visits its own nodes in its
+// own order. A lane skips a leaf whose box (grown by 1 % on the host, far above
+// rounding) is farther than its best so far, which the reference tests all the same;
+// its triangle cannot win.
+__device__ inline uint32_t trimesh_walk(const float4 *__restrict__ node, const float4 *__restrict__ leaf,
+                                        uint32_t nodes, float3 pt, float max_dist) {
     float best = max_dist;
-    float3 best_p = pt;
-    uint32_t best_tri = 0u, best_feat = 3u, best_id = 0u;
-    bool found = false;
-    uint32_t cur = 0u;
-    for (uint32_t steps = 0; cur < nodes && steps < nodes; steps++) {
-        const uint32_t entry = topo[3u * cur], exit_ = topo[3u * cur + 1u];
-        if (entry == 0xffffffffu) {
-            const uint32_t tri = topo[3u * cur + 2u];
-            const float4 va = verts[tri_idx[3u * tri]], vb = verts[tri_idx[3u * tri + 1u]],
-                         vc = verts[tri_idx[3u * tri + 2u]];
-            uint32_t feat, id;
-            const float3 p = triangle_project(make_float3(va.x, va.y, va.z), make_float3(vb.x, vb.y, vb.z),
-                                              make_float3(vc.x, vc.y, vc.z), pt, &feat, &id);
-            const float dx = p.x - pt.x, dy = p.y - pt.y, dz = p.z - pt.z;
-            const float dist = sqrtf(dx * dx + dy * dy + dz * dz);
-            if (dist <= best) {
-                best = dist;
-                best_p = p;
-                best_tri = tri; best_feat = feat; best_id = id;
-                found = true;
+    uint32_t best_leaf = SLOSH_NONE;
+    uint32_t cur = 0u, at = 0u;  // this lane's next node, the wave's
+    while (at < nodes) {
+        const float4 mn = node[2u * at], mx = node[2u * at + 1u];
+        const uint32_t entry = __float_as_uint(mn.w), exit_ = __float_as_uint(mx.w);
+        if (cur == at) {
+            const float dbox = box_distance(mn, mx, pt);
+            const bool is_leaf = entry == SLOSH_NONE;
+            cur = !is_leaf && dbox < best ? entry : exit_;
+            if (is_leaf && dbox <= best) {
+                float3 p;
+                uint32_t tri, feat, id;
+                const float dist = leaf_distance(leaf + 3u * (size_t)at, pt, &p, &tri, &feat, &id);
+                if (dist <= best) {
+                    best = dist;
+                    best_leaf = at;
+                }
             }
-            cur = exit_;
+        }
+        // The first node a lane is at now: usually the next one.
+        if (__ballot(cur == at + 1u)) {
+            at = at + 1u;
         } else {
-            const float4 mn = cs.mesh_vtx[vroot + 2u * cur], mx = cs.mesh_vtx[vroot + 2u * cur + 1u];
-            const float qx = (pt.x + (fmaxf(mn.x - pt.x, 0.0f) - fmaxf(pt.x - mx.x, 0.0f))) - pt.x;
-            const float qy = (pt.y + (fmaxf(mn.y - pt.y, 0.0f) - fmaxf(pt.y - mx.y, 0.0f))) - pt.y;
-            const float qz = (pt.z + (fmaxf(mn.z - pt.z, 0.0f) - fmaxf(pt.z - mx.z, 0.0f))) - pt.z;
-            cur = sqrtf(qx * qx + qy * qy + qz * qz) < best ? entry : exit_;
+            uint32_t m = __builtin_amdgcn_readfirstlane(cur);
+            for (uint64_t less = __ballot(cur < m); less; less = __ballot(cur < m))
+                m = __builtin_amdgcn_readlane(cur, __ffsll((unsigned long long)less) - 1);
+            at = m;
         }
     }
-    if (!found) return false;
-    // TriMesh::pseudo_normal (trimesh.slang:83-109)
+    return best_leaf;
+}
+
+// The projection on leaf `lf` of trimesh collider `i`, and TriMesh::pseudo_normal
+// (trimesh.slang:83-109) of the feature it lies on, which tells inside from outside.
+__device__ inline void trimesh_contact(const Colliders &cs, uint32_t i, uint32_t lf, float3 pt, float3 *out,
+                                       bool *inside) {
+#pragma clang fp contract(off)
+    const float4 a = cs.shapes[2 * i], b = cs.shapes[2 * i + 1];
+    const uint32_t vroot = __float_as_uint(a.x), iroot = __float_as_uint(a.y), nodes = __float_as_uint(a.z);
+    const uint32_t nvert = __float_as_uint(b.y);
+    const uint32_t *tri_idx = cs.mesh_idx + iroot + 3u * nodes;
+    const float4 *verts = cs.mesh_vtx + vroot + 2u * nodes;
+    uint32_t tri, feat, id;
+    leaf_distance(cs.mesh_leaves + 3u * (size_t)(cs.mesh_base[i] + lf), pt, out, &tri, &feat, &id);
     float3 pn;
-    const uint32_t *tv = tri_idx + 3u * best_tri;
-    if (best_feat == 0u) {
-        const float4 q = verts[tv[best_id] + nvert];
+    const uint32_t *tv = tri_idx + 3u * tri;
+    if (feat == 0u) {
+        const float4 q = verts[tv[id] + nvert];
         pn = make_float3(q.x, q.y, q.z);
-    } else if (best_feat == 1u) {
-        const float4 q = verts[2u * nvert + 3u * best_tri + best_id];
+    } else if (feat == 1u) {
+        const float4 q = verts[2u * nvert + 3u * tri + id];
         pn = make_float3(q.x, q.y, q.z);
     } else {
         const float4 va = verts[tv[0]], vb = verts[tv[1]], vc = verts[tv[2]];
         pn = cross3f(make_float3(vb.x - va.x, vb.y - va.y, vb.z - va.z),
                      make_float3(vc.x - va.x, vc.y - va.y, vc.z - va.z));
     }
-    *inside = pn.x * (pt.x - best_p.x) + pn.y * (pt.y - best_p.y) + pn.z * (pt.z - best_p.z) <= 0.0f;
-    *out = best_p;
-    return true;
+    *inside = pn.x * (pt.x - out->x) + pn.y * (pt.y - out->y) + pn.z * (pt.z - out->z) <= 0.0f;
+}
+
+// The closest triangles of a block's 64 nodes by a workgroup of MESH_WAVES waves,
+// for every trimesh collider: one wave collects the leaves near the block, a level of
+// the BVH at a time; then each wave tests its share of them for all nodes (lane =
+// node) and the closest wins by an LDS minimum over (distance, later leaf first),
+// the order the walk decides ties in.
+//
+// Bound by latency: a block is 64 nodes with ~50 triangles in reach, and one triangle
+// test ~300 dependent instructions, so one wave per block left the chip idle. The
+// grid update of 85k particles over an 874-triangle heightfield (429 blocks): walked
+// per lane 110 us, walked by the wave together 114 us, shared by 8 waves 29 us (4 waves 37, 16 waves 48).
+#define MESH_WAVES 8
+#define MESH_CAND 512  // leaves near a block that the workgroup shares; more are walked
+#define MESH_FRONT 256
+struct MeshShared {
+    uint32_t cand[MESH_CAND];
+    uint32_t front[2][MESH_FRONT];
+    uint32_t n_cand;  // SLOSH_NONE: more than fit
+    unsigned long long key[SLOSH_MAX_COLLIDERS][NODES_PER_BLOCK];  // all ones: none in reach
+};
+
+// Appends `v` of the lanes in `on` to list[0, *n) (wave-uniform *n); false if it does not fit.
+__device__ inline bool push(uint32_t *list, uint32_t cap, uint32_t *n, bool on, uint32_t v) {
+    const uint64_t m = __ballot(on);
+    const uint32_t at = *n + (uint32_t)__popcll(m & lanemask_lt());
+    if (on && at < cap) list[at] = v;
+    *n += (uint32_t)__popcll(m);
+    return *n <= cap;
+}
+
+// Leaves of trimesh `node` whose boxes come within `reach` of the box c +- e, into
+// S.cand; by one wave.
+__device__ inline void mesh_candidates(MeshShared &S, const float4 *__restrict__ node, float3 c, float3 e,
+                                       float reach) {
+    const uint32_t lane = lane_id();
+    uint32_t n_cand = 0u, nf = 1u, cur = 0u;
+    bool fits = true;
+    if (lane == 0) S.front[0][0] = 0u;
+    while (nf > 0u && fits) {
+        uint32_t next = 0u;
+        for (uint32_t b = 0; b < nf && fits; b += 64u) {
+            __asm__ volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            const bool have = b + lane < nf;
+            const uint32_t k = have ? S.front[cur][b + lane] : 0u;
+            const float4 mn = node[2u * k], mx = node[2u * k + 1u];
+            const float gx = fmaxf(fmaxf(mn.x - (c.x + e.x), (c.x - e.x) - mx.x), 0.0f);
+            const float gy = fmaxf(fmaxf(mn.y - (c.y + e.y), (c.y - e.y) - mx.y), 0.0f);
+            const float gz = fmaxf(fmaxf(mn.z - (c.z + e.z), (c.z - e.z) - mx.z), 0.0f);
+            const bool near = have && gx * gx + gy * gy + gz * gz <= reach * reach;
+            const uint32_t entry = __float_as_uint(mn.w), end = __float_as_uint(mx.w);
+            fits = push(S.cand, MESH_CAND, &n_cand, near && entry == SLOSH_NONE, k);
+            // The children: the entry, then each child's exit up to this node's.
+            uint32_t ch = near && entry != SLOSH_NONE ? entry : end;
+            while (fits && __ballot(ch != end)) {
+                const bool on = ch != end;
+                fits = push(S.front[cur ^ 1u], MESH_FRONT, &next, on, ch);
+                if (on) ch = __float_as_uint(node[2u * ch + 1u].w);
+            }
+        }
+        cur ^= 1u;
+        nf = next;
+    }
+    if (lane == 0) S.n_cand = fits ? n_cand : SLOSH_NONE;
 }
 
 struct NodeColl {
@@ -873,9 +974,11 @@ __device__ inline void collider_box(const Colliders &cs, uint32_t i, float reach
     *hi = make_float4(cw.x + ext.x + m, cw.y + ext.y + m, cw.z + ext.z + m, 0.0f);
 }
 
-// `box`: collider_box of each collider (reach 1.5 h).
+// `box`: collider_box of each collider (reach 1.5 h). `keys`: per trimesh collider the
+// point's closest leaf (MeshShared::key at the point's node).
 template <bool MESH>
-__device__ inline NodeColl collide(const Colliders &cs, const float4 *box, float h, float3 point) {
+__device__ inline NodeColl collide(const Colliders &cs, const float4 *box, float h, float3 point,
+                                   const unsigned long long (*keys)[NODES_PER_BLOCK], uint32_t lane) {
 #pragma clang fp contract(off)
     NodeColl c;
     c.normal_id = make_float4(0.0f, 0.0f, 0.0f, __uint_as_float(0u));
@@ -894,10 +997,10 @@ __device__ inline NodeColl collide(const Colliders &cs, const float4 *box, float
         bool inside = false;
         if (MESH && ty == 6u) {
             // collide.slang:120-130: only a triangle within dist_cap counts.
+            const unsigned long long key = keys[i][lane];
+            if (key == ~0ull) continue;
             float3 lproj;
-            if (!trimesh_project(cs, a, cs.shapes[2 * i + 1], sim_inv_mul_pt(rot, ts, point), dist_cap, &lproj,
-                                 &inside))
-                continue;
+            trimesh_contact(cs, i, ~(uint32_t)key, sim_inv_mul_pt(rot, ts, point), &lproj, &inside);
             proj = sim_mul_pt(rot, ts, lproj);
         } else if (ty <= 4u) {
             float3 lp = sim_inv_mul_pt(rot, ts, point);
@@ -1613,6 +1716,71 @@ __global__ __launch_bounds__(192, P2G_CHUNK <= 384 ? 4 : 1) void k_p2g(StepParam
     }
 }
 
+// The closest leaves of a block's nodes (lane = node, at cell_pos; those in `need`)
+// for every trimesh collider into S.key, by the whole workgroup.
+__device__ inline void mesh_queries(const Colliders &cs, const float4 *box, MeshShared &S, float h, float3 cell_pos,
+                                    bool need) {
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const float cap = h * 1.5f;
+    for (uint32_t i = 0; i < cs.count; i++) {
+        const float4 a = cs.shapes[2 * i];
+        if (__float_as_uint(a.w) != 6u) continue;
+        const float4 lo = box[2 * i], hi = box[2 * i + 1];
+        const bool on = need && cell_pos.x >= lo.x && cell_pos.x <= hi.x && cell_pos.y >= lo.y && cell_pos.y <= hi.y &&
+                        cell_pos.z >= lo.z && cell_pos.z <= hi.z;
+        if (wave == 0u) S.key[i][lane] = ~0ull;
+        if (__ballot(on) == 0ull) continue;  // (every wave holds the same nodes)
+        const float4 rot = cs.poses[2 * i], ts = cs.poses[2 * i + 1];
+        const uint32_t base = cs.mesh_base[i];
+        const float4 *node = cs.mesh_nodes + 2u * (size_t)base, *leaf = cs.mesh_leaves + 3u * (size_t)base;
+        const float3 pt = sim_inv_mul_pt(rot, ts, cell_pos);
+        if (wave == 0u) {
+            // The block's box in the mesh's frame, from its first node.
+            const float3 w0 = make_float3(__shfl(cell_pos.x, 0), __shfl(cell_pos.y, 0), __shfl(cell_pos.z, 0));
+            const float3 c = sim_inv_mul_pt(rot, ts, make_float3(w0.x + cap, w0.y + cap, w0.z + cap));
+            const float4 inv = make_float4(-rot.x, -rot.y, -rot.z, rot.w);
+            const float3 ix = quat_rotate(inv, make_float3(1.0f, 0.0f, 0.0f));
+            const float3 iy = quat_rotate(inv, make_float3(0.0f, 1.0f, 0.0f));
+            const float3 iz = quat_rotate(inv, make_float3(0.0f, 0.0f, 1.0f));
+            const float s = 1.001f * cap / fabsf(ts.w);
+            const float3 e = make_float3((fabsf(ix.x) + fabsf(iy.x) + fabsf(iz.x)) * s,
+                                         (fabsf(ix.y) + fabsf(iy.y) + fabsf(iz.y)) * s,
+                                         (fabsf(ix.z) + fabsf(iy.z) + fabsf(iz.z)) * s);
+            const float size = fmaxf(fmaxf(fabsf(c.x), fabsf(c.y)), fabsf(c.z));
+            mesh_candidates(S, node, c, e, 1.001f * cap + 1.0e-5f * size);
+        }
+        __syncthreads();
+        const uint32_t n = S.n_cand;
+        if (n == SLOSH_NONE) {
+            if (wave == 0u && on) {
+                const uint32_t lf = trimesh_walk(node, leaf, __float_as_uint(a.z), pt, cap);
+                if (lf != SLOSH_NONE) S.key[i][lane] = (unsigned long long)~lf;
+            }
+        } else {
+            float best = cap;
+            unsigned long long key = ((unsigned long long)__float_as_uint(cap) << 32) | 0xffffffffull;
+            bool found = false;
+            for (uint32_t q = wave; q < n; q += MESH_WAVES) {
+                const uint32_t lf = __builtin_amdgcn_readfirstlane(S.cand[q]);
+                if (on && box_distance(node[2u * lf], node[2u * lf + 1u], pt) <= best) {
+                    float3 p;
+                    uint32_t tri, feat, id;
+                    const float dist = leaf_distance(leaf + 3u * (size_t)lf, pt, &p, &tri, &feat, &id);
+                    const unsigned long long k = ((unsigned long long)__float_as_uint(dist) << 32) | (uint32_t)~lf;
+                    if (dist <= best && k < key) {
+                        best = dist;
+                        key = k;
+                        found = true;
+                    }
+                }
+            }
+            if (found) atomicMin(&S.key[i][lane], key);
+        }
+        __syncthreads();
+    }
+}
+
 // The work list of the fused G2P kernel: an item is 64 consecutive entries of a
 // block's sequence (header id, index of the 64).
 struct ItemLists {
@@ -1643,7 +1811,7 @@ __device__ inline void write_items(const Members &M, const ItemLists &L, uint32_
 // mode 0: node momentum from tiles; mode 1: nodes already hold momentum (P2G hook).
 // do_update 0: only combine tiles (grid update disabled).
 template <bool MESH>
-__global__ __launch_bounds__(256) void k_grid_update(StepParams P, const float4 *__restrict__ tiles,
+__global__ __launch_bounds__(MESH ? 64 * MESH_WAVES : 256) void k_grid_update(StepParams P, const float4 *__restrict__ tiles,
                                                      float4 *__restrict__ nodes, const uint32_t *__restrict__ nbr,
                                                      const uint32_t *__restrict__ blist,
                                                      const uint32_t *__restrict__ keys, Colliders cs,
@@ -1658,12 +1826,16 @@ __global__ __launch_bounds__(256) void k_grid_update(StepParams P, const float4 
     const uint32_t B = counters[CTR_NUM_BLOCKS];
     const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63u;
     const int x = lane & 3, y = (lane >> 2) & 3, z = lane >> 4;
-    const uint32_t waves_per_grid = gridDim.x * 4;
-    for (uint32_t k = blockIdx.x * 4 + wave; k < B; k += waves_per_grid) {
+    // With trimesh colliders a workgroup shares one block: every wave holds its nodes
+    // (and takes part in mesh_queries), the first one writes them.
+    __shared__ typename std::conditional<MESH, MeshShared, char>::type shared;
+    const uint32_t first = MESH ? blockIdx.x : blockIdx.x * 4 + wave, step = MESH ? gridDim.x : gridDim.x * 4;
+    const bool owner = !MESH || wave == 0u;
+    for (uint32_t k = first; k < B; k += step) {
         const uint32_t hid = blist[k];
         float4 acc;
         if (mode == 0) {
-            write_items(M, L, hid, lane);
+            if (owner) write_items(M, L, hid, lane);
             // Tiles of blocks without particles were not written (they count as
             // zero). Each tile value is loaded together with its block's particle
             // count and then selected by it, so the tile loads wait only for the
@@ -1708,8 +1880,9 @@ __global__ __launch_bounds__(256) void k_grid_update(StepParams P, const float4 
         } else {
             acc = nodes[(size_t)hid * NODES_PER_BLOCK + lane];
         }
+        if (MESH) __syncthreads();  // every wave has read the nodes (mode 1) and is done with the last block
         if (!do_update) {
-            nodes[(size_t)hid * NODES_PER_BLOCK + lane] = acc;
+            if (owner) nodes[(size_t)hid * NODES_PER_BLOCK + lane] = acc;
             continue;
         }
         int bx, by, bz;
@@ -1725,18 +1898,25 @@ __global__ __launch_bounds__(256) void k_grid_update(StepParams P, const float4 
         v.x = fminf(fmaxf((acc.x + mass * P.gravity[0] * dt) * inv_mass, -lim), lim);
         v.y = fminf(fmaxf((acc.y + mass * P.gravity[1] * dt) * inv_mass, -lim), lim);
         v.z = fminf(fmaxf((acc.z + mass * P.gravity[2] * dt) * inv_mass, -lim), lim);
+        const uint32_t prev = P.coll_cache ? nbr[(size_t)hid * NBR_STRIDE + NBR_PREV] : SLOSH_NONE;
+        const unsigned long long(*mesh_keys)[NODES_PER_BLOCK] = nullptr;
+        if constexpr (MESH) {
+            mesh_queries(cs, cbox, shared, h, cell_pos,
+                         P.coll_cache ? prev == SLOSH_NONE || coll_prev == nullptr : mass > 0.0f);
+            if (!owner) continue;
+            mesh_keys = shared.key;
+        }
         if (cs.count > 0) {
             NodeColl c;
             bool have = true;
             if (P.coll_cache) {
-                uint32_t prev = nbr[(size_t)hid * NBR_STRIDE + NBR_PREV];
                 if (prev != SLOSH_NONE && coll_prev != nullptr) c = coll_prev[(size_t)prev * NODES_PER_BLOCK + lane];
-                else c = collide<MESH>(cs, cbox, h, cell_pos);
+                else c = collide<MESH>(cs, cbox, h, cell_pos, mesh_keys, lane);
                 coll_cur[(size_t)hid * NODES_PER_BLOCK + lane] = c;
             } else if (mass > 0.0f) {
                 // Static colliders: the cached record equals a fresh collide(); a
                 // zero-mass node has v = 0, which every boundary condition keeps.
-                c = collide<MESH>(cs, cbox, h, cell_pos);
+                c = collide<MESH>(cs, cbox, h, cell_pos, mesh_keys, lane);
             } else {
                 have = false;
             }
@@ -2350,6 +2530,9 @@ hipError_t launch_grid_update(const StepParams &P, const TransferBuffers &t, con
     cs.count = c.count;
     cs.mesh_vtx = c.mesh_vtx;
     cs.mesh_idx = c.mesh_idx;
+    cs.mesh_nodes = c.mesh_nodes;
+    cs.mesh_leaves = c.mesh_leaves;
+    cs.mesh_base = c.mesh_base;
     ItemLists items;
     items.items = t.items;
     items.item_start = t.item_start;
@@ -2358,8 +2541,8 @@ hipError_t launch_grid_update(const StepParams &P, const TransferBuffers &t, con
     items.fast = t.fast;
     // Trimesh projection (a BVH walk) is compiled into its own instance so that
     // scenes without meshes keep the smaller kernel.
-    launch_kernel(ev, c.mesh_vtx ? k_grid_update<true> : k_grid_update<false>, dim3(block_grid(P, 4)), dim3(256), 0,
-                  stream, P,
+    launch_kernel(ev, c.mesh_vtx ? k_grid_update<true> : k_grid_update<false>, dim3(block_grid(P, c.mesh_vtx ? 1 : 4)),
+                  dim3(c.mesh_vtx ? 64 * MESH_WAVES : 256), 0, stream, P,
                   (const float4 *)t.tiles, t.nodes, t.nbr, t.blist, t.keys, cs, (const NodeColl *)t.coll_prev,
                   (NodeColl *)t.coll_cur, t.counters, members_of(t), items, mode, do_update);
     return hipGetLastError();

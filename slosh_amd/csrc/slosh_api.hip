@@ -207,6 +207,8 @@ struct slosh_data {
     // body is a trimesh, so the buffers are required.
     float *mesh_vtx = nullptr;
     uint32_t *mesh_idx = nullptr;
+    float4 *mesh_nodes = nullptr, *mesh_leaves = nullptr;  // the BVHs as the walk reads them
+    uint32_t *mesh_base = nullptr;
     size_t mesh_nv = 0, mesh_ni = 0;
     bool has_trimesh = false;
     // Pinned host arenas that appends stage particles in, each reused once the
@@ -1150,6 +1152,9 @@ static int run_step(slosh_pipeline *pl, slosh_data *d, hipStream_t st, const slo
     cb.count = d->nbodies;
     cb.mesh_vtx = d->has_trimesh ? (const float4 *)d->mesh_vtx : nullptr;
     cb.mesh_idx = d->has_trimesh ? d->mesh_idx : nullptr;
+    cb.mesh_nodes = d->mesh_nodes;
+    cb.mesh_leaves = d->mesh_leaves;
+    cb.mesh_base = d->mesh_base;
     if (K.grid_update || !p2g_by_hook) {
         const uint32_t mode = p2g_by_hook ? 1u : 0u;
         HIP_TRY(launch_grid_update(P, t, cb, mode, K.grid_update ? 1u : 0u, pass_events(ts, PASS_GRID_UPDATE, &pe),
@@ -1457,6 +1462,9 @@ static void free_data(slosh_data *d) {
     dfree(d->scene_rec);
     dfree(d->mesh_vtx);
     dfree(d->mesh_idx);
+    dfree(d->mesh_nodes);
+    dfree(d->mesh_leaves);
+    dfree(d->mesh_base);
     dfree(d->dt_bound);
     release_ring(d);
     for (hipEvent_t e : d->ring_events) (void)hipEventDestroy(e);
@@ -1853,6 +1861,64 @@ void slosh_graph_destroy(slosh_graph *g) {
     delete g;
 }
 
+// The trimesh bodies' BVHs in the layout of the grid update's walk: per node its box
+// with the entry link (all ones: a leaf) and the exit link in the spare components,
+// and for a leaf its triangle's vertices with the triangle index. A leaf's box is that
+// of its triangle (the reference never reads a leaf's own), grown by 1 % of its extent
+// and well above the rounding of its coordinates.
+static int pack_meshes(slosh_data *d, const float *vertices4, const uint32_t *indices) {
+    std::vector<float4> nodes, leaves;
+    std::vector<uint32_t> base(SLOSH_MAX_COLLIDERS, 0u);
+    for (uint32_t b = 0; b < d->nbodies; b++) {
+        const slosh_shape &sh = d->bodies_host[b].shape;
+        if (f2u(sh.a[3]) != 6u) continue;
+        const size_t vroot = f2u(sh.a[0]), iroot = f2u(sh.a[1]), count = f2u(sh.a[2]);
+        base[b] = (uint32_t)(nodes.size() / 2);
+        for (size_t k = 0; k < count; k++) {
+            const uint32_t *nd = indices + iroot + 3 * k;
+            const float *mn = vertices4 + 4 * (vroot + 2 * k), *mx = mn + 4;
+            float lo[3] = {mn[0], mn[1], mn[2]}, hi[3] = {mx[0], mx[1], mx[2]};
+            float4 v[3] = {};
+            if (nd[0] == 0xffffffffu) {
+                const uint32_t *t = indices + iroot + 3 * count + 3 * nd[2];
+                for (int j = 0; j < 3; j++) {
+                    const float *p = vertices4 + 4 * (vroot + 2 * count + t[j]);
+                    v[j] = make_float4(p[0], p[1], p[2], u2f(nd[2]));
+                    for (int c = 0; c < 3; c++) {
+                        lo[c] = j == 0 ? p[c] : std::min(lo[c], p[c]);
+                        hi[c] = j == 0 ? p[c] : std::max(hi[c], p[c]);
+                    }
+                }
+                float extent = 0.0f, size = 0.0f;
+                for (int c = 0; c < 3; c++) {
+                    extent = std::max(extent, hi[c] - lo[c]);
+                    size = std::max({size, std::fabs(lo[c]), std::fabs(hi[c])});
+                }
+                const float grow = 0.01f * extent + 1.0e-5f * size;
+                for (int c = 0; c < 3; c++) {
+                    lo[c] -= grow;
+                    hi[c] += grow;
+                }
+            }
+            nodes.push_back(make_float4(lo[0], lo[1], lo[2], u2f(nd[0])));
+            nodes.push_back(make_float4(hi[0], hi[1], hi[2], u2f(nd[1])));
+            leaves.insert(leaves.end(), v, v + 3);
+        }
+    }
+    dfree(d->mesh_nodes);
+    dfree(d->mesh_leaves);
+    dfree(d->mesh_base);
+    TRY(dalloc(&d->mesh_nodes, std::max<size_t>(nodes.size(), 2)));
+    TRY(dalloc(&d->mesh_leaves, std::max<size_t>(leaves.size(), 3)));
+    TRY(dalloc(&d->mesh_base, base.size()));
+    if (!nodes.empty()) {
+        HIP_TRY(hipMemcpy(d->mesh_nodes, nodes.data(), 16 * nodes.size(), hipMemcpyHostToDevice));
+        HIP_TRY(hipMemcpy(d->mesh_leaves, leaves.data(), 16 * leaves.size(), hipMemcpyHostToDevice));
+    }
+    HIP_TRY(hipMemcpy(d->mesh_base, base.data(), 4 * base.size(), hipMemcpyHostToDevice));
+    return SLOSH_OK;
+}
+
 int slosh_data_set_collision_mesh(slosh_data *d, const float *vertices4, size_t num_vertices,
                                   const uint32_t *indices, size_t num_indices) {
     if (!d) return fail(SLOSH_E_INVALID, "null data");
@@ -1889,6 +1955,8 @@ int slosh_data_set_collision_mesh(slosh_data *d, const float *vertices4, size_t 
                                                      ": the root BVH box does not hold every triangle");
         }
     }
+    invalidate_graphs(d);
+    TRY(pack_meshes(d, vertices4, indices));
     dfree(d->mesh_vtx);
     dfree(d->mesh_idx);
     TRY(dalloc(&d->mesh_vtx, 4 * std::max<size_t>(num_vertices, 1)));
