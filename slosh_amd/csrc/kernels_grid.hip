@@ -8,23 +8,23 @@
 // substep's hash table; the order of the block list differs from the
 // reference's header order (which depends on atomic order as well).
 //
-// Steady state (the previous substep's fused G2P kernel inserted every
-// particle's primary block and its +1 neighbours into this substep's table, wrote
-// each block's particles contiguously with the ones that stay in the block first,
-// and listed the particles that left their block with their new block key):
-//   k_sort_fast        one launch: the block list (occupied slots, workgroup
-//                      scan and one atomic per workgroup), each block's +1 / -1
-//                      neighbour ids and its id in the previous table, and the
-//                      movers bucketed into per-block lists (one lookup and one
-//                      atomic per run of equal keys). A block's particles are
-//                      then the stayers of its previous-substep range plus its
-//                      movers; the per-block kernels read them from there.
+// Steady state: nothing runs here. The previous substep's fused G2P kernel inserted
+// every particle's primary block and its +1 neighbours into this substep's table,
+// appended the new blocks to the regions' lists, wrote each block's particles
+// contiguously and appended the ones that left their block to their new block's list.
+// P2G finds each block's range in the previous storage and looks up its neighbours, and
+// the grid update gives the blocks their storage. (A launch between G2P and P2G for
+// all this took 4-6 us of a substep of a small scene and 21 us of one with 42k blocks.
+// Substep without it, before and after: 2k particles 33.5 -> 30.2 us, 131k 45.5 -> 39.9,
+// 1M 105 -> 97, 2.1M in 42k blocks 652 -> 616.)
 // Full sort (first substep, after host mutations, with hooks):
 //   k_reset_table      hash slots <- NONE, per-step counters <- 0
 //   k_touch_primary    each particle's primary block and its 7 +1 neighbours are
 //                      inserted, once per run of equal keys in a wavefront; the
 //                      thread that creates a block clears its counters
-//   k_sort_fast        (block list and neighbour tables only)
+//   k_block_list       the block list (occupied slots, workgroup scan and one
+//                      atomic per workgroup), each block's +1 / -1 neighbour ids
+//                      and its id in the previous table
 //   k_count            per-particle hash lookup (one per run of equal block keys)
 //                      and per-(block, cell) rank via one aggregated atomic per
 //                      run of equal (block, cell) keys
@@ -40,15 +40,16 @@ constexpr int ASSOC[8][3] = {{0, 0, 0}, {0, 0, 1}, {0, 1, 0}, {0, 1, 1},
                              {1, 0, 0}, {1, 0, 1}, {1, 1, 0}, {1, 1, 1}};
 
 __global__ __launch_bounds__(256) void k_reset_table(uint32_t *__restrict__ keys, uint32_t cap,
-                                                     uint32_t *__restrict__ counters) {
+                                                     uint32_t *__restrict__ counters,
+                                                     unsigned long long *__restrict__ rsum) {
     uint32_t stride = gridDim.x * blockDim.x;
     for (uint32_t s = blockIdx.x * blockDim.x + threadIdx.x; s < cap; s += stride) keys[s] = SLOSH_NONE;
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         counters[CTR_NUM_BLOCKS] = 0u;
         counters[CTR_SORTED_ALLOC] = 0u;
-        counters[CTR_MOVERS] = 0u;
         counters[CTR_OVERFLOW] = 0u;
     }
+    if (blockIdx.x == 0 && threadIdx.x < REGIONS) rsum[threadIdx.x * RSUM_STRIDE] = 0ull;
 }
 
 __global__ __launch_bounds__(256) void k_touch_primary(const float4 *__restrict__ pos, uint32_t n, float h,
@@ -60,28 +61,16 @@ __global__ __launch_bounds__(256) void k_touch_primary(const float4 *__restrict_
     if (valid) key = particle_key(pos[i], h, batched, &cell);
     // One insertion round per run of equal keys: the block and its 7 +1 neighbours.
     const uint64_t heads = run_heads(key, valid) & __ballot(valid);
-    insert_blocks(keys, cap, batched, key, heads, counters, init);
+    ListEntry none;
+    insert_blocks(keys, cap, batched, key, heads, counters, init, none);
 }
-
-struct MoverLists {
-    const uint32_t *key, *slot;  // movers listed by the previous substep (new block key, storage slot)
-    uint32_t *mcount, *mlist;    // per block: movers received, the first MOVER_CAP of them
-    uint32_t *ovf_slot, *ovf_hid;  // the others, with their block
-    // Steady state: per block of the previous table its storage range and stayer
-    // count; per block of this table the same three of its previous-table block
-    // (null in the full sort).
-    const uint32_t *prev_start, *prev_cnt, *prev_stay;
-    uint4 *bin;
-};
 
 // Neighbour table entry `l` (0..15) of block `hid`: [0..6] the +1 neighbours in
 // the reference's associated-block order (grid.slang:362-382), [7] the block's
-// id in the previous substep's table, [8..14] the -1 neighbours. With the
-// previous table's block ranges given, lane 7 also records the block's range in
-// the previous substep's storage and its stayer count.
+// id in the previous substep's table, [8..14] the -1 neighbours.
 __device__ inline void block_neighbour(uint32_t hid, uint32_t key, uint32_t l, uint32_t *__restrict__ nbr,
                                        const uint32_t *__restrict__ keys, const uint32_t *__restrict__ prev_keys,
-                                       uint32_t cap, uint32_t batched, const MoverLists &mv) {
+                                       uint32_t cap, uint32_t batched) {
     int bx, by, bz;
     uint32_t scene;
     unpack_key(batched, key, &bx, &by, &bz, &scene);
@@ -91,11 +80,6 @@ __device__ inline void block_neighbour(uint32_t hid, uint32_t key, uint32_t l, u
         out = hash_find(keys, cap, pack_key(batched, scene, bx + o[0], by + o[1], bz + o[2]));
     } else if (l == NBR_PREV) {
         out = hash_find(prev_keys, cap, key);
-        if (mv.bin) {
-            uint4 r = make_uint4(0u, 0u, 0u, 0u);
-            if (out != SLOSH_NONE) r = make_uint4(mv.prev_start[out], mv.prev_cnt[out], mv.prev_stay[out], 0u);
-            mv.bin[hid] = r;
-        }
     } else if (l >= NBR_MINUS && l < NBR_MINUS + 7) {
         const int *o = ASSOC[l - NBR_MINUS + 1];
         out = hash_find(keys, cap, pack_key(batched, scene, bx - o[0], by - o[1], bz - o[2]));
@@ -103,65 +87,22 @@ __device__ inline void block_neighbour(uint32_t hid, uint32_t key, uint32_t l, u
     nbr[(size_t)hid * NBR_STRIDE + l] = out;
 }
 
-
-// The sort of a steady-state substep (update_block_particle_count and
-// update_nbh_block_ids, sort.slang:100-246, for a table the previous substep
-// filled), one launch of three kinds of workgroups, in dispatch order:
-// [0, mv_wgs) the listed movers, each appended to its new block's list (one
-// lookup and one atomic per run of equal keys; those beyond a block's MOVER_CAP
-// list slots go to the overflow list with their block); [mv_wgs, mv_wgs +
-// cmp_wgs) the block list: each takes 256 * ITEMS slots and appends the occupied
-// ones (workgroup scan, one atomic); the rest the neighbour tables, 16 lanes per
-// slot, every occupied slot's 15 lookups at once.
+// The block list and the neighbour tables of a full sort, one launch of two kinds of
+// workgroups: [0, cmp_wgs) the block list: each takes 256 * ITEMS slots and appends
+// the occupied ones (workgroup scan, one atomic); the rest the neighbour tables, 16
+// lanes per slot, every occupied slot's 15 lookups at once.
 template <uint32_t ITEMS>
-__global__ __launch_bounds__(256) void k_sort_fast(const uint32_t *__restrict__ keys,
-                                                   const uint32_t *__restrict__ prev_keys, uint32_t cap,
-                                                   uint32_t batched, uint32_t *__restrict__ counters,
-                                                   uint32_t *__restrict__ blist, uint32_t *__restrict__ nbr,
-                                                   uint32_t mv_wgs, uint32_t cmp_wgs, MoverLists mv) {
+__global__ __launch_bounds__(256) void k_block_list(const uint32_t *__restrict__ keys,
+                                                    const uint32_t *__restrict__ prev_keys, uint32_t cap,
+                                                    uint32_t batched, uint32_t *__restrict__ counters,
+                                                    uint32_t *__restrict__ blist, uint32_t *__restrict__ nbr,
+                                                    uint32_t cmp_wgs) {
     __shared__ uint32_t wsum[4];
     __shared__ uint32_t wg_base;
     const uint32_t tid = threadIdx.x, wave = tid >> 6, lane = tid & 63u;
-    if (blockIdx.x < mv_wgs) {
-        // Movers. The loop bound is wavefront-uniform (run detection uses every lane).
-        const uint32_t nmov = counters[CTR_MOVERS];
-        const uint32_t stride = mv_wgs * 256u;
-        for (uint32_t base = blockIdx.x * 256u + wave * 64u; base < nmov; base += stride) {
-            const uint32_t i = base + lane;
-            const bool valid = i < nmov;
-            const uint32_t key = valid ? mv.key[i] : 0u;
-            const uint32_t slot = valid ? mv.slot[i] : 0u;
-            const uint64_t heads = run_heads(key, valid);
-            uint32_t hv = SLOSH_NONE;
-            if (valid && ((heads >> lane) & 1ull)) hv = hash_find(keys, cap, key);
-            const int head = run_head_of(heads);
-            const uint32_t hid = __shfl(hv, head);
-            const bool ok = valid && hid != SLOSH_NONE;
-            if (valid && hid == SLOSH_NONE) atomicOr(&counters[CTR_ERRORS], ERR_LOOKUP);
-            uint32_t r0 = 0u;
-            if (ok && ((heads >> lane) & 1ull)) r0 = atomicAdd(&mv.mcount[hid], run_length(heads));
-            const uint32_t r = __shfl(r0, head) + (lane - (uint32_t)head);
-            const bool over = ok && r >= MOVER_CAP;
-            if (ok && !over) mv.mlist[(size_t)hid * MOVER_CAP + r] = slot;
-            const uint64_t om = __ballot(over);
-            if (om) {
-                const int first = __ffsll((unsigned long long)om) - 1;
-                uint32_t ob = 0u;
-                if ((int)lane == first) ob = atomicAdd(&counters[CTR_OVERFLOW], (uint32_t)__popcll(om));
-                ob = __shfl(ob, first);
-                if (over) {
-                    const uint32_t q = ob + (uint32_t)__popcll(om & lanemask_lt());
-                    mv.ovf_slot[q] = slot;
-                    mv.ovf_hid[q] = hid;
-                }
-            }
-        }
-        return;
-    }
-    if (blockIdx.x < mv_wgs + cmp_wgs) {
-        const uint32_t w = blockIdx.x - mv_wgs;
+    if (blockIdx.x < cmp_wgs) {
         constexpr uint32_t SLOTS = 256u * ITEMS;
-        for (uint32_t base = w * SLOTS; base < cap; base += cmp_wgs * SLOTS) {
+        for (uint32_t base = blockIdx.x * SLOTS; base < cap; base += cmp_wgs * SLOTS) {
             uint32_t occ[ITEMS];
             uint32_t mine = 0;
 #pragma unroll
@@ -194,12 +135,16 @@ __global__ __launch_bounds__(256) void k_sort_fast(const uint32_t *__restrict__ 
         }
         return;
     }
-    const uint32_t nbr_wgs = gridDim.x - mv_wgs - cmp_wgs;
-    for (uint32_t s = (blockIdx.x - mv_wgs - cmp_wgs) * 16u + (tid >> 4); s < cap; s += nbr_wgs * 16u) {
+    const uint32_t nbr_wgs = gridDim.x - cmp_wgs;
+    for (uint32_t s = (blockIdx.x - cmp_wgs) * 16u + (tid >> 4); s < cap; s += nbr_wgs * 16u) {
         const uint32_t key = keys[s];
-        if (key != SLOSH_NONE) block_neighbour(s, key, tid & 15u, nbr, keys, prev_keys, cap, batched, mv);
+        if (key != SLOSH_NONE) block_neighbour(s, key, tid & 15u, nbr, keys, prev_keys, cap, batched);
     }
 }
+
+// Stands for the sort in a timed steady-state substep, so that each pass is counted
+// once per substep (its work is done by the kernels around it).
+__global__ void k_no_sort() {}
 
 // update_block_particle_count (sort.slang:208-246) of the full sort: block
 // totals and per-(block, cell) ranks.
@@ -389,54 +334,37 @@ __global__ __launch_bounds__(256) void k_scatter(const uint32_t *__restrict__ ps
 static inline uint32_t div_up(uint64_t a, uint32_t b) { return (uint32_t)((a + b - 1) / b); }
 static inline uint32_t min_u(uint32_t a, uint32_t b) { return a < b ? a : b; }
 
-// `fast`: the previous substep's fused G2P kernel filled this table, wrote every
-// block's stayers first and listed the movers; one launch then sorts. Otherwise
-// the full sort. `ev` (optional) brackets the whole sequence.
+// `fast`: the previous substep's fused kernels prepared this table. Otherwise the full
+// sort. `ev` (optional) brackets the whole sequence.
 hipError_t launch_grid_build(const GridBuffers &g, const float4 *pos, uint32_t n, float h, uint32_t batched,
                              uint32_t cap, bool fast, const PassEvents *ev, hipStream_t stream) {
+    if (fast) {
+        if (ev) launch_kernel(ev, k_no_sort, dim3(1), dim3(64), 0, stream);
+        return hipGetLastError();
+    }
     const uint32_t slot_grid = min_u(div_up(cap, 256), 2048);
     const uint32_t part_grid = div_up(n, 256);
-    MoverLists mv;
-    mv.key = g.mv_key;
-    mv.slot = g.mv_slot;
-    mv.mcount = g.mcount;
-    mv.mlist = g.mlist;
-    mv.ovf_slot = g.ovf_slot;
-    mv.ovf_hid = g.ovf_hid;
-    mv.prev_start = fast ? g.prev_start : nullptr;
-    mv.prev_cnt = fast ? g.prev_cnt : nullptr;
-    mv.prev_stay = fast ? g.prev_stay : nullptr;
-    mv.bin = fast ? g.bin : nullptr;
     const bool wide = cap > 65536u;
     const uint32_t cmp_wgs = wide ? min_u(div_up(cap, 2048), 2048) : min_u(div_up(cap, 256), 2048);
     const uint32_t nbr_wgs = min_u(div_up(cap, 16), 4096);
-    auto sort_kernel = wide ? k_sort_fast<8> : k_sort_fast<1>;
-    if (fast) {
-        // Grid-stride over the movers (their count is on the device).
-        const uint32_t mv_wgs = n > 0 ? min_u(div_up(n, 4096), 1024) : 0u;
-        launch_kernel(ev, sort_kernel, dim3(mv_wgs + cmp_wgs + nbr_wgs), dim3(256), 0, stream,
-                      (const uint32_t *)g.keys, (const uint32_t *)g.prev_keys, cap, batched, g.counters, g.blist,
-                      g.nbr, mv_wgs, cmp_wgs, mv);
-        return hipGetLastError();
-    }
+    auto list_kernel = wide ? k_block_list<8> : k_block_list<1>;
     PassEvents first, last;
     if (ev) {
         first.start = ev->start;
         last.stop = ev->stop;
     }
     launch_kernel(ev ? &first : nullptr, k_reset_table, dim3(slot_grid), dim3(256), 0, stream, g.keys, cap,
-                  g.counters);
+                  g.counters, g.rsum);
     if (n > 0) {
-        BlockInit init;
-        init.mcount = g.mcount;
+        BlockInit init{};
         init.blk_cnt = g.blk_cnt;
         init.cell_cnt = g.cell_cnt;
         launch_kernel(nullptr, k_touch_primary, dim3(part_grid), dim3(256), 0, stream, pos, n, h, batched, g.keys,
                       cap, g.counters, init);
     }
     const PassEvents *sort_ev = n > 0 ? nullptr : (ev ? &last : nullptr);
-    launch_kernel(sort_ev, sort_kernel, dim3(cmp_wgs + nbr_wgs), dim3(256), 0, stream, (const uint32_t *)g.keys,
-                  (const uint32_t *)g.prev_keys, cap, batched, g.counters, g.blist, g.nbr, 0u, cmp_wgs, mv);
+    launch_kernel(sort_ev, list_kernel, dim3(cmp_wgs + nbr_wgs), dim3(256), 0, stream, (const uint32_t *)g.keys,
+                  (const uint32_t *)g.prev_keys, cap, batched, g.counters, g.blist, g.nbr, cmp_wgs);
     if (n == 0) return hipGetLastError();
     launch_kernel(nullptr, k_count, dim3(part_grid), dim3(256), 0, stream, pos, n, h, batched,
                   (const uint32_t *)g.keys, cap, g.cell_cnt, g.pslot, g.prank, g.counters, g.blk_cnt);

@@ -1283,12 +1283,30 @@ __device__ inline void finish_particle(const StepParams &P, bool ok, float mass,
 struct Members {
     uint32_t fast;
     const uint32_t *blist;                   // block list (header ids = table slots)
-    const uint32_t *nbr;                     // neighbour tables (NBR_PREV: id in the previous table)
-    const uint4 *bin;                        // per block: range (start, count) and stayers of its previous-table block
-    const uint32_t *mcount, *mlist;          // movers received per block, the first MOVER_CAP of them
+    const uint32_t *nbr;                     // neighbour tables
+    const uint4 *bin;                        // per block: its previous-table block's range (start, count) and
+                                             // stayers, the movers it received
+    const uint32_t *mlist;                   // the first MOVER_CAP of them
     const uint32_t *ovf_slot, *ovf_hid;      // the others
     const uint32_t *perm, *blk_start, *blk_cnt;  // the full sort's result
     const uint32_t *counters;                // CTR_NUM_BLOCKS, CTR_OVERFLOW of this substep
+};
+
+// What P2G of a steady-state substep finds and leaves for the kernels after it: the
+// regional block lists, what each block receives (movers; slot, start and count in the
+// previous table), the previous table's keys and stayers; the flat block list, each
+// block's range (Members::bin) and neighbour table.
+struct SortInputs {
+    const uint2 *rlist;
+    const uint4 *arrive;
+    const uint32_t *rcnt, *prev_keys, *prev_stay;
+    uint32_t *blist, *num_blocks, *nbr, *blk_cnt;
+    uint4 *bin;
+    // Per region (slot >> rshift) the sums of its blocks' particles (high word) and G2P
+    // items (low word), and each block's place in them.
+    unsigned long long *rsum;
+    uint2 *rel;
+    uint32_t rshift;
 };
 
 struct BlockRange {
@@ -1301,28 +1319,33 @@ struct BlockRange {
 
 // FAST (a template parameter, so that each kernel instance loads only the
 // buffers of its mode): the steady state's stayer ranges and mover lists.
-template <bool FAST>
-__device__ inline BlockRange block_range(const Members &M, uint32_t hid) {
+__device__ inline BlockRange steady_range(const Members &M, uint32_t hid, uint4 in) {
+    const uint32_t mc = in.w;
     BlockRange r;
-    if constexpr (FAST) {
-        const uint4 in = M.bin[hid];
-        const uint32_t mc = M.mcount[hid];
-        r.cand_lo = in.x;
-        r.cand_n = in.y;
-        r.list = M.mlist + (size_t)hid * MOVER_CAP;
-        r.list_n = mc < MOVER_CAP ? mc : MOVER_CAP;
-        r.total = in.z + mc;
-        r.overflow = mc > MOVER_CAP;
-    } else {
-        r.cand_lo = 0u;
-        r.cand_n = 0u;
-        r.list = M.perm + M.blk_start[hid];
-        r.list_n = M.blk_cnt[hid];
-        r.total = r.list_n;
-        r.overflow = false;
-    }
+    r.cand_lo = in.x;
+    r.cand_n = in.y;
+    r.list = M.mlist + (size_t)hid * MOVER_CAP;
+    r.list_n = mc < MOVER_CAP ? mc : MOVER_CAP;
+    r.total = in.z + mc;
+    r.overflow = mc > MOVER_CAP;
     return r;
 }
+
+template <bool FAST>
+__device__ inline BlockRange block_range(const Members &M, uint32_t hid) {
+    if constexpr (FAST) return steady_range(M, hid, M.bin[hid]);
+    BlockRange r;
+    r.cand_lo = 0u;
+    r.cand_n = 0u;
+    r.list = M.perm + M.blk_start[hid];
+    r.list_n = M.blk_cnt[hid];
+    r.total = r.list_n;
+    r.overflow = false;
+    return r;
+}
+
+// G2P items of a block: 64 entries each.
+__device__ inline uint32_t item_count(const BlockRange &r) { return r.total ? (r.cand_n + r.list_n + 63u) >> 6 : 0u; }
 
 // Storage slot of entry m of a block's sequence (candidates, then list members).
 __device__ inline uint32_t entry_slot(const BlockRange &r, uint32_t m) {
@@ -1356,88 +1379,6 @@ __device__ inline uint32_t entry_slot(const BlockRange &r, uint32_t m) {
 // groups of 16-byte elements.
 __device__ inline uint32_t p2g_slot(uint32_t q) { return q + (q >> 4); }
 
-// Next substep's hash table, reset here and filled with primary blocks by the
-// fused G2P / particle-update kernel (replaces k_reset_table + k_touch_primary
-// of the next substep).
-struct NextTable {
-    uint32_t *keys, *counters;
-    uint32_t prime;
-};
-
-// Per block, in block-list order, by one workgroup of 192 threads: in the steady
-// state its total (stayers of its previous range + movers received) and storage
-// start; in both modes the start of its G2P items (one per 64 entries of its
-// sequence) and, into `counters`, the number of items. Runs beside the per-block
-// work of the same launch (nothing in it reads them).
-template <bool FAST>
-__device__ void p2g_block_scan(const Members &M, uint32_t *__restrict__ blk_start, uint32_t *__restrict__ blk_cnt,
-                               uint32_t *__restrict__ item_start, uint32_t *__restrict__ n_items, uint32_t *wsum) {
-    const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
-    const uint32_t B = M.counters[CTR_NUM_BLOCKS];
-    // 24 entries per thread: up to 4608 blocks in one pass of two dependent loads.
-    constexpr uint32_t PER = 24u, TILE = 192u * PER;
-    uint32_t carry = 0u, icarry = 0u;
-    for (uint32_t base = 0; base < B; base += TILE) {
-        uint32_t hid[PER], c[PER], it[PER];
-#pragma unroll
-        for (uint32_t j = 0; j < PER; j++) {
-            const uint32_t k = base + tid * PER + j;
-            hid[j] = k < B ? M.blist[k] : SLOSH_NONE;
-        }
-        uint32_t t = 0u, ti = 0u;
-#pragma unroll
-        for (uint32_t j = 0; j < PER; j++) {
-            c[j] = 0u;
-            it[j] = 0u;
-            if (hid[j] != SLOSH_NONE) {
-                const BlockRange br = block_range<FAST>(M, hid[j]);
-                c[j] = br.total;
-                it[j] = br.total ? (br.cand_n + br.list_n + 63u) >> 6 : 0u;
-            }
-            t += c[j];
-            ti += it[j];
-        }
-        uint32_t x = t, xi = ti;
-#pragma unroll
-        for (int d = 1; d < 64; d <<= 1) {
-            const uint32_t y = __shfl_up(x, d), yi = __shfl_up(xi, d);
-            if ((int)lane >= d) {
-                x += y;
-                xi += yi;
-            }
-        }
-        if (lane == 63) {
-            wsum[wave] = x;
-            wsum[4 + wave] = xi;
-        }
-        __syncthreads();
-        uint32_t e = carry + x - t, ei = icarry + xi - ti;
-#pragma unroll
-        for (uint32_t w = 0; w < 3; w++) {
-            if (w < wave) {
-                e += wsum[w];
-                ei += wsum[4 + w];
-            }
-            carry += wsum[w];
-            icarry += wsum[4 + w];
-        }
-#pragma unroll
-        for (uint32_t j = 0; j < PER; j++) {
-            if (hid[j] != SLOSH_NONE) {
-                if (FAST) {
-                    blk_start[hid[j]] = e;
-                    blk_cnt[hid[j]] = c[j];
-                }
-                item_start[hid[j]] = ei;
-            }
-            e += c[j];
-            ei += it[j];
-        }
-        __syncthreads();  // wsum is reused by the next tile
-    }
-    if (tid == 0) *n_items = icarry;
-}
-
 // LDS element of node (x, y, z) of a P2G slab tile (z = 0..3), 16-byte elements.
 // Within a z plane, x < 4 maps to x + 4 y (0..23) and x >= 4 to x + 4 y + 24
 // (28..49), one to one;
@@ -1464,7 +1405,7 @@ struct P2GShared {
                               // p2g_chunk before it stages anything
     };
     uint32_t lcnt[64];
-    uint32_t wsum[8];
+    uint32_t wsum[3];
 };
 static_assert(sizeof(float4) * 3 * P2G_SLAB_LDS <= sizeof(P2GShared<192>::sp4),
               "the slab tiles take no LDS beyond the staging of the smallest chunk");
@@ -1542,13 +1483,7 @@ __device__ inline void p2g_chunk(const StepParams &P, P2GShared<P2G_CHUNK> &S, u
     __syncthreads();
     // Every wave scans the 64 counts (lane = cell) and writes the same starts.
     const uint32_t cnt = S.lcnt[lane];
-    uint32_t x = cnt;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-        const uint32_t y = __shfl_up(x, d);
-        if ((int)lane >= d) x += y;
-    }
-    const uint32_t cs = x - cnt;
+    const uint32_t cs = wave_inclusive_scan(cnt) - cnt;
     if (kz == 0) tot += cnt;
     // Each member's cell start from the lane of its cell (every wave holds all 64).
     uint32_t cstart[R];
@@ -1606,51 +1541,108 @@ __device__ inline void p2g_chunk(const StepParams &P, P2GShared<P2G_CHUNK> &S, u
 
 // Chunks of up to 384 members fit in 128 VGPRs (4 waves/SIMD; their LDS allows 5
 // workgroups per CU); 512 needs 132 (3 waves/SIMD, as its 35 KB of LDS allow).
-template <int P2G_CHUNK, bool FAST>
-__global__ __launch_bounds__(192, P2G_CHUNK <= 384 ? 4 : 1) void k_p2g(StepParams P, NextTable nt, const float4 *__restrict__ pos,
-                                             const float4 *__restrict__ vm, const float *__restrict__ C,
-                                             const float *__restrict__ fdt, uint32_t pcap, Members M,
-                                             const uint32_t *__restrict__ keys, float4 *__restrict__ tiles,
-                                             uint32_t *__restrict__ cell_cnt, uint32_t *__restrict__ blk_start_out,
-                                             uint32_t *__restrict__ blk_cnt_out, uint32_t *__restrict__ item_start,
-                                             uint32_t *__restrict__ n_items) {
-    __shared__ P2GShared<P2G_CHUNK> S;
-    if (nt.prime) {
-        for (uint32_t s = blockIdx.x * blockDim.x + threadIdx.x; s < P.cap; s += gridDim.x * blockDim.x)
-            nt.keys[s] = SLOSH_NONE;
-        if (blockIdx.x == 0 && threadIdx.x == 0) {
-            nt.counters[CTR_NUM_BLOCKS] = 0u;
-            nt.counters[CTR_SORTED_ALLOC] = 0u;
-            nt.counters[CTR_MOVERS] = 0u;
-            nt.counters[CTR_OVERFLOW] = 0u;
+//
+// One workgroup per block, the blocks of a region on the XCD that also updates their
+// nodes and particles (xcd_item). In the steady state it starts from the regional
+// lists and finds the block's particles through the previous table.
+// A lane's lookup in progress: its key, the slot probed first and what is there.
+struct Lookup {
+    uint32_t key, slot, seen;
+};
+
+// Entry `lane` (see NBR_STRIDE) of a block's neighbour table: the first probe. Most
+// lookups end there, and the load is in flight through the block's sums.
+__device__ inline void find_neighbours(const StepParams &P, const uint32_t *__restrict__ keys,
+                                       const uint32_t *__restrict__ prev_keys, uint32_t block_key, uint32_t lane,
+                                       Lookup &l) {
+    if (lane >= NBR_MINUS + 7u) return;
+    int bx, by, bz;
+    uint32_t scene;
+    unpack_key(P.batched, block_key, &bx, &by, &bz, &scene);
+    const int d = lane == NBR_PREV ? 0 : (int)(lane & 7u) + 1, s = lane < NBR_MINUS ? 1 : -1;
+    l.key = pack_key(P.batched, scene, bx + s * ((d >> 2) & 1), by + s * ((d >> 1) & 1), bz + s * (d & 1));
+    l.slot = hash_key(l.key) & (P.cap - 1u);
+    l.seen = (lane == NBR_PREV ? prev_keys : keys)[l.slot];
+}
+
+// By P2G's first wave, of a steady-state block: the rest of the lookups, and what the
+// kernels after it read.
+__device__ inline void finish_block(const StepParams &P, const SortInputs &in, const uint32_t *__restrict__ keys,
+                                    uint32_t hid, uint32_t lane, uint4 range, const BlockRange &br, const Lookup &l) {
+    if (lane < NBR_MINUS + 7u) {
+        const uint32_t *table = lane == NBR_PREV ? in.prev_keys : keys;
+        uint32_t slot = l.slot, seen = l.seen;
+        for (uint32_t k = 1; seen != l.key && seen != SLOSH_NONE && k < P.cap; k++) {
+            slot = (slot + 1u) & (P.cap - 1u);
+            seen = table[slot];
         }
+        in.nbr[(size_t)hid * NBR_STRIDE + lane] = seen == l.key ? slot : SLOSH_NONE;
     }
-    // Workgroup 0 computes the block totals and starts (steady state) and the item starts.
-    if (blockIdx.x == 0) {
-        p2g_block_scan<FAST>(M, blk_start_out, blk_cnt_out, item_start, n_items, S.wsum);
-        return;
+    if (lane == 0u) {
+        in.bin[hid] = range;
+        in.blk_cnt[hid] = br.total;
     }
-    const uint32_t B = M.counters[CTR_NUM_BLOCKS];
+}
+
+template <int P2G_CHUNK, bool FAST>
+__global__ __launch_bounds__(192, P2G_CHUNK <= 384 ? 4 : 1) void k_p2g(StepParams P, const float4 *__restrict__ pos,
+                                             const float4 *__restrict__ vm, const float *__restrict__ C,
+                                             const float *__restrict__ fdt, uint32_t pcap, Members M, SortInputs in,
+                                             const uint32_t *__restrict__ keys, float4 *__restrict__ tiles,
+                                             uint32_t *__restrict__ cell_cnt) {
+    __shared__ P2GShared<P2G_CHUNK> S;
     const uint32_t n_ovf = M.counters[CTR_OVERFLOW];
     const uint32_t kz = threadIdx.x >> 6, lane = threadIdx.x & 63u;
     const int lx = lane & 3, ly = (lane >> 2) & 3, lz = lane >> 4;
-
+    uint32_t B, upto = 0u;  // blocks; FAST: those of the regions up to the lane's
+    if constexpr (FAST) {
+        upto = wave_inclusive_scan(in.rcnt[lane * RCNT_STRIDE]);
+        B = __builtin_amdgcn_readlane(upto, 63);
+        if (blockIdx.x == 0u && threadIdx.x == 0u) *in.num_blocks = B;
+    } else {
+        B = M.counters[CTR_NUM_BLOCKS];
+    }
     if (threadIdx.x < 64) S.lcnt[threadIdx.x] = 0u;
-    for (uint32_t k = blockIdx.x - 1u; k < B; k += gridDim.x - 1u) {
-        const uint32_t hid = M.blist[k];
-        const BlockRange br = block_range<FAST>(M, hid);
+    for (uint32_t j = blockIdx.x >> 3;; j += gridDim.x >> 3) {
+        const uint32_t k = xcd_item(blockIdx.x & 7u, j, B);
+        if (k >= B) break;
+        uint32_t hid, block_key;
+        BlockRange br;
+        uint4 range;
+        Lookup look;
+        if constexpr (FAST) {
+            const uint32_t r = (uint32_t)__popcll(__ballot(upto <= k));
+            const uint32_t before = r ? __builtin_amdgcn_readlane(upto, r - 1u) : 0u;
+            const uint2 e = in.rlist[(r << in.rshift) + (k - before)];
+            hid = __builtin_amdgcn_readfirstlane(e.x);
+            block_key = __builtin_amdgcn_readfirstlane(e.y);
+            const uint4 a = in.arrive[hid];
+            range = make_uint4(0u, 0u, 0u, a.x);
+            if (a.y != SLOSH_NONE) range = make_uint4(a.z, a.w, in.prev_stay[a.y], a.x);
+            br = steady_range(M, hid, range);
+            // The neighbours' first probes, resolved after the sums (below).
+            if (kz == 0u) find_neighbours(P, keys, in.prev_keys, block_key, lane, look);
+            if (threadIdx.x == 0u) in.blist[k] = hid;
+        } else {
+            hid = M.blist[k];
+            block_key = keys[hid];
+            br = block_range<false>(M, hid);
+        }
         // A block without particles (a "+1" neighbour only) has an all-zero tile:
-        // nothing is written and the grid update skips it.
-        if (br.total == 0) {
-            if (threadIdx.x < 64) cell_cnt[(size_t)hid * NODES_PER_BLOCK + threadIdx.x] = 0u;
+        // nothing is written and the grid update skips it. (The stayers are waited for
+        // only below: a block that all its particles left writes a zero tile.)
+        const uint32_t n_main = br.cand_n + br.list_n;
+        if (n_main == 0u) {
+            if (kz == 0u) {
+                cell_cnt[(size_t)hid * NODES_PER_BLOCK + lane] = 0u;
+                if constexpr (FAST) finish_block(P, in, keys, hid, lane, range, br, look);
+            }
             continue;
         }
-        const uint32_t block_key = keys[hid];
         float acc[9][4];
 #pragma unroll
         for (int q = 0; q < 9; q++) acc[q][0] = acc[q][1] = acc[q][2] = acc[q][3] = 0.0f;
         uint32_t tot = 0u;
-        const uint32_t n_main = br.cand_n + br.list_n;
         for (uint32_t chunk = 0; chunk < n_main; chunk += P2G_CHUNK) {
             const uint32_t kn = n_main - chunk < (uint32_t)P2G_CHUNK ? n_main - chunk : (uint32_t)P2G_CHUNK;
             p2g_chunk<P2G_CHUNK>(P, S, kn, [&](uint32_t t) { return entry_slot(br, chunk + t); }, pos, vm, C, fdt,
@@ -1674,6 +1666,10 @@ __global__ __launch_bounds__(192, P2G_CHUNK <= 384 ? 4 : 1) void k_p2g(StepParam
                                          block_key, acc, tot);
             }
         }
+        // The block's place in its region's storage and items (stored below).
+        unsigned long long rel = 0ull;
+        if (threadIdx.x == 0u)
+            rel = atomicAdd(&in.rsum[(hid >> in.rshift) * RSUM_STRIDE], ((unsigned long long)br.total << 32) | item_count(br));
         // Each wave adds its registers into its own slab tile (sharing the staging's
         // LDS), in 9 rounds in which its 64 lanes touch 64 distinct nodes; then each
         // node is the sum of the slabs that cover it, in wave order.
@@ -1713,6 +1709,9 @@ __global__ __launch_bounds__(192, P2G_CHUNK <= 384 ? 4 : 1) void k_p2g(StepParam
             tiles[(size_t)hid * TILE_NODES + tile_index(x, y, z)] = t;
         }
         if (kz == 0) cell_cnt[(size_t)hid * NODES_PER_BLOCK + lane] = tot;
+        if (threadIdx.x == 0u) in.rel[hid] = make_uint2((uint32_t)(rel >> 32), (uint32_t)rel);
+        if constexpr (FAST)
+            if (kz == 0u) finish_block(P, in, keys, hid, lane, range, br, look);
     }
 }
 
@@ -1781,30 +1780,43 @@ __device__ inline void mesh_queries(const Colliders &cs, const float4 *box, Mesh
     }
 }
 
-// The work list of the fused G2P kernel: an item is 64 consecutive entries of a
-// block's sequence (header id, index of the 64).
+// What the grid update prepares for the fused G2P kernel: each block's storage start
+// and its items (64 consecutive entries of its sequence: header id, index of the 64),
+// from the regions' sums and the block's place in them, and cleared counters (output
+// slots taken, stayers).
 struct ItemLists {
     uint2 *items;
-    const uint32_t *item_start;  // per block: its first item
-    uint32_t *taken, *stay;      // per block, counted by G2P: output slots taken, stayers
-    uint32_t fast;
+    const unsigned long long *rsum;
+    const uint2 *rel;
+    uint32_t *blk_start, *taken, *stay, *n_items;
+    uint32_t rshift;
 };
 
-// Writes a block's items and clears its counters; the lanes of one wave.
-__device__ inline void write_items(const Members &M, const ItemLists &L, uint32_t hid, uint32_t lane) {
-    uint32_t entries, total;
-    if (L.fast) {
-        const BlockRange br = block_range<true>(M, hid);
-        entries = br.cand_n + br.list_n;
-        total = br.total;
-    } else {
-        entries = total = M.blk_cnt[hid];
+// The next substep's table, reset here (`prime`).
+struct NextTable {
+    uint32_t *keys, *counters, *mlist, *ovf_slot, *ovf_hid;
+    uint4 *arrive;  // per block: movers; slot, start and count of its stayers' range (else SLOSH_NONE)
+    uint2 *rlist;
+    uint32_t *rcnt;
+    unsigned long long *rsum;
+    uint32_t rshift, prime;
+};
+
+__device__ inline void reset_next_table(const NextTable &nt, uint32_t cap) {
+    if (!nt.prime) return;
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    for (uint32_t s = i; s < cap; s += gridDim.x * blockDim.x) {
+        nt.keys[s] = SLOSH_NONE;
+        nt.arrive[s] = make_uint4(0u, SLOSH_NONE, 0u, 0u);
     }
-    const uint32_t n = total ? (entries + 63u) >> 6 : 0u;
-    for (uint32_t c = lane; c < n; c += 64u) L.items[L.item_start[hid] + c] = make_uint2(hid, c);
-    if (lane == 0) {
-        L.taken[hid] = 0u;
-        L.stay[hid] = 0u;
+    if (blockIdx.x == 0u && threadIdx.x < REGIONS) {
+        nt.rcnt[threadIdx.x * RCNT_STRIDE] = 0u;
+        nt.rsum[threadIdx.x * RSUM_STRIDE] = 0ull;
+    }
+    if (i == 0u) {
+        nt.counters[CTR_NUM_BLOCKS] = 0u;
+        nt.counters[CTR_SORTED_ALLOC] = 0u;
+        nt.counters[CTR_OVERFLOW] = 0u;
     }
 }
 
@@ -1813,29 +1825,51 @@ __device__ inline void write_items(const Members &M, const ItemLists &L, uint32_
 template <bool MESH>
 __global__ __launch_bounds__(MESH ? 64 * MESH_WAVES : 256) void k_grid_update(StepParams P, const float4 *__restrict__ tiles,
                                                      float4 *__restrict__ nodes, const uint32_t *__restrict__ nbr,
-                                                     const uint32_t *__restrict__ blist,
                                                      const uint32_t *__restrict__ keys, Colliders cs,
                                                      const NodeColl *__restrict__ coll_prev, NodeColl *__restrict__ coll_cur,
-                                                     const uint32_t *__restrict__ counters,
-                                                     Members M, ItemLists L, uint32_t mode,
+                                                     Members M, ItemLists L, NextTable nt, uint32_t mode,
                                                      uint32_t do_update) {
     const uint32_t *__restrict__ blk_cnt = M.blk_cnt;
+    reset_next_table(nt, P.cap);
     __shared__ float4 cbox[2 * SLOSH_MAX_COLLIDERS];
     if (threadIdx.x < cs.count) collider_box<MESH>(cs, threadIdx.x, 1.5f * P.h, &cbox[2 * threadIdx.x], &cbox[2 * threadIdx.x + 1]);
     __syncthreads();
-    const uint32_t B = counters[CTR_NUM_BLOCKS];
+    const uint32_t B = M.counters[CTR_NUM_BLOCKS];
     const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63u;
     const int x = lane & 3, y = (lane >> 2) & 3, z = lane >> 4;
+    // Storage and items before the lane's region.
+    const unsigned long long rs = L.rsum[lane * RSUM_STRIDE];
+    const uint32_t up_p = wave_inclusive_scan((uint32_t)(rs >> 32)), up_i = wave_inclusive_scan((uint32_t)rs);
+    if (blockIdx.x == 0u && threadIdx.x == 0u) *L.n_items = __builtin_amdgcn_readlane(up_i, 63);
     // With trimesh colliders a workgroup shares one block: every wave holds its nodes
     // (and takes part in mesh_queries), the first one writes them.
     __shared__ typename std::conditional<MESH, MeshShared, char>::type shared;
-    const uint32_t first = MESH ? blockIdx.x : blockIdx.x * 4 + wave, step = MESH ? gridDim.x : gridDim.x * 4;
+    const uint32_t xcd = blockIdx.x & 7u, wg = blockIdx.x >> 3, wgs = gridDim.x >> 3;
     const bool owner = !MESH || wave == 0u;
-    for (uint32_t k = first; k < B; k += step) {
-        const uint32_t hid = blist[k];
+    for (uint32_t j = MESH ? wg : wg * 4u + wave;; j += MESH ? wgs : wgs * 4u) {
+        const uint32_t k = xcd_item(xcd, j, B);
+        if (k >= B) break;
+        const uint32_t hid = __builtin_amdgcn_readfirstlane(M.blist[k]);
+        const uint32_t block_key = __builtin_amdgcn_readfirstlane(keys[hid]);
+        // The neighbour table (lane l: entry l, see NBR_STRIDE).
+        const uint32_t nb = lane < NBR_STRIDE ? nbr[(size_t)hid * NBR_STRIDE + lane] : SLOSH_NONE;
+        const uint32_t prev = __builtin_amdgcn_readlane(nb, NBR_PREV);
+        if (mode == 0 && owner) {
+            const BlockRange br = M.fast ? block_range<true>(M, hid) : block_range<false>(M, hid);
+            const uint32_t n = item_count(br), r = hid >> L.rshift;
+            if (n) {
+                const uint2 rel = L.rel[hid];
+                const uint32_t item0 = rel.y + (r ? __builtin_amdgcn_readlane(up_i, r - 1u) : 0u);
+                for (uint32_t c = lane; c < n; c += 64u) L.items[item0 + c] = make_uint2(hid, c);
+                if (M.fast && lane == 0u) L.blk_start[hid] = rel.x + (r ? __builtin_amdgcn_readlane(up_p, r - 1u) : 0u);
+            }
+            if (lane == 0u) {
+                L.taken[hid] = 0u;
+                L.stay[hid] = 0u;
+            }
+        }
         float4 acc;
         if (mode == 0) {
-            if (owner) write_items(M, L, hid, lane);
             // Tiles of blocks without particles were not written (they count as
             // zero). Each tile value is loaded together with its block's particle
             // count and then selected by it, so the tile loads wait only for the
@@ -1851,8 +1885,8 @@ __global__ __launch_bounds__(MESH ? 64 * MESH_WAVES : 256) void k_grid_update(St
                 const int ox = ASSOC[d][0], oy = ASSOC[d][1], oz = ASSOC[d][2];
                 t[d] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
                 c[d] = 0u;
+                const uint32_t src = __builtin_amdgcn_readlane(nb, NBR_MINUS + d - 1);
                 if ((ox == 0 || x <= 1) && (oy == 0 || y <= 1) && (oz == 0 || z <= 1)) {
-                    const uint32_t src = nbr[(size_t)hid * NBR_STRIDE + NBR_MINUS + d - 1];
                     if (src != SLOSH_NONE) {
                         t[d] = tiles[(size_t)src * TILE_NODES + tile_index(x + 4 * ox, y + 4 * oy, z + 4 * oz)];
                         c[d] = blk_cnt[src];
@@ -1885,10 +1919,10 @@ __global__ __launch_bounds__(MESH ? 64 * MESH_WAVES : 256) void k_grid_update(St
             if (owner) nodes[(size_t)hid * NODES_PER_BLOCK + lane] = acc;
             continue;
         }
+        const float h = P.h, dt = P.dt;
         int bx, by, bz;
         uint32_t scene;
-        unpack_key(P.batched, keys[hid], &bx, &by, &bz, &scene);
-        const float h = P.h, dt = P.dt;
+        unpack_key(P.batched, block_key, &bx, &by, &bz, &scene);
         float3 cell_pos = make_float3((float)(bx * 4 + x) * h, (float)(by * 4 + y) * h, (float)(bz * 4 + z) * h);
         // update_single_cell, grid_update.slang:154-163
         const float mass = acc.w;
@@ -1898,7 +1932,6 @@ __global__ __launch_bounds__(MESH ? 64 * MESH_WAVES : 256) void k_grid_update(St
         v.x = fminf(fmaxf((acc.x + mass * P.gravity[0] * dt) * inv_mass, -lim), lim);
         v.y = fminf(fmaxf((acc.y + mass * P.gravity[1] * dt) * inv_mass, -lim), lim);
         v.z = fminf(fmaxf((acc.z + mass * P.gravity[2] * dt) * inv_mass, -lim), lim);
-        const uint32_t prev = P.coll_cache ? nbr[(size_t)hid * NBR_STRIDE + NBR_PREV] : SLOSH_NONE;
         const unsigned long long(*mesh_keys)[NODES_PER_BLOCK] = nullptr;
         if constexpr (MESH) {
             mesh_queries(cs, cbox, shared, h, cell_pos,
@@ -2040,19 +2073,16 @@ __device__ inline void load_halo_wave(float4 *__restrict__ sh, const float4 *__r
     }
 }
 
-// What the fused G2P kernel prepares for the next substep: its table (keys
-// inserted, a new block's mover count cleared), the list of particles that
-// leave their block, and every block's stayer count.
+// What the fused G2P kernel counts per block of this table: output slots handed out
+// and particles that stay. For the next substep it inserts the blocks into NextTable
+// and appends the particles that leave their block to their new block's list.
 struct NextSort {
-    uint32_t *mcount;         // next table: movers per block (cleared at insertion)
-    uint32_t *mv_key, *mv_slot;  // movers: new block key, output slot
-    uint32_t *taken;          // this table: output slots each block has handed out
-    uint32_t *stay;           // this table: particles of each block that stay in it
+    uint32_t *taken, *stay;
     uint32_t *errors;         // this substep's error word (ERR_KEY_RANGE)
 };
 
-// F64: the SVD-based steps refined to FP64 accuracy. The bound keeps that
-// variant at three waves per SIMD (168 VGPRs).
+// F64: the SVD-based steps refined to FP64 accuracy. The bounds keep that variant of
+// every material at three waves per SIMD (168 VGPRs), the others at four or more.
 //
 // One wave per item: 64 consecutive entries of a block's sequence, with the
 // block's node halo in an LDS tile of the wave's own, so that waves share no
@@ -2060,52 +2090,73 @@ struct NextSort {
 // workgroup. With one workgroup per block a second round of 256 entries cost a
 // block 3.8 us of serial latency, and a block of 50 particles kept four waves;
 // per wave (medians of the kernel, before and after): 2.1M sand and spheres (42k
-// blocks) 643 -> 282 us, 48 scenes of three materials (2.0M) 320 -> 172 us, sand on
-// a heightfield (85k) 43 -> 21 us, dam break of 131k 15.7 -> 13.6 us and of 1M
-// 52 us both at its start, 66 -> 52 us once it moves. The small scenes are bound by
+// blocks) 643 -> 280 us, 48 scenes of three materials (2.0M) 320 -> 168 us, sand on
+// a heightfield (85k) 43 -> 19 us, dam break of 131k 15.7 -> 13.1 us and of 1M
+// 66 -> 46 us once it moves. The small scenes are bound by
 // the chain of dependent loads and the ~1000 instructions of one particle, the
 // large ones by memory (188 MB per launch at 1M) and issue.
 //
 // Output order: a block's members take the output slots [start, start + total)
 // of the block in order of arrival of their waves (one atomic per wave, issued
 // before the sums that hide it), so a block's particles stay together in
-// storage. The particles whose updated position leaves the block are listed,
-// with their new block key, for the next substep's sort; the others are counted
-// (the block's stayers).
+// storage. The particles whose updated position leaves the block join their new
+// block's list in the next substep's table; the others are counted (the block's
+// stayers).
+// The arguments, read where they are used: held in scalar registers from the start
+// 118 of them spilled to VGPR lanes. late_args() gives the compiler a new, opaque address
+// of the kernel's argument block, so that what is read through it is loaded after that
+// point: the neo-Hookean instance needs 93 instead of 108 VGPRs (five waves per SIMD
+// instead of four; 1M particles 53.0 -> 48.6 us), the FP32 one of every material 128
+// instead of 145 (four instead of three).
+struct G2pArgs {
+    StepParams P;
+    PBuf in, out;
+    PStatic st;
+    uint32_t pcap;
+    float *fdt;
+    NextTable nt;
+    NextSort ns;
+    Bodies bodies;
+};
+
+template <typename T>
+__device__ inline const T &late_args() {
+    auto p = (const __attribute__((address_space(4))) char *)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(p));
+    return *(const T *)p;
+}
+
 template <uint32_t MODELS, bool F64>
-__global__ __launch_bounds__(256, F64 ? (MODELS == 3u ? 4 : 3) : 1) void k_g2p_update(StepParams P, PBuf in, PBuf out, PStatic st, uint32_t pcap_arg,
-                                                    float *__restrict__ fdt, Members M,
+__global__ __launch_bounds__(256, F64 && MODELS != 3u ? 3 : 4) void k_g2p_update(G2pArgs args, Members M,
                                                     const uint2 *__restrict__ items,
                                                     const uint32_t *__restrict__ blk_start,
                                                     const float4 *__restrict__ nodes,
-                                                    const uint32_t *__restrict__ keys, NextTable nt, NextSort ns,
-                                                    Bodies bodies) {
+                                                    const uint32_t *__restrict__ keys) {
     extern __shared__ float4 halo[];  // TILE_NODES per wave
     // integrate_bodies: reads no particle or grid state (the impulses it applies
     // are only written by the host), so the last workgroup runs it alongside the
     // particle update.
-    if (blockIdx.x == gridDim.x - 1u) {
-        if (threadIdx.x < bodies.count) integrate_body(P, bodies, threadIdx.x);
+    if (blockIdx.x == gridDim.x - 1u) {  // (the eighth range's last workgroup takes no items)
+        if (threadIdx.x < args.bodies.count) integrate_body(args.P, args.bodies, threadIdx.x);
         return;
     }
     const uint32_t n_items = M.counters[CTR_ITEMS];
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), waves = blockDim.x >> 6;
     float4 *sh = halo + wave * TILE_NODES;
-    for (uint32_t i = blockIdx.x * waves + wave; i < n_items; i += (gridDim.x - 1u) * waves) {
-        // Opaque copies: most waves take one item, so nothing is worth computing
+    for (uint32_t j = (blockIdx.x >> 3) * waves + wave;; j += (gridDim.x >> 3) * waves) {
+        const uint32_t i = xcd_item(blockIdx.x & 7u, j, n_items);
+        if (i >= n_items) break;
+        // An opaque copy: most waves take one item, so nothing is worth computing
         // ahead of the loop and holding in (spilled) registers.
-        uint32_t lane = threadIdx.x & 63u, pcap = pcap_arg;
-        asm volatile("" : "+v"(lane), "+s"(pcap));
-        BlockInit init;
-        init.mcount = ns.mcount;
-        init.blk_cnt = nullptr;
-        init.cell_cnt = nullptr;
+        uint32_t lane = threadIdx.x & 63u;
+        asm volatile("" : "+v"(lane));
         const uint2 item = items[i];
         const uint32_t hid = __builtin_amdgcn_readfirstlane(item.x);
         const uint32_t first = __builtin_amdgcn_readfirstlane(item.y) * 64u;
         const BlockRange br = M.fast ? block_range<true>(M, hid) : block_range<false>(M, hid);
-        const uint32_t s0 = blk_start[hid];
-        const uint32_t block_key = keys[hid];
+        const uint32_t s0 = __builtin_amdgcn_readfirstlane(blk_start[hid]);
+        const uint32_t block_key = __builtin_amdgcn_readfirstlane(keys[hid]);
+        const uint32_t total = __builtin_amdgcn_readfirstlane(br.total);
         // The item's entries (a candidate is a member only if it is still in the
         // block); the block's first item then takes the overflow list, only if some
         // of the block's movers overflowed theirs (entries of other blocks are
@@ -2116,6 +2167,7 @@ __global__ __launch_bounds__(256, F64 ? (MODELS == 3u ? 4 : 3) : 1) void k_g2p_u
         const uint32_t n_main = br.cand_n + br.list_n;
         const uint32_t n_ovf = first == 0u && br.overflow ? M.counters[CTR_OVERFLOW] : 0u;
         for (uint32_t o = 0; o < 64u + n_ovf; o += 64u) {
+            const G2pArgs &A = late_args<G2pArgs>();
             bool entry;
             uint32_t p = 0u;
             if (o == 0u) {
@@ -2135,34 +2187,41 @@ __global__ __launch_bounds__(256, F64 ? (MODELS == 3u ? 4 : 3) : 1) void k_g2p_u
             float F[9];
             uint32_t oid = 0u;
             if (entry) {
-                ps = in.pos[p];
+                ps = A.in.pos[p];
                 if (EARLY) {
 #pragma unroll
-                    for (int q = 0; q < 9; q++) F[q] = in.F[(size_t)q * pcap + p];
-                    oid = in.ids[p];
+                    for (int q = 0; q < 9; q++) F[q] = A.in.F[(size_t)q * A.pcap + p];
+                    oid = A.in.ids[p];
                 }
             }
             load_halo_wave(sh, nodes, M.nbr, hid, lane);  // (the last iteration may have reused the tile)
             const uint32_t wbits = __float_as_uint(ps.w);
             const uint32_t scene = wbits >> 1;
-            const Stencil at = stencil_of(P.h, ps.x, ps.y, ps.z);
+            const Stencil at = stencil_of(A.P.h, ps.x, ps.y, ps.z);
             int blk[3];
             uint32_t lc[3];
             block_of_cell(at.cell, blk, lc);
-            const bool valid = entry && pack_key(P.batched, scene, blk[0], blk[1], blk[2]) == block_key;
+            const bool valid = entry && pack_key(A.P.batched, scene, blk[0], blk[1], blk[2]) == block_key;
             const uint64_t vmask = __ballot(valid);
             if (vmask == 0ull) continue;
             uint32_t ob = 0u;
-            if (lane == 0) ob = atomicAdd(&ns.taken[hid], (uint32_t)__popcll(vmask));
+            if (lane == 0) ob = atomicAdd(&A.ns.taken[hid], (uint32_t)__popcll(vmask));
             const float3 pos = make_float3(ps.x, ps.y, ps.z);
             float3 v;
             float aff[9], vgd;
-            if (valid) g2p_particle(sh, P.h, P.inv_d, at, lc, (wbits & 1u) != 0u, &v, aff, &vgd);
+            if (valid) g2p_particle(sh, A.P.h, A.P.inv_d, at, lc, (wbits & 1u) != 0u, &v, aff, &vgd);
             // The wave's first slot, from lane 0 (every lane is active here).
-            const uint32_t slot = s0 + __builtin_amdgcn_readfirstlane(ob) + (uint32_t)__popcll(vmask & lanemask_lt());
+            const uint32_t out0 = __builtin_amdgcn_readfirstlane(ob);
+            const uint32_t slot = s0 + out0 + (uint32_t)__popcll(vmask & lanemask_lt());
             uint32_t next_key = 0u;
             bool in_range = true;
             if (valid) {
+                const G2pArgs &U = late_args<G2pArgs>();
+                const StepParams &P = U.P;
+                const PBuf &in = U.in, &out = U.out;
+                const PStatic &st = U.st;
+                const uint32_t pcap = U.pcap;
+                float *const fdt = U.fdt;
                 // Uniform masses (one for all, or one per scene) skip the 16-byte
                 // velocity / mass load (the velocity comes from the grid): only the
                 // update disables, and it zeroes the mass.
@@ -2234,38 +2293,75 @@ __global__ __launch_bounds__(256, F64 ? (MODELS == 3u ? 4 : 3) : 1) void k_g2p_u
                     next_key = block_key;
                 }
             }
+            const G2pArgs &N = late_args<G2pArgs>();
+            const NextTable &nt = N.nt;
             const bool mover = valid && next_key != block_key;
             const uint64_t sm = __ballot(valid && !mover);
             uint32_t before = 1u;
-            if (sm && lane == 0) before = atomicAdd(&ns.stay[hid], (uint32_t)__popcll(sm));
+            if (sm && lane == 0) before = atomicAdd(&N.ns.stay[hid], (uint32_t)__popcll(sm));
             const uint64_t mv = __ballot(mover);
             if (mv) {
                 // Only a particle that leaves its block can leave the key space (a
                 // block outside it would alias another one): reported, once per wave.
                 const uint64_t bad = __ballot(mover && !in_range);
-                if (bad && lane == 0) atomicOr(ns.errors, ERR_KEY_RANGE);
-                if (nt.prime) {
-                    // The movers, listed for the next substep's sort.
-                    uint32_t lb = 0u;
-                    if (lane == 0) lb = atomicAdd(&nt.counters[CTR_MOVERS], (uint32_t)__popcll(mv));
-                    lb = __shfl(lb, 0);
-                    if (mover) {
-                        const uint32_t e = lb + (uint32_t)__popcll(mv & lanemask_lt());
-                        ns.mv_key[e] = next_key;
-                        ns.mv_slot[e] = slot;
-                    }
-                }
+                if (bad && lane == 0) atomicOr(N.ns.errors, ERR_KEY_RANGE);
             }
             if (nt.prime) {
                 // touch_primary_blocks and touch_neighbor_blocks of the next
                 // substep (sort.slang:50-92). Particles that stay in this block
-                // only flag it (its 8 blocks are inserted once below); the others
-                // insert theirs, one round per run of equal keys.
-                const uint64_t heads = run_heads(next_key, mover) & mv;
-                insert_blocks(nt.keys, P.cap, P.batched, next_key, heads, nt.counters, init);
-                // The first wave with stayers inserts the block itself and its +1 neighbours.
-                if (__builtin_amdgcn_readfirstlane(before) == 0u)
-                    insert_blocks(nt.keys, P.cap, P.batched, block_key, 1ull, nt.counters, init);
+                // only flag it: its 8 blocks are inserted once, by the block's first
+                // wave to arrive if it has stayers, else by the first wave that has (the
+                // first one need not wait for the stayers' count). The others insert
+                // theirs, one round per run of equal keys, and join their new block's
+                // list, one atomic per run. Atomics on what every XCD writes take ~1 us
+                // each: the chain is the insertion, then the list places, at once.
+                BlockInit init{};
+                init.list = nt.rlist;
+                init.rcnt = nt.rcnt;
+                init.rshift = nt.rshift;
+                ListEntry entry;
+                const uint64_t rheads = run_heads(next_key, mover);
+                const bool opener = out0 == 0u && sm;
+                const uint64_t self = opener ? sm & (0ull - sm) : 0ull;
+                const uint64_t heads = (rheads & mv) | self;
+                uint32_t own = SLOSH_NONE;
+                if (heads) {
+                    own = insert_blocks(nt.keys, N.P.cap, N.P.batched, next_key, heads, nt.counters, init, entry);
+                    const int head = run_head_of(rheads);
+                    const uint32_t to = __shfl(own, head);
+                    const bool listed = mover && to != SLOSH_NONE;
+                    uint32_t r0 = 0u;
+                    if (listed && (int)lane == head) r0 = atomicAdd(&nt.arrive[to].x, run_length(rheads));
+                    store_entry(init, entry);
+                    const uint32_t r = __shfl(r0, head) + (lane - (uint32_t)head);
+                    const bool over = listed && r >= MOVER_CAP;
+                    if (listed && !over) nt.mlist[(size_t)to * MOVER_CAP + r] = slot;
+                    const uint64_t om = __ballot(over);
+                    if (om) {
+                        uint32_t q0 = 0u;
+                        if (lane == 0u) q0 = atomicAdd(&nt.counters[CTR_OVERFLOW], (uint32_t)__popcll(om));
+                        q0 = __builtin_amdgcn_readfirstlane(q0);
+                        if (over) {
+                            const uint32_t q = q0 + (uint32_t)__popcll(om & lanemask_lt());
+                            nt.ovf_slot[q] = slot;
+                            nt.ovf_hid[q] = to;
+                        }
+                    }
+                }
+                bool mine = (self >> lane) & 1ull;
+                if (!opener && __builtin_amdgcn_readfirstlane(before) == 0u) {
+                    own = insert_blocks(nt.keys, N.P.cap, N.P.batched, block_key, 1ull, nt.counters, init, entry);
+                    store_entry(init, entry);
+                    mine = lane == 0u;
+                }
+                // Where the block's range is found again: by whoever inserted it, with
+                // the same values.
+                if (mine && own != SLOSH_NONE) {
+                    uint32_t *a = &nt.arrive[own].x;
+                    a[1] = hid;
+                    a[2] = s0;
+                    a[3] = total;
+                }
             }
         }
     }
@@ -2469,18 +2565,59 @@ static inline PBuf to_pbuf(const ParticleBuffers &b) {
     return p;
 }
 
-// Workgroups of a per-block kernel: one block (per_wg blocks) per workgroup up to
-// the tuned persistent width; workgroups loop over the device-side block count.
+// Workgroups of a per-block kernel (a multiple of the XCDs): one block (per_wg
+// blocks) per workgroup up to the tuned persistent width; workgroups loop over the
+// device-side block count. The count is not known here: dense scenes have a block per
+// 300 to 500 particles, so one per 256 leaves few workgroups without a block (an idle
+// one costs 0.2 ns of dispatch: 16384 of them 2.8 us), and 2048 fill the chip when
+// particles are sparse.
 static uint32_t block_grid(const StepParams &P, uint32_t per_wg) {
-    return min_t(div_up_t(P.cap, per_wg), P.block_wgs ? P.block_wgs : 8192u);
+    const uint32_t likely = P.n / 256u > 2048u ? P.n / 256u : 2048u;
+    const uint32_t wgs = div_up_t(P.cap < likely ? P.cap : likely, per_wg);
+    return (min_t(wgs, P.block_wgs ? P.block_wgs : 8192u) + 7u) & ~7u;
 }
 
-// Workgroups of `waves` items each: every entry sequence is at most its block's
-// candidates and listed movers (together at most 2 n entries), in 64s.
+// Workgroups of `waves` items each (a multiple of the XCDs): every entry sequence is at
+// most its block's candidates and listed movers (together at most 2 n entries), in
+// 64s; dense scenes have an item per 55 particles.
 static uint32_t item_grid(const StepParams &P, uint32_t waves) {
-    const uint64_t items = max_items(P.n, P.cap);
-    const uint32_t wgs = div_up_t(items, waves);
-    return wgs == 0u ? 1u : min_t(wgs, P.block_wgs ? P.block_wgs : 8192u);
+    const uint64_t likely = P.n / 48u > 4096u ? P.n / 48u : 4096u, most = max_items(P.n, P.cap);
+    const uint32_t wgs = div_up_t(likely < most ? likely : most, waves);
+    return (min_t(wgs, P.block_wgs ? P.block_wgs : 8192u) + 7u) & ~7u;
+}
+
+static SortInputs sort_inputs(const TransferBuffers &t) {
+    SortInputs in;
+    in.rlist = t.rlist;
+    in.rcnt = t.rcnt;
+    in.prev_keys = t.prev_keys;
+    in.arrive = t.arrive;
+    in.prev_stay = t.prev_stay;
+    in.blist = t.blist_out;
+    in.num_blocks = t.num_blocks;
+    in.nbr = t.nbr_out;
+    in.blk_cnt = t.blk_cnt;
+    in.bin = t.bin;
+    in.rsum = t.rsum;
+    in.rel = t.rel;
+    in.rshift = t.rshift;
+    return in;
+}
+
+static NextTable next_table(const NextTableBuffers &next) {
+    NextTable nt;
+    nt.keys = next.keys;
+    nt.counters = next.counters;
+    nt.arrive = next.arrive;
+    nt.mlist = next.mlist;
+    nt.ovf_slot = next.ovf_slot;
+    nt.ovf_hid = next.ovf_hid;
+    nt.rlist = next.rlist;
+    nt.rcnt = next.rcnt;
+    nt.rsum = next.rsum;
+    nt.rshift = next.rshift;
+    nt.prime = next.prime;
+    return nt;
 }
 
 static Members members_of(const TransferBuffers &t) {
@@ -2489,7 +2626,6 @@ static Members members_of(const TransferBuffers &t) {
     M.blist = t.blist;
     M.nbr = t.nbr;
     M.bin = t.bin;
-    M.mcount = t.mcount;
     M.mlist = t.mlist;
     M.ovf_slot = t.ovf_slot;
     M.ovf_hid = t.ovf_hid;
@@ -2501,11 +2637,7 @@ static Members members_of(const TransferBuffers &t) {
 }
 
 hipError_t launch_p2g(const StepParams &P, const ParticleBuffers &pb, uint32_t pcap, const TransferBuffers &t,
-                      const NextTableBuffers &next, const PassEvents *ev, hipStream_t stream) {
-    NextTable nt;
-    nt.keys = next.keys;
-    nt.counters = next.counters;
-    nt.prime = next.prime;
+                      const PassEvents *ev, hipStream_t stream) {
     auto kern = t.fast ? (P.p2g_chunk == 192u   ? k_p2g<192, true>
                           : P.p2g_chunk == 256u ? k_p2g<256, true>
                           : P.p2g_chunk == 384u ? k_p2g<384, true>
@@ -2514,15 +2646,15 @@ hipError_t launch_p2g(const StepParams &P, const ParticleBuffers &pb, uint32_t p
                           : P.p2g_chunk == 256u ? k_p2g<256, false>
                           : P.p2g_chunk == 384u ? k_p2g<384, false>
                                                 : k_p2g<512, false>);
-    // One more workgroup (the first) computes the block and item starts.
-    launch_kernel(ev, kern, dim3(block_grid(P, 1) + 1u), dim3(192), 0, stream, P, nt,
-                  (const float4 *)pb.pos, (const float4 *)pb.vm, (const float *)pb.C, (const float *)t.fdt, pcap,
-                  members_of(t), t.keys, t.tiles, t.cell_cnt, t.blk_start, t.blk_cnt, t.item_start, t.n_items);
+    launch_kernel(ev, kern, dim3(block_grid(P, 1)), dim3(192), 0, stream, P, (const float4 *)pb.pos,
+                  (const float4 *)pb.vm, (const float *)pb.C, (const float *)t.fdt, pcap, members_of(t), sort_inputs(t),
+                  t.keys, t.tiles, t.cell_cnt);
     return hipGetLastError();
 }
 
-hipError_t launch_grid_update(const StepParams &P, const TransferBuffers &t, const ColliderBuffers &c, uint32_t mode,
-                              uint32_t do_update, const PassEvents *ev, hipStream_t stream) {
+hipError_t launch_grid_update(const StepParams &P, const TransferBuffers &t, const ColliderBuffers &c,
+                              const NextTableBuffers &next, uint32_t mode, uint32_t do_update, const PassEvents *ev,
+                              hipStream_t stream) {
     Colliders cs;
     cs.shapes = c.shapes;
     cs.poses = c.poses;
@@ -2535,16 +2667,19 @@ hipError_t launch_grid_update(const StepParams &P, const TransferBuffers &t, con
     cs.mesh_base = c.mesh_base;
     ItemLists items;
     items.items = t.items;
-    items.item_start = t.item_start;
+    items.rsum = t.rsum;
+    items.rel = t.rel;
+    items.blk_start = t.blk_start;
     items.taken = t.taken;
     items.stay = t.stay;
-    items.fast = t.fast;
+    items.n_items = t.n_items;
+    items.rshift = t.rshift;
     // Trimesh projection (a BVH walk) is compiled into its own instance so that
     // scenes without meshes keep the smaller kernel.
     launch_kernel(ev, c.mesh_vtx ? k_grid_update<true> : k_grid_update<false>, dim3(block_grid(P, c.mesh_vtx ? 1 : 4)),
                   dim3(c.mesh_vtx ? 64 * MESH_WAVES : 256), 0, stream, P,
-                  (const float4 *)t.tiles, t.nodes, t.nbr, t.blist, t.keys, cs, (const NodeColl *)t.coll_prev,
-                  (NodeColl *)t.coll_cur, t.counters, members_of(t), items, mode, do_update);
+                  (const float4 *)t.tiles, t.nodes, t.nbr, t.keys, cs, (const NodeColl *)t.coll_prev,
+                  (NodeColl *)t.coll_cur, members_of(t), items, next_table(next), mode, do_update);
     return hipGetLastError();
 }
 
@@ -2552,30 +2687,27 @@ hipError_t launch_g2p_update(const StepParams &P, const ParticleBuffers &in, con
                              const StaticBuffers &s, uint32_t pcap, const TransferBuffers &t,
                              const NextTableBuffers &next, const BodyBuffers &bb, const PassEvents *ev,
                              hipStream_t stream) {
-    NextTable nt;
-    nt.keys = next.keys;
-    nt.counters = next.counters;
-    nt.prime = next.prime;
-    NextSort ns;
-    ns.mcount = next.mcount;
-    ns.mv_key = next.mv_key;
-    ns.mv_slot = next.mv_slot;
-    ns.taken = t.taken;
-    ns.stay = t.stay;
-    ns.errors = t.errors;
-    Bodies b;
-    b.poses = bb.poses;
-    b.vels = bb.vels;
-    b.mprops = bb.mprops;
-    b.local_com = bb.local_com;
-    b.impulses = bb.impulses;
-    b.count = bb.count;
-    PStatic st;
-    st.prop = s.prop;
-    st.model = s.model;
-    st.dp0 = s.dp0;
-    st.dp1 = s.dp1;
-    st.scene_rec = s.scene_rec;
+    G2pArgs args;
+    args.P = P;
+    args.in = to_pbuf(in);
+    args.out = to_pbuf(out);
+    args.st.prop = s.prop;
+    args.st.model = s.model;
+    args.st.dp0 = s.dp0;
+    args.st.dp1 = s.dp1;
+    args.st.scene_rec = s.scene_rec;
+    args.pcap = pcap;
+    args.fdt = t.fdt;
+    args.nt = next_table(next);
+    args.ns.taken = t.taken;
+    args.ns.stay = t.stay;
+    args.ns.errors = t.errors;
+    args.bodies.poses = bb.poses;
+    args.bodies.vels = bb.vels;
+    args.bodies.mprops = bb.mprops;
+    args.bodies.local_com = bb.local_com;
+    args.bodies.impulses = bb.impulses;
+    args.bodies.count = bb.count;
     // The lightest instance that handles every material present: neo-Hookean
     // only (no SVD code), fixed-corotated and neo-Hookean, every material.
     const bool nh_only = (P.tag_mask & ~2u) == 0u;
@@ -2586,9 +2718,8 @@ hipError_t launch_g2p_update(const StepParams &P, const ParticleBuffers &in, con
     const uint32_t waves = P.g2p_threads == 128u ? 2u : 4u;
     // One more workgroup (the last) integrates the rigid bodies.
     launch_kernel(ev, kern, dim3(item_grid(P, waves) + 1u), dim3(64u * waves),
-                  waves * TILE_NODES * (uint32_t)sizeof(float4), stream, P, to_pbuf(in),
-                  to_pbuf(out), st, pcap, t.fdt, members_of(t), (const uint2 *)t.items, (const uint32_t *)t.blk_start,
-                  (const float4 *)t.nodes, t.keys, nt, ns, b);
+                  waves * TILE_NODES * (uint32_t)sizeof(float4), stream, args, members_of(t), (const uint2 *)t.items,
+                  (const uint32_t *)t.blk_start, (const float4 *)t.nodes, t.keys);
     return hipGetLastError();
 }
 

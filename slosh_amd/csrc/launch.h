@@ -12,18 +12,11 @@ struct GridBuffers {
     uint32_t *blist, *nbr, *cell_cnt, *cell_start, *blk_start, *blk_cnt;
     uint32_t *pslot, *prank, *perm, *counters;
     uint32_t *tile_sums;  // ceil(cap / 4096) words
-    // Movers listed by the previous substep and their per-block lists.
-    const uint32_t *mv_key, *mv_slot;
-    uint32_t *mcount, *mlist, *ovf_slot, *ovf_hid;
-    // Previous table's block ranges and stayer counts, and per block of this
-    // table those of its previous-table block (written by the steady-state sort).
-    const uint32_t *prev_start, *prev_cnt, *prev_stay;
-    uint4 *bin;
+    unsigned long long *rsum;  // REGIONS
 };
 
-// `fast`: the previous substep's fused G2P kernel filled this table, wrote every
-// block's stayers first and listed the movers. `ev` (optional) brackets the
-// whole sequence.
+// `fast`: the previous substep's fused kernels prepared this table. `ev` (optional)
+// brackets the whole sequence.
 hipError_t launch_grid_build(const GridBuffers &g, const float4 *pos, uint32_t n, float h, uint32_t batched,
                              uint32_t cap, bool fast, const PassEvents *ev, hipStream_t stream);
 
@@ -33,10 +26,23 @@ struct TransferBuffers {
     const uint32_t *keys, *blist, *nbr, *counters;
     const uint32_t *perm;                             // full sort
     uint32_t *cell_cnt, *blk_start, *blk_cnt, *stay;  // this table
+    // The steady state: this table's regional block lists, what the previous substep
+    // left for each block (see NextTableBuffers), the previous table's keys and stayers;
+    // written by P2G: the flat list and its length, the neighbour tables, each block's
+    // range (start, count), stayers and movers.
+    const uint2 *rlist;
+    const uint4 *arrive;
+    const uint32_t *rcnt, *prev_keys, *prev_stay;
+    uint32_t rshift;
+    uint32_t *blist_out, *num_blocks, *nbr_out;
+    uint4 *bin;
+    // Per region, the sums of its blocks' particles (high word) and items (low word),
+    // and each block's place in them.
+    unsigned long long *rsum;
+    uint2 *rel;
     uint2 *items;  // the fused G2P kernel's items (max_items of them)
-    uint32_t *item_start, *n_items, *taken;
-    const uint4 *bin;  // per block: range (start, count) and stayers of its previous-table block
-    const uint32_t *mcount, *mlist, *ovf_slot, *ovf_hid;
+    uint32_t *n_items, *taken;
+    const uint32_t *mlist, *ovf_slot, *ovf_hid;
     uint32_t *errors;  // this substep's error word
     float4 *tiles, *nodes;
     void *coll_prev, *coll_cur;
@@ -77,19 +83,26 @@ struct BodyBuffers {
     uint32_t count;
 };
 
-// The next substep's table and sort inputs, prepared by this substep's P2G
-// (reset) and fused G2P (insertion, mover list).
+// The next substep's table and sort inputs, prepared by this substep's grid update
+// (reset) and fused G2P (insertion, block lists, movers).
 struct NextTableBuffers {
     uint32_t *keys, *counters;
-    uint32_t *mcount;            // next table: movers per block
-    uint32_t *mv_key, *mv_slot;  // movers: new block key, output slot
-    uint32_t prime;
+    // Per block: the movers it receives; its slot in the table before and its range there
+    // (start, count), if it has stayers (else SLOSH_NONE).
+    uint4 *arrive;
+    uint32_t *mlist;                // the first MOVER_CAP movers of each block
+    uint32_t *ovf_slot, *ovf_hid;   // the others
+    uint2 *rlist;                   // regional block lists (slot, key)
+    uint32_t *rcnt;
+    unsigned long long *rsum;
+    uint32_t rshift, prime;
 };
 
 hipError_t launch_p2g(const StepParams &P, const ParticleBuffers &pb, uint32_t pcap, const TransferBuffers &t,
-                      const NextTableBuffers &next, const PassEvents *ev, hipStream_t stream);
-hipError_t launch_grid_update(const StepParams &P, const TransferBuffers &t, const ColliderBuffers &c, uint32_t mode,
-                              uint32_t do_update, const PassEvents *ev, hipStream_t stream);
+                      const PassEvents *ev, hipStream_t stream);
+hipError_t launch_grid_update(const StepParams &P, const TransferBuffers &t, const ColliderBuffers &c,
+                              const NextTableBuffers &next, uint32_t mode, uint32_t do_update, const PassEvents *ev,
+                              hipStream_t stream);
 hipError_t launch_g2p_update(const StepParams &P, const ParticleBuffers &in, const ParticleBuffers &out,
                              const StaticBuffers &s, uint32_t pcap, const TransferBuffers &t,
                              const NextTableBuffers &next, const BodyBuffers &bb, const PassEvents *ev,

@@ -15,12 +15,12 @@
 //     model (tag, lambda, mu, cfl of the elastic part), dp0 (h0..h3), dp1 (lambda, mu)
 //   grid: two hash tables (ping-pong = previous substep; a block's header id is
 //     the slot of its key), per block of each table its storage range, stayer
-//     count and mover count, and per block the block list entry, neighbour
-//     table, 64 cell counts/starts, MOVER_CAP mover slots, a 6x6x6 float4 P2G
-//     tile, 64 float4 nodes, two collision caches (moving colliders).
-// The fused G2P/particle-update kernel writes the next buffer block by block
-// (each block's stayers first, its leavers last, listed for the next sort), so
-// storage follows the block order of the previous substep; readback restores
+//     count, what it receives (movers, the range of its stayers), MOVER_CAP mover
+//     slots and its entry of the regional block lists, and per block its entry of the
+//     flat list, neighbour table, 64 cell counts/starts, a 6x6x6 float4 P2G tile,
+//     64 float4 nodes, two collision caches (moving colliders).
+// The fused G2P/particle-update kernel writes the next buffer block by block and
+// prepares the next table (blocks, lists, movers), so storage follows the block order of the previous substep; readback restores
 // the original order through `ids`.
 #include <hip/hip_runtime.h>
 
@@ -183,17 +183,23 @@ struct slosh_data {
     // table, each block's storage range, stayer count and received movers
     uint32_t *keys[2] = {nullptr, nullptr};
     uint32_t *blk_start[2] = {nullptr, nullptr}, *blk_cnt[2] = {nullptr, nullptr};
-    uint32_t *stay[2] = {nullptr, nullptr}, *mcount[2] = {nullptr, nullptr};
+    uint32_t *stay[2] = {nullptr, nullptr};
+    uint4 *arrive[2] = {nullptr, nullptr};
     uint32_t *blist = nullptr, *nbr = nullptr, *cell_cnt = nullptr, *cell_start = nullptr;
-    uint32_t *mlist = nullptr;  // MOVER_CAP movers per block
-    // The fused G2P kernel's items, and per block their start and the output slots taken.
+    uint32_t *mlist[2] = {nullptr, nullptr};  // per table: MOVER_CAP movers per block
+    // Per table: block lists by region (slot, key), and per region their length and the
+    // sums of its blocks' particles and items; per block its place in those sums.
+    uint2 *rlist[2] = {nullptr, nullptr};
+    uint32_t *rcnt[2] = {nullptr, nullptr};
+    unsigned long long *rsum[2] = {nullptr, nullptr};
+    uint2 *rel = nullptr;
+    // The fused G2P kernel's items, and per block the output slots taken.
     uint2 *items = nullptr;
-    uint32_t *item_start = nullptr, *taken = nullptr;
-    uint4 *bin = nullptr;       // per block: its previous-table block's range and stayers
+    uint32_t *taken = nullptr;
+    uint4 *bin = nullptr;       // per block: its previous-table block's range and stayers, its movers
     uint32_t *pslot = nullptr, *prank = nullptr, *perm = nullptr;
-    // per particle: movers listed for the next substep, and movers beyond a
-    // block's list slots
-    uint32_t *mv_key = nullptr, *mv_slot = nullptr, *ovf_slot = nullptr, *ovf_hid = nullptr;
+    // per table and particle: movers beyond a block's list slots
+    uint32_t *ovf_slot[2] = {nullptr, nullptr}, *ovf_hid[2] = {nullptr, nullptr};
     uint32_t *blk_tile_sums = nullptr;
     uint32_t *dt_bound = nullptr;  // GpuTimestepBounds word
     uint32_t *counters = nullptr;
@@ -275,6 +281,13 @@ static uint32_t next_pow2(uint32_t v) {
     return c;
 }
 
+// Table slots per region, as a shift (REGIONS of them, or one slot each).
+static uint32_t region_shift(uint32_t cap) {
+    uint32_t s = 0;
+    while ((cap >> s) > REGIONS) s++;
+    return s;
+}
+
 static float u2f(uint32_t x) {
     float f;
     std::memcpy(&f, &x, 4);
@@ -349,10 +362,10 @@ static int alloc_particle_buffers(slosh_data *d, size_t pcap, bool sand) {
     TRY(dalloc(&d->pslot, pcap));
     TRY(dalloc(&d->prank, pcap));
     TRY(dalloc(&d->perm, pcap));
-    TRY(dalloc(&d->mv_key, pcap));
-    TRY(dalloc(&d->mv_slot, pcap));
-    TRY(dalloc(&d->ovf_slot, pcap));
-    TRY(dalloc(&d->ovf_hid, pcap));
+    for (int i = 0; i < 2; i++) {
+        TRY(dalloc(&d->ovf_slot[i], pcap));
+        TRY(dalloc(&d->ovf_hid[i], pcap));
+    }
     TRY(dalloc(&d->items, max_items(pcap, d->cap)));
     // Every entry a kernel can read is a particle index even before the first sort.
     HIP_TRY(hipMemset(d->perm, 0, sizeof(uint32_t) * (pcap ? pcap : 1)));
@@ -385,10 +398,10 @@ static void free_particle_buffers(slosh_data *d) {
     dfree(d->pslot);
     dfree(d->prank);
     dfree(d->perm);
-    dfree(d->mv_key);
-    dfree(d->mv_slot);
-    dfree(d->ovf_slot);
-    dfree(d->ovf_hid);
+    for (int i = 0; i < 2; i++) {
+        dfree(d->ovf_slot[i]);
+        dfree(d->ovf_hid[i]);
+    }
     dfree(d->items);
 }
 
@@ -1060,8 +1073,8 @@ static int run_step(slosh_pipeline *pl, slosh_data *d, hipStream_t st, const slo
     StepParams P = make_params(d);
     const uint32_t n = (uint32_t)d->n;
 
-    // Steady state: the previous substep's fused kernels prepared this table and
-    // the mover list, so the sort is one launch. Hooks observe or replace passes
+    // Steady state: the previous substep's fused kernels prepared this table, its block
+    // lists and the mover lists, so nothing is left of the sort to launch. Hooks observe or replace passes
     // with the full sort's result (the sorted list), so they get the full sort.
     const bool fast = d->next_primed && !any_hook;
     GridBuffers g;
@@ -1078,16 +1091,7 @@ static int run_step(slosh_pipeline *pl, slosh_data *d, hipStream_t st, const slo
     g.perm = d->perm;
     g.counters = ctr_set(d, cur_g);
     g.tile_sums = d->blk_tile_sums;
-    g.mv_key = d->mv_key;
-    g.mv_slot = d->mv_slot;
-    g.mcount = d->mcount[cur_g];
-    g.mlist = d->mlist;
-    g.ovf_slot = d->ovf_slot;
-    g.ovf_hid = d->ovf_hid;
-    g.prev_start = d->blk_start[prev_g];
-    g.prev_cnt = d->blk_cnt[prev_g];
-    g.prev_stay = d->stay[prev_g];
-    g.bin = d->bin;
+    g.rsum = d->rsum[cur_g];
 
     // The fused path (no hooks, built-in P2G and particle update) prepares the
     // next substep's table and sort inside this substep's kernels.
@@ -1095,9 +1099,14 @@ static int run_step(slosh_pipeline *pl, slosh_data *d, hipStream_t st, const slo
     NextTableBuffers next;
     next.keys = d->keys[prev_g];
     next.counters = ctr_set(d, prev_g);
-    next.mcount = d->mcount[prev_g];
-    next.mv_key = d->mv_key;
-    next.mv_slot = d->mv_slot;
+    next.arrive = d->arrive[prev_g];
+    next.mlist = d->mlist[prev_g];
+    next.ovf_slot = d->ovf_slot[prev_g];
+    next.ovf_hid = d->ovf_hid[prev_g];
+    next.rlist = d->rlist[prev_g];
+    next.rcnt = d->rcnt[prev_g];
+    next.rsum = d->rsum[prev_g];
+    next.rshift = region_shift(d->cap);
     next.prime = prime ? 1u : 0u;
 
     PassEvents pe;
@@ -1119,15 +1128,24 @@ static int run_step(slosh_pipeline *pl, slosh_data *d, hipStream_t st, const slo
     t.blk_start = d->blk_start[cur_g];
     t.blk_cnt = d->blk_cnt[cur_g];
     t.stay = d->stay[cur_g];
+    t.rlist = d->rlist[cur_g];
+    t.rcnt = d->rcnt[cur_g];
+    t.prev_keys = d->keys[prev_g];
+    t.arrive = d->arrive[cur_g];
+    t.prev_stay = d->stay[prev_g];
+    t.rshift = region_shift(d->cap);
+    t.blist_out = d->blist;
+    t.num_blocks = ctr_set(d, cur_g) + CTR_NUM_BLOCKS;
+    t.nbr_out = d->nbr;
+    t.rsum = d->rsum[cur_g];
+    t.rel = d->rel;
     t.items = d->items;
-    t.item_start = d->item_start;
     t.n_items = ctr_set(d, cur_g) + CTR_ITEMS;
     t.taken = d->taken;
     t.bin = d->bin;
-    t.mcount = d->mcount[cur_g];
-    t.mlist = d->mlist;
-    t.ovf_slot = d->ovf_slot;
-    t.ovf_hid = d->ovf_hid;
+    t.mlist = d->mlist[cur_g];
+    t.ovf_slot = d->ovf_slot[cur_g];
+    t.ovf_hid = d->ovf_hid[cur_g];
     t.tiles = d->tiles;
     t.nodes = d->nodes;
     t.coll_prev = (d->coll_cache && d->coll_prev_valid) ? (void *)d->coll[prev_g] : nullptr;
@@ -1141,7 +1159,7 @@ static int run_step(slosh_pipeline *pl, slosh_data *d, hipStream_t st, const slo
     if (!p2g_by_hook) {
         if (!K.builtin_transfers)
             return fail(SLOSH_E_NO_KERNELS, "pipeline built without builtin transfer kernels; a hook must handle run_p2g");
-        HIP_TRY(launch_p2g(P, pbufs(d, d->cur_p), (uint32_t)d->pcap, t, next, pass_events(ts, PASS_P2G, &pe), st));
+        HIP_TRY(launch_p2g(P, pbufs(d, d->cur_p), (uint32_t)d->pcap, t, pass_events(ts, PASS_P2G, &pe), st));
     }
     if (hooks && hooks->after_p2g && hooks->after_p2g(d, st, hs) != 0) return fail(SLOSH_E_HOOK, "after_p2g hook failed");
 
@@ -1157,8 +1175,8 @@ static int run_step(slosh_pipeline *pl, slosh_data *d, hipStream_t st, const slo
     cb.mesh_base = d->mesh_base;
     if (K.grid_update || !p2g_by_hook) {
         const uint32_t mode = p2g_by_hook ? 1u : 0u;
-        HIP_TRY(launch_grid_update(P, t, cb, mode, K.grid_update ? 1u : 0u, pass_events(ts, PASS_GRID_UPDATE, &pe),
-                                   st));
+        HIP_TRY(launch_grid_update(P, t, cb, next, mode, K.grid_update ? 1u : 0u,
+                                   pass_events(ts, PASS_GRID_UPDATE, &pe), st));
     }
     if (d->coll_cache) d->coll_prev_valid = 1;
     if (hooks && hooks->after_grid_update && hooks->after_grid_update(d, st, hs) != 0)
@@ -1437,15 +1455,18 @@ static void free_data(slosh_data *d) {
         dfree(d->blk_start[i]);
         dfree(d->blk_cnt[i]);
         dfree(d->stay[i]);
-        dfree(d->mcount[i]);
+        dfree(d->arrive[i]);
+        dfree(d->mlist[i]);
+        dfree(d->rlist[i]);
+        dfree(d->rcnt[i]);
+        dfree(d->rsum[i]);
     }
     dfree(d->blist);
     dfree(d->nbr);
     dfree(d->cell_cnt);
     dfree(d->cell_start);
-    dfree(d->mlist);
     dfree(d->bin);
-    dfree(d->item_start);
+    dfree(d->rel);
     dfree(d->taken);
     dfree(d->blk_tile_sums);
     dfree(d->counters);
@@ -1616,15 +1637,20 @@ static int create_impl(slosh_pipeline *pipeline, const slosh_sim_params *params,
         TRY(dalloc(&d->blk_start[i], cap));
         TRY(dalloc(&d->blk_cnt[i], cap));
         TRY(dalloc(&d->stay[i], cap));
-        TRY(dalloc(&d->mcount[i], cap));
+        TRY(dalloc(&d->arrive[i], cap));
+        TRY(dalloc(&d->mlist[i], cap * MOVER_CAP));
+        TRY(dalloc(&d->rlist[i], std::max<size_t>(cap, REGIONS)));
+        TRY(dalloc(&d->rcnt[i], REGIONS * RCNT_STRIDE));
+        TRY(dalloc(&d->rsum[i], REGIONS * RSUM_STRIDE));
+        HIP_TRY(hipMemset(d->rcnt[i], 0, 4 * REGIONS * RCNT_STRIDE));
+        HIP_TRY(hipMemset(d->rsum[i], 0, 8 * REGIONS * RSUM_STRIDE));
     }
     TRY(dalloc(&d->blist, cap));
     TRY(dalloc(&d->nbr, cap * NBR_STRIDE));
     TRY(dalloc(&d->cell_cnt, cap * NODES_PER_BLOCK));
     TRY(dalloc(&d->cell_start, cap * NODES_PER_BLOCK));
-    TRY(dalloc(&d->mlist, cap * MOVER_CAP));
     TRY(dalloc(&d->bin, cap));
-    TRY(dalloc(&d->item_start, cap));
+    TRY(dalloc(&d->rel, cap));
     TRY(dalloc(&d->taken, cap));
     TRY(dalloc(&d->blk_tile_sums, (cap + 4095) / 4096 + 1));
     TRY(dalloc(&d->counters, 16));
