@@ -1355,7 +1355,7 @@ __device__ inline uint32_t entry_slot(const BlockRange &r, uint32_t m) {
 // ---------------------------------------------------------------------------
 // Kernels.
 
-// P2G for one block per workgroup of 3 waves.
+// P2G for one block per workgroup of 3 SUB waves.
 // Phase 1 (per chunk of up to P2G_CHUNK members of the block): each thread
 // loads one particle (stayers are contiguous in storage) and stages in LDS what
 // every node of its stencil shares: mass, the APIC momentum at the stencil's
@@ -1365,7 +1365,7 @@ __device__ inline uint32_t entry_slot(const BlockRange &r, uint32_t m) {
 // The chunk is grouped by associated cell in LDS (a rank per particle from an
 // LDS counter per cell, a scan of the 64 counts, a list of staging indices).
 // Phase 2: lane = associated cell of the block, wave = z offset kz of the
-// stencil; each lane accumulates, over the particles of its cell in the chunk,
+// stencil (and which of every SUB members of the cell); each lane accumulates, over the particles of its cell in the chunk,
 // the contributions w_n (A0 + C^T (n h)) to the 9 nodes n = (kx, ky, kz) in 36
 // registers.
 // Phase 3: each wave sums its registers into its own slab tile (z planes kz to
@@ -1392,36 +1392,38 @@ __device__ inline uint32_t p2g_tile_lds(uint32_t x, uint32_t y, uint32_t z) {
 }
 
 // 35,088 bytes at 512 particles per chunk: four workgroups (12 waves) fit in a
-// CU's 160 KiB of LDS, as many as the registers allow.
-template <int P2G_CHUNK>
+// CU's 160 KiB of LDS, as many as the registers allow; 26,384 bytes at 384.
+template <int P2G_CHUNK, int SUB>
 struct P2GShared {
     static constexpr int LDS = P2G_CHUNK + P2G_CHUNK / 16;
     union {
         // (m, A0), (f, C0), (C1..C4), (C5..C8) per member, grouped by associated cell
         float4 sp4[4][LDS];
         // after the block's last chunk: each wave's sums over its slab (z planes kz..kz+3)
-        float4 slab[3][P2G_SLAB_LDS];
-        uint32_t extra[192];  // this block's overflow movers of one round: read by
-                              // p2g_chunk before it stages anything
+        float4 slab[3 * SUB][P2G_SLAB_LDS];
+        uint32_t extra[192 * SUB];  // this block's overflow movers of one round: read by
+                                    // p2g_chunk before it stages anything
     };
     uint32_t lcnt[64];
-    uint32_t wsum[3];
+    uint32_t wsum[3 * SUB];
 };
-static_assert(sizeof(float4) * 3 * P2G_SLAB_LDS <= sizeof(P2GShared<192>::sp4),
+static_assert(sizeof(float4) * 3 * P2G_SLAB_LDS <= sizeof(P2GShared<192, 1>::sp4),
               "the slab tiles take no LDS beyond the staging of the smallest chunk");
-static_assert(sizeof(P2GShared<512>) <= 163840 / 4, "P2G at 512 per chunk must fit four workgroups per CU");
+static_assert(sizeof(P2GShared<512, 1>) <= 163840 / 4, "P2G at 512 per chunk must fit four workgroups per CU");
 
 // Phase 1 and 2 for `kn` entries of the block's sequence; entry t's storage slot
 // is slot_of(t). An entry is a member if its associated block is this block
 // (candidates that moved to another block are skipped; every other entry is one
 // by construction). Every thread of the workgroup calls it. `tot` (wave 0, lane
 // = cell) accumulates the block's cell counts.
-template <int P2G_CHUNK, typename SlotOf>
-__device__ inline void p2g_chunk(const StepParams &P, P2GShared<P2G_CHUNK> &S, uint32_t kn, SlotOf slot_of, const float4 *__restrict__ pos, const float4 *__restrict__ vm,
+template <int P2G_CHUNK, int SUB, typename SlotOf>
+__device__ inline void p2g_chunk(const StepParams &P, P2GShared<P2G_CHUNK, SUB> &S, uint32_t kn, SlotOf slot_of, const float4 *__restrict__ pos, const float4 *__restrict__ vm,
                                  const float *__restrict__ C, const float *__restrict__ fdt, uint32_t pcap,
                                  uint32_t block_key, float (&acc)[9][4], uint32_t &tot) {
-    constexpr int R = (P2G_CHUNK + 191) / 192;
-    const uint32_t kz = threadIdx.x >> 6, lane = threadIdx.x & 63u;
+    constexpr uint32_t T = 192 * SUB;
+    constexpr int R = (P2G_CHUNK + T - 1) / T;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63u;
+    const uint32_t kz = SUB == 1 ? wave : wave % 3u, part = SUB == 1 ? 0u : wave / 3u;
     const float h = P.h;
     const float kzh = (float)kz * h;
     // The slab's z weight is one piece of the quadratic B-spline of the offset f,
@@ -1435,7 +1437,7 @@ __device__ inline void p2g_chunk(const StepParams &P, P2GShared<P2G_CHUNK> &S, u
     uint32_t pp[R];
 #pragma unroll
     for (int r = 0; r < R; r++) {
-        const uint32_t t = threadIdx.x + 192u * r;
+        const uint32_t t = threadIdx.x + T * r;
         pp[r] = t < kn ? slot_of(t) : SLOSH_NONE;
     }
     float4 ps[R], vv[R];
@@ -1484,7 +1486,7 @@ __device__ inline void p2g_chunk(const StepParams &P, P2GShared<P2G_CHUNK> &S, u
     // Every wave scans the 64 counts (lane = cell) and writes the same starts.
     const uint32_t cnt = S.lcnt[lane];
     const uint32_t cs = wave_inclusive_scan(cnt) - cnt;
-    if (kz == 0) tot += cnt;
+    if (wave == 0) tot += cnt;
     // Each member's cell start from the lane of its cell (every wave holds all 64).
     uint32_t cstart[R];
 #pragma unroll
@@ -1500,7 +1502,7 @@ __device__ inline void p2g_chunk(const StepParams &P, P2GShared<P2G_CHUNK> &S, u
         S.sp4[3][q] = make_float4(cc[r][5], cc[r][6], cc[r][7], cc[r][8]);
     }
     __syncthreads();
-    for (uint32_t j = cs; j < cs + cnt; j++) {
+    for (uint32_t j = cs + part; j < cs + cnt; j += SUB) {
         const uint32_t q = p2g_slot(j);
         const float4 s0 = S.sp4[0][q], s1 = S.sp4[1][q], s2 = S.sp4[2][q], s3 = S.sp4[3][q];
         const float m = s0.x;
@@ -1536,63 +1538,79 @@ __device__ inline void p2g_chunk(const StepParams &P, P2GShared<P2G_CHUNK> &S, u
         }
     }
     __syncthreads();
-    if (kz == 0) S.lcnt[lane] = 0u;
+    if (wave == 0) S.lcnt[lane] = 0u;
 }
 
-// Chunks of up to 384 members fit in 128 VGPRs (4 waves/SIMD; their LDS allows 5
-// workgroups per CU); 512 needs 132 (3 waves/SIMD, as its 35 KB of LDS allow).
-//
-// One workgroup per block, the blocks of a region on the XCD that also updates their
-// nodes and particles (xcd_item). In the steady state it starts from the regional
-// lists and finds the block's particles through the previous table.
-// A lane's lookup in progress: its key, the slot probed first and what is there.
-struct Lookup {
-    uint32_t key, slot, seen;
-};
-
-// Entry `lane` (see NBR_STRIDE) of a block's neighbour table: the first probe. Most
-// lookups end there, and the load is in flight through the block's sums.
-__device__ inline void find_neighbours(const StepParams &P, const uint32_t *__restrict__ keys,
-                                       const uint32_t *__restrict__ prev_keys, uint32_t block_key, uint32_t lane,
-                                       Lookup &l) {
-    if (lane >= NBR_MINUS + 7u) return;
+// Key and first slot of entry `lane` (see NBR_STRIDE) of a block's neighbour table.
+__device__ inline uint32_t neighbour_key(const StepParams &P, uint32_t block_key, uint32_t lane, uint32_t *slot) {
     int bx, by, bz;
     uint32_t scene;
     unpack_key(P.batched, block_key, &bx, &by, &bz, &scene);
     const int d = lane == NBR_PREV ? 0 : (int)(lane & 7u) + 1, s = lane < NBR_MINUS ? 1 : -1;
-    l.key = pack_key(P.batched, scene, bx + s * ((d >> 2) & 1), by + s * ((d >> 1) & 1), bz + s * (d & 1));
-    l.slot = hash_key(l.key) & (P.cap - 1u);
-    l.seen = (lane == NBR_PREV ? prev_keys : keys)[l.slot];
+    const uint32_t key = pack_key(P.batched, scene, bx + s * ((d >> 2) & 1), by + s * ((d >> 1) & 1), bz + s * (d & 1));
+    *slot = hash_key(key) & (P.cap - 1u);
+    return key;
+}
+
+// The neighbours' first probes: most lookups end there, and the load is in flight
+// through the block's sums.
+__device__ inline uint32_t probe_neighbours(const StepParams &P, const SortInputs &in, const uint32_t *__restrict__ keys,
+                                            uint32_t block_key, uint32_t lane) {
+    uint32_t slot, seen = 0u;
+    neighbour_key(P, block_key, lane, &slot);
+    if (lane < NBR_MINUS + 7u) seen = (lane == NBR_PREV ? in.prev_keys : keys)[slot];
+    return seen;
 }
 
 // By P2G's first wave, of a steady-state block: the rest of the lookups, and what the
 // kernels after it read.
 __device__ inline void finish_block(const StepParams &P, const SortInputs &in, const uint32_t *__restrict__ keys,
-                                    uint32_t hid, uint32_t lane, uint4 range, const BlockRange &br, const Lookup &l) {
+                                    uint32_t hid, uint32_t block_key, uint32_t lane, uint4 range, uint32_t total,
+                                    uint32_t seen) {
+    uint32_t slot;
+    const uint32_t key = neighbour_key(P, block_key, lane, &slot);
     if (lane < NBR_MINUS + 7u) {
         const uint32_t *table = lane == NBR_PREV ? in.prev_keys : keys;
-        uint32_t slot = l.slot, seen = l.seen;
-        for (uint32_t k = 1; seen != l.key && seen != SLOSH_NONE && k < P.cap; k++) {
+        for (uint32_t k = 1; seen != key && seen != SLOSH_NONE && k < P.cap; k++) {
             slot = (slot + 1u) & (P.cap - 1u);
             seen = table[slot];
         }
-        in.nbr[(size_t)hid * NBR_STRIDE + lane] = seen == l.key ? slot : SLOSH_NONE;
+        in.nbr[(size_t)hid * NBR_STRIDE + lane] = seen == key ? slot : SLOSH_NONE;
     }
     if (lane == 0u) {
         in.bin[hid] = range;
-        in.blk_cnt[hid] = br.total;
+        in.blk_cnt[hid] = total;
     }
 }
 
-template <int P2G_CHUNK, bool FAST>
-__global__ __launch_bounds__(192, P2G_CHUNK <= 384 ? 4 : 1) void k_p2g(StepParams P, const float4 *__restrict__ pos,
+// One workgroup per block, a block's on the XCD that also updates its nodes and
+// particles (xcd_item); SUB = 2 gives each cell's members to two sets of three waves. In
+// the steady state it starts from the regional lists and the ranges the previous substep
+// left. A block takes ~6 us from its first dependent load (list entry, range, member
+// slots, particles) to its tile, so what counts with many blocks is how many are
+// resident: 512 members per chunk hold four workgroups to a CU (35 KB of LDS, 135 VGPRs),
+// 384 let in five (113 VGPRs): 1M particles 43 -> 39 us, 48 scenes 101 -> 88, 2.1M in 42k
+// blocks 248 -> 206. Chunks of 256 or 192 take no fewer registers than that and more
+// rounds (2.1M: 204, 209; 1M: 42, 44).
+// While all blocks are resident at once, the longest one's latency counts instead: a
+// block of 512 then goes in one chunk (131k particles: 14.2 us against 15.3), and with a
+// CU for each, in six waves that halve its longest cells and its loads per thread (2k
+// particles 11.8 -> 9.7 us, 33k 12.2 -> 10.4, 80k 12.6 -> 12.2; but 131k 14.2 -> 16.6,
+// 2.1M 248 -> 437). The count of blocks is not known to the host; scenes have one (with
+// the empty neighbours) per 150 to 300 particles.
+#define P2G_SUB_N 98304u    // two sets of waves up to here
+#define P2G_WIDE_N 262144u  // chunks of 512 up to here
+
+template <int P2G_CHUNK, bool FAST, int SUB>
+__global__ __launch_bounds__(192 * SUB, SUB == 1 && P2G_CHUNK <= 384 ? 4 : 1) void k_p2g(StepParams P, const float4 *__restrict__ pos,
                                              const float4 *__restrict__ vm, const float *__restrict__ C,
                                              const float *__restrict__ fdt, uint32_t pcap, Members M, SortInputs in,
                                              const uint32_t *__restrict__ keys, float4 *__restrict__ tiles,
                                              uint32_t *__restrict__ cell_cnt) {
-    __shared__ P2GShared<P2G_CHUNK> S;
+    __shared__ P2GShared<P2G_CHUNK, SUB> S;
+    constexpr uint32_t T = 192 * SUB;
     const uint32_t n_ovf = M.counters[CTR_OVERFLOW];
-    const uint32_t kz = threadIdx.x >> 6, lane = threadIdx.x & 63u;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63u;
     const int lx = lane & 3, ly = (lane >> 2) & 3, lz = lane >> 4;
     uint32_t B, upto = 0u;  // blocks; FAST: those of the regions up to the lane's
     if constexpr (FAST) {
@@ -1609,7 +1627,7 @@ __global__ __launch_bounds__(192, P2G_CHUNK <= 384 ? 4 : 1) void k_p2g(StepParam
         uint32_t hid, block_key;
         BlockRange br;
         uint4 range;
-        Lookup look;
+        uint32_t seen = 0u;
         if constexpr (FAST) {
             const uint32_t r = (uint32_t)__popcll(__ballot(upto <= k));
             const uint32_t before = r ? __builtin_amdgcn_readlane(upto, r - 1u) : 0u;
@@ -1617,11 +1635,15 @@ __global__ __launch_bounds__(192, P2G_CHUNK <= 384 ? 4 : 1) void k_p2g(StepParam
             hid = __builtin_amdgcn_readfirstlane(e.x);
             block_key = __builtin_amdgcn_readfirstlane(e.y);
             const uint4 a = in.arrive[hid];
-            range = make_uint4(0u, 0u, 0u, a.x);
-            if (a.y != SLOSH_NONE) range = make_uint4(a.z, a.w, in.prev_stay[a.y], a.x);
+            const uint32_t prev = __builtin_amdgcn_readfirstlane(a.y);
+            range = make_uint4(0u, 0u, 0u, __builtin_amdgcn_readfirstlane(a.x));
+            if (prev != SLOSH_NONE) {
+                range.x = __builtin_amdgcn_readfirstlane(a.z);
+                range.y = __builtin_amdgcn_readfirstlane(a.w);
+                range.z = in.prev_stay[prev];
+            }
             br = steady_range(M, hid, range);
-            // The neighbours' first probes, resolved after the sums (below).
-            if (kz == 0u) find_neighbours(P, keys, in.prev_keys, block_key, lane, look);
+            if (wave == 0u) seen = probe_neighbours(P, in, keys, block_key, lane);
             if (threadIdx.x == 0u) in.blist[k] = hid;
         } else {
             hid = M.blist[k];
@@ -1633,9 +1655,9 @@ __global__ __launch_bounds__(192, P2G_CHUNK <= 384 ? 4 : 1) void k_p2g(StepParam
         // only below: a block that all its particles left writes a zero tile.)
         const uint32_t n_main = br.cand_n + br.list_n;
         if (n_main == 0u) {
-            if (kz == 0u) {
+            if (wave == 0u) {
                 cell_cnt[(size_t)hid * NODES_PER_BLOCK + lane] = 0u;
-                if constexpr (FAST) finish_block(P, in, keys, hid, lane, range, br, look);
+                if constexpr (FAST) finish_block(P, in, keys, hid, block_key, lane, range, br.total, seen);
             }
             continue;
         }
@@ -1645,24 +1667,28 @@ __global__ __launch_bounds__(192, P2G_CHUNK <= 384 ? 4 : 1) void k_p2g(StepParam
         uint32_t tot = 0u;
         for (uint32_t chunk = 0; chunk < n_main; chunk += P2G_CHUNK) {
             const uint32_t kn = n_main - chunk < (uint32_t)P2G_CHUNK ? n_main - chunk : (uint32_t)P2G_CHUNK;
-            p2g_chunk<P2G_CHUNK>(P, S, kn, [&](uint32_t t) { return entry_slot(br, chunk + t); }, pos, vm, C, fdt,
+            p2g_chunk<P2G_CHUNK, SUB>(P, S, kn, [&](uint32_t t) { return entry_slot(br, chunk + t); }, pos, vm, C, fdt,
                                  pcap, block_key, acc, tot);
         }
         if (br.overflow) {
             // This block's movers beyond its list: picked out of the overflow list,
-            // one round of 192 entries at a time.
-            for (uint32_t ob = 0; ob < n_ovf; ob += 192u) {
+            // one round of T entries at a time.
+            for (uint32_t ob = 0; ob < n_ovf; ob += T) {
                 const uint32_t i = ob + threadIdx.x;
                 const bool mine = i < n_ovf && M.ovf_hid[i] == hid;
                 const uint64_t mm = __ballot(mine);
                 __syncthreads();  // the previous round's readers of `extra` are done
-                if (lane == 0) S.wsum[kz] = (uint32_t)__popcll(mm);
+                if (lane == 0) S.wsum[wave] = (uint32_t)__popcll(mm);
                 __syncthreads();
-                const uint32_t before = (kz > 0 ? S.wsum[0] : 0u) + (kz > 1 ? S.wsum[1] : 0u);
-                const uint32_t kn = S.wsum[0] + S.wsum[1] + S.wsum[2];
+                uint32_t before = 0u, kn = 0u;
+#pragma unroll
+                for (uint32_t w = 0; w < 3u * SUB; w++) {
+                    before += w < wave ? S.wsum[w] : 0u;
+                    kn += S.wsum[w];
+                }
                 if (mine) S.extra[before + (uint32_t)__popcll(mm & lanemask_lt())] = M.ovf_slot[i];
                 if (kn > 0)
-                    p2g_chunk<P2G_CHUNK>(P, S, kn, [&](uint32_t t) { return S.extra[t]; }, pos, vm, C, fdt, pcap,
+                    p2g_chunk<P2G_CHUNK, SUB>(P, S, kn, [&](uint32_t t) { return S.extra[t]; }, pos, vm, C, fdt, pcap,
                                          block_key, acc, tot);
             }
         }
@@ -1674,7 +1700,7 @@ __global__ __launch_bounds__(192, P2G_CHUNK <= 384 ? 4 : 1) void k_p2g(StepParam
         // LDS), in 9 rounds in which its 64 lanes touch 64 distinct nodes; then each
         // node is the sum of the slabs that cover it, in wave order.
         __syncthreads();  // the staging's readers are done
-        float4 *slab = S.slab[kz];
+        float4 *slab = S.slab[wave];
         for (uint32_t j = lane; j < P2G_SLAB_LDS; j += 64) slab[j] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
         __asm__ volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
 #pragma unroll
@@ -1694,24 +1720,27 @@ __global__ __launch_bounds__(192, P2G_CHUNK <= 384 ? 4 : 1) void k_p2g(StepParam
                 __asm__ volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
             }
         __syncthreads();
-        for (uint32_t j = threadIdx.x; j < TILE_NODES; j += 192) {
+        for (uint32_t j = threadIdx.x; j < TILE_NODES; j += T) {
             const uint32_t x = j % 6u, y = (j / 6u) % 6u, z = j / 36u;
             float4 t = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
 #pragma unroll
             for (uint32_t w = 0; w < 3; w++) {
                 if (z < w || z > w + 3u) continue;
-                const float4 u = S.slab[w][p2g_tile_lds(x, y, z - w)];
-                t.x += u.x;
-                t.y += u.y;
-                t.z += u.z;
-                t.w += u.w;
+#pragma unroll
+                for (uint32_t p = 0; p < SUB; p++) {
+                    const float4 u = S.slab[w + 3u * p][p2g_tile_lds(x, y, z - w)];
+                    t.x += u.x;
+                    t.y += u.y;
+                    t.z += u.z;
+                    t.w += u.w;
+                }
             }
             tiles[(size_t)hid * TILE_NODES + tile_index(x, y, z)] = t;
         }
-        if (kz == 0) cell_cnt[(size_t)hid * NODES_PER_BLOCK + lane] = tot;
+        if (wave == 0u) cell_cnt[(size_t)hid * NODES_PER_BLOCK + lane] = tot;
         if (threadIdx.x == 0u) in.rel[hid] = make_uint2((uint32_t)(rel >> 32), (uint32_t)rel);
         if constexpr (FAST)
-            if (kz == 0u) finish_block(P, in, keys, hid, lane, range, br, look);
+            if (wave == 0u) finish_block(P, in, keys, hid, block_key, lane, range, br.total, seen);
     }
 }
 
@@ -2638,15 +2667,21 @@ static Members members_of(const TransferBuffers &t) {
 
 hipError_t launch_p2g(const StepParams &P, const ParticleBuffers &pb, uint32_t pcap, const TransferBuffers &t,
                       const PassEvents *ev, hipStream_t stream) {
-    auto kern = t.fast ? (P.p2g_chunk == 192u   ? k_p2g<192, true>
-                          : P.p2g_chunk == 256u ? k_p2g<256, true>
-                          : P.p2g_chunk == 384u ? k_p2g<384, true>
-                                                : k_p2g<512, true>)
-                       : (P.p2g_chunk == 192u   ? k_p2g<192, false>
-                          : P.p2g_chunk == 256u ? k_p2g<256, false>
-                          : P.p2g_chunk == 384u ? k_p2g<384, false>
-                                                : k_p2g<512, false>);
-    launch_kernel(ev, kern, dim3(block_grid(P, 1)), dim3(192), 0, stream, P, (const float4 *)pb.pos,
+    // 512 by size (the comment at P2G_SUB_N).
+    const bool by_size = P.p2g_chunk == 512u;
+    const bool sub = by_size && P.n <= P2G_SUB_N;
+    const uint32_t chunk = by_size && P.n > P2G_WIDE_N ? 384u : P.p2g_chunk;
+    auto kern = t.fast ? (sub             ? k_p2g<512, true, 2>
+                          : chunk == 192u ? k_p2g<192, true, 1>
+                          : chunk == 256u ? k_p2g<256, true, 1>
+                          : chunk == 384u ? k_p2g<384, true, 1>
+                                          : k_p2g<512, true, 1>)
+                       : (sub             ? k_p2g<512, false, 2>
+                          : chunk == 192u ? k_p2g<192, false, 1>
+                          : chunk == 256u ? k_p2g<256, false, 1>
+                          : chunk == 384u ? k_p2g<384, false, 1>
+                                          : k_p2g<512, false, 1>);
+    launch_kernel(ev, kern, dim3(block_grid(P, 1)), dim3(sub ? 384 : 192), 0, stream, P, (const float4 *)pb.pos,
                   (const float4 *)pb.vm, (const float *)pb.C, (const float *)t.fdt, pcap, members_of(t), sort_inputs(t),
                   t.keys, t.tiles, t.cell_cnt);
     return hipGetLastError();
