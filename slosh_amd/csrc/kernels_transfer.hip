@@ -1810,11 +1810,11 @@ __device__ inline void mesh_queries(const Colliders &cs, const float4 *box, Mesh
 }
 
 // What the grid update prepares for the fused G2P kernel: each block's storage start
-// and its items (64 consecutive entries of its sequence: header id, index of the 64),
-// from the regions' sums and the block's place in them, and cleared counters (output
-// slots taken, stayers).
+// and its items (ITEM_*, one per 64 consecutive entries of its sequence), from the
+// regions' sums and the block's place in them, and cleared counters (output slots taken,
+// stayers).
 struct ItemLists {
-    uint2 *items;
+    uint32_t *items;
     const unsigned long long *rsum;
     const uint2 *rel;
     uint32_t *blk_start, *taken, *stay, *n_items;
@@ -1889,8 +1889,22 @@ __global__ __launch_bounds__(MESH ? 64 * MESH_WAVES : 256) void k_grid_update(St
             if (n) {
                 const uint2 rel = L.rel[hid];
                 const uint32_t item0 = rel.y + (r ? __builtin_amdgcn_readlane(up_i, r - 1u) : 0u);
-                for (uint32_t c = lane; c < n; c += 64u) L.items[item0 + c] = make_uint2(hid, c);
-                if (M.fast && lane == 0u) L.blk_start[hid] = rel.x + (r ? __builtin_amdgcn_readlane(up_p, r - 1u) : 0u);
+                const uint32_t start =
+                    M.fast ? rel.x + (r ? __builtin_amdgcn_readlane(up_p, r - 1u) : 0u) : M.blk_start[hid];
+                if (M.fast && lane == 0u) L.blk_start[hid] = start;
+                // Four items at a time, a word per lane.
+                const uint32_t w = lane & 15u;
+                uint32_t v = (uint32_t)__shfl((int)nb, (int)w);
+                v = w == ITEM_HID ? hid : v;
+                v = w == ITEM_CAND_LO ? br.cand_lo : v;
+                v = w == ITEM_CAND_N ? br.cand_n : v;
+                v = w == ITEM_LIST_N ? br.list_n : v;
+                v = w == ITEM_START ? start : v;
+                v = w == ITEM_KEY ? block_key : v;
+                v = w == ITEM_TOTAL ? br.total : v;
+                v = w == ITEM_OVERFLOW ? (br.overflow ? 1u : 0u) : v;
+                for (uint32_t c = lane >> 4; c < n; c += 4u)
+                    L.items[(size_t)(item0 + c) * ITEM_WORDS + w] = w == ITEM_FIRST ? 64u * c : v;
             }
             if (lane == 0u) {
                 L.taken[hid] = 0u;
@@ -2077,11 +2091,10 @@ __device__ inline void load_halo(float4 *__restrict__ sh, const float4 *__restri
     }
 }
 
-// The same by one wave into its own LDS tile: lanes 0..6 load the neighbour ids,
-// each lane takes its nodes' from them.
-__device__ inline void load_halo_wave(float4 *__restrict__ sh, const float4 *__restrict__ nodes,
-                                      const uint32_t *__restrict__ nbr, uint32_t hid, uint32_t lane) {
-    const uint32_t nb = lane < 7u ? nbr[(size_t)hid * NBR_STRIDE + lane] : hid;
+// The same by one wave into its own LDS tile: lanes 0..6 hold the neighbour ids, lane 7
+// the block's, and each lane takes its nodes' from them.
+__device__ inline void load_halo_wave(float4 *__restrict__ sh, const float4 *__restrict__ nodes, uint32_t nb,
+                                      uint32_t lane) {
     constexpr uint32_t R = (TILE_NODES + 63u) / 64u;
     float4 v[R];
 #pragma unroll
@@ -2157,10 +2170,8 @@ __device__ inline const T &late_args() {
 
 template <uint32_t MODELS, bool F64>
 __global__ __launch_bounds__(256, F64 && MODELS != 3u ? 3 : 4) void k_g2p_update(G2pArgs args, Members M,
-                                                    const uint2 *__restrict__ items,
-                                                    const uint32_t *__restrict__ blk_start,
-                                                    const float4 *__restrict__ nodes,
-                                                    const uint32_t *__restrict__ keys) {
+                                                    const uint32_t *__restrict__ items,
+                                                    const float4 *__restrict__ nodes) {
     extern __shared__ float4 halo[];  // TILE_NODES per wave
     // integrate_bodies: reads no particle or grid state (the impulses it applies
     // are only written by the host), so the last workgroup runs it alongside the
@@ -2179,13 +2190,17 @@ __global__ __launch_bounds__(256, F64 && MODELS != 3u ? 3 : 4) void k_g2p_update
         // ahead of the loop and holding in (spilled) registers.
         uint32_t lane = threadIdx.x & 63u;
         asm volatile("" : "+v"(lane));
-        const uint2 item = items[i];
-        const uint32_t hid = __builtin_amdgcn_readfirstlane(item.x);
-        const uint32_t first = __builtin_amdgcn_readfirstlane(item.y) * 64u;
-        const BlockRange br = M.fast ? block_range<true>(M, hid) : block_range<false>(M, hid);
-        const uint32_t s0 = __builtin_amdgcn_readfirstlane(blk_start[hid]);
-        const uint32_t block_key = __builtin_amdgcn_readfirstlane(keys[hid]);
-        const uint32_t total = __builtin_amdgcn_readfirstlane(br.total);
+        const uint32_t item = items[(size_t)i * ITEM_WORDS + (lane & 15u)];
+        const uint32_t hid = __builtin_amdgcn_readlane(item, ITEM_HID);
+        const uint32_t first = __builtin_amdgcn_readlane(item, ITEM_FIRST);
+        const uint32_t s0 = __builtin_amdgcn_readlane(item, ITEM_START);
+        const uint32_t block_key = __builtin_amdgcn_readlane(item, ITEM_KEY);
+        const uint32_t total = __builtin_amdgcn_readlane(item, ITEM_TOTAL);
+        BlockRange br;
+        br.cand_lo = __builtin_amdgcn_readlane(item, ITEM_CAND_LO);
+        br.cand_n = __builtin_amdgcn_readlane(item, ITEM_CAND_N);
+        br.list = M.fast ? M.mlist + (size_t)hid * MOVER_CAP : M.perm + s0;
+        br.list_n = __builtin_amdgcn_readlane(item, ITEM_LIST_N);
         // The item's entries (a candidate is a member only if it is still in the
         // block); the block's first item then takes the overflow list, only if some
         // of the block's movers overflowed theirs (entries of other blocks are
@@ -2194,7 +2209,8 @@ __global__ __launch_bounds__(256, F64 && MODELS != 3u ? 3 : 4) void k_g2p_update
         // next table. Every lane runs the same number of iterations (the wave-level
         // counting and run detection see all lanes).
         const uint32_t n_main = br.cand_n + br.list_n;
-        const uint32_t n_ovf = first == 0u && br.overflow ? M.counters[CTR_OVERFLOW] : 0u;
+        const uint32_t n_ovf =
+            first == 0u && __builtin_amdgcn_readlane(item, ITEM_OVERFLOW) ? M.counters[CTR_OVERFLOW] : 0u;
         for (uint32_t o = 0; o < 64u + n_ovf; o += 64u) {
             const G2pArgs &A = late_args<G2pArgs>();
             bool entry;
@@ -2223,7 +2239,7 @@ __global__ __launch_bounds__(256, F64 && MODELS != 3u ? 3 : 4) void k_g2p_update
                     oid = A.in.ids[p];
                 }
             }
-            load_halo_wave(sh, nodes, M.nbr, hid, lane);  // (the last iteration may have reused the tile)
+            load_halo_wave(sh, nodes, item, lane);  // (the last iteration may have reused the tile)
             const uint32_t wbits = __float_as_uint(ps.w);
             const uint32_t scene = wbits >> 1;
             const Stencil at = stencil_of(A.P.h, ps.x, ps.y, ps.z);
@@ -2753,8 +2769,8 @@ hipError_t launch_g2p_update(const StepParams &P, const ParticleBuffers &in, con
     const uint32_t waves = P.g2p_threads == 128u ? 2u : 4u;
     // One more workgroup (the last) integrates the rigid bodies.
     launch_kernel(ev, kern, dim3(item_grid(P, waves) + 1u), dim3(64u * waves),
-                  waves * TILE_NODES * (uint32_t)sizeof(float4), stream, args, members_of(t), (const uint2 *)t.items,
-                  (const uint32_t *)t.blk_start, (const float4 *)t.nodes, t.keys);
+                  waves * TILE_NODES * (uint32_t)sizeof(float4), stream, args, members_of(t),
+                  (const uint32_t *)t.items, (const float4 *)t.nodes);
     return hipGetLastError();
 }
 

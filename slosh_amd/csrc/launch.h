@@ -40,7 +40,7 @@ struct TransferBuffers {
     // and each block's place in them.
     unsigned long long *rsum;
     uint2 *rel;
-    uint2 *items;  // the fused G2P kernel's items (max_items of them)
+    uint32_t *items;  // the fused G2P kernel's items (max_items of ITEM_WORDS words)
     uint32_t *n_items, *taken;
     const uint32_t *mlist, *ovf_slot, *ovf_hid;
     uint32_t *errors;  // this substep's error word

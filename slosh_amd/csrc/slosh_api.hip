@@ -194,7 +194,7 @@ struct slosh_data {
     unsigned long long *rsum[2] = {nullptr, nullptr};
     uint2 *rel = nullptr;
     // The fused G2P kernel's items, and per block the output slots taken.
-    uint2 *items = nullptr;
+    uint32_t *items = nullptr;
     uint32_t *taken = nullptr;
     uint4 *bin = nullptr;       // per block: its previous-table block's range and stayers, its movers
     uint32_t *pslot = nullptr, *prank = nullptr, *perm = nullptr;
@@ -366,7 +366,7 @@ static int alloc_particle_buffers(slosh_data *d, size_t pcap, bool sand) {
         TRY(dalloc(&d->ovf_slot[i], pcap));
         TRY(dalloc(&d->ovf_hid[i], pcap));
     }
-    TRY(dalloc(&d->items, max_items(pcap, d->cap)));
+    TRY(dalloc(&d->items, ITEM_WORDS * max_items(pcap, d->cap)));
     // Every entry a kernel can read is a particle index even before the first sort.
     HIP_TRY(hipMemset(d->perm, 0, sizeof(uint32_t) * (pcap ? pcap : 1)));
     HIP_TRY(hipMemset(d->fdt, 0, sizeof(float) * 3 * (pcap ? pcap : 1)));

@@ -37,13 +37,13 @@ MAX_SCENES = 16383
 # Device bytes per particle slot of a batched MpmData: two particle buffers
 # (pos 16, vel+mass 16, C 36, F 36, vel_grad_det 4, id 4, Drucker-Prager state 12),
 # force_dt 12 x 2, by-id records 64 x 2, full-sort scratch 12 (slot, rank,
-# permutation), overflow movers (slot, block) 8 x 2, G2P items 1.
-BYTES_PER_PARTICLE = 2 * (16 + 16 + 36 + 36 + 4 + 4 + 12) + 2 * 12 + 2 * 64 + 12 + 16 + 1
+# permutation), overflow movers (slot, block) 8 x 2, G2P items 2.
+BYTES_PER_PARTICLE = 2 * (16 + 16 + 36 + 36 + 4 + 4 + 12) + 2 * 12 + 2 * 64 + 12 + 16 + 2
 # Device bytes per hash-grid slot: per table (two) the key, block start, count and
 # stayers 16, what the block receives 16, mover list 64 x 4 and block-list entry 8; the
 # flat block list 4, neighbour table 64, cell counts and starts 512, range 16, place in
-# its region 8, output slots taken 4, P2G tile 216 x 16, nodes 64 x 16, G2P items 8.
-BYTES_PER_BLOCK = 2 * (16 + 16 + 256 + 8) + 4 + 64 + 512 + 16 + 8 + 4 + 216 * 16 + 64 * 16 + 8
+# its region 8, output slots taken 4, P2G tile 216 x 16, nodes 64 x 16, G2P items 64.
+BYTES_PER_BLOCK = 2 * (16 + 16 + 256 + 8) + 4 + 64 + 512 + 16 + 8 + 4 + 216 * 16 + 64 * 16 + 64
 # Pinned host bytes an append stages one particle in.
 STAGING_BYTES_PER_PARTICLE = 200
 
