@@ -1229,20 +1229,20 @@ __device__ inline void advance_particle(const StepParams &P, float3 pos, float3 
 template <uint32_t MODELS, bool F64>
 __device__ inline void material_update(const StepParams &P, float *F, float4 model, const PStatic &st, uint32_t oid,
                                        uint32_t scene, float *dps, float *stress) {
-    uint32_t tag = __float_as_uint(model.x);
-    if ((MODELS & 2u) && tag == 1u) {
-        nh_stress(model.y, model.z, F, stress);
-    } else if ((MODELS & 1u) && tag == 0u) {
-        if (F64) fc_stress_f64(model.y, model.z, F, stress);
-        else fc_stress(model.y, model.z, F, stress);
-    } else if (((MODELS & 4u) && tag == 2u) || ((MODELS & 8u) && tag == 3u)) {
+    // A wave of several materials runs each step once, for the lanes of all the tags
+    // that take it.
+    const uint32_t tag = __float_as_uint(model.x);
+    if (((MODELS & 4u) && tag == 2u) || ((MODELS & 8u) && tag == 3u)) {
         float4 hp, pl;
         plastic_records(P, st, oid, scene, &hp, &pl);
         if (F64) dp_project_f64(dps, hp, pl.x, pl.y, F);
         else dp_project(dps, hp, pl.x, pl.y, F);
-        if (tag == 3u) nh_stress(model.y, model.z, F, stress);
-        else if (F64) fc_stress_f64(model.y, model.z, F, stress);
+    }
+    if (((MODELS & 1u) && tag == 0u) || ((MODELS & 4u) && tag == 2u)) {
+        if (F64) fc_stress_f64(model.y, model.z, F, stress);
         else fc_stress(model.y, model.z, F, stress);
+    } else if (((MODELS & 2u) && tag == 1u) || ((MODELS & 8u) && tag == 3u)) {
+        nh_stress(model.y, model.z, F, stress);
     } else {
 #pragma unroll
         for (int k = 0; k < 9; k++) stress[k] = 0.0f;
