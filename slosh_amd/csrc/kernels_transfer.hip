@@ -2213,6 +2213,8 @@ __global__ __launch_bounds__(256, F64 && MODELS != 3u ? 3 : 4) void k_g2p_update
             first == 0u && __builtin_amdgcn_readlane(item, ITEM_OVERFLOW) ? M.counters[CTR_OVERFLOW] : 0u;
         for (uint32_t o = 0; o < 64u + n_ovf; o += 64u) {
             const G2pArgs &A = late_args<G2pArgs>();
+            uint32_t l = lane;  // (opaque again: else the halo's addresses take 15 VGPRs throughout)
+            asm volatile("" : "+v"(l));
             bool entry;
             uint32_t p = 0u;
             if (o == 0u) {
@@ -2239,7 +2241,7 @@ __global__ __launch_bounds__(256, F64 && MODELS != 3u ? 3 : 4) void k_g2p_update
                     oid = A.in.ids[p];
                 }
             }
-            load_halo_wave(sh, nodes, item, lane);  // (the last iteration may have reused the tile)
+            load_halo_wave(sh, nodes, item, l);  // (the last iteration may have reused the tile)
             const uint32_t wbits = __float_as_uint(ps.w);
             const uint32_t scene = wbits >> 1;
             const Stencil at = stencil_of(A.P.h, ps.x, ps.y, ps.z);
