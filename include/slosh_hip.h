@@ -339,8 +339,9 @@ int slosh_device_view_get(slosh_data *data, slosh_device_view *out);
 
 /* ---- Launch shape (no reference counterpart: the wgpu pipeline fixes its
  * workgroup sizes in the shaders). p2g_chunk: particles staged in LDS per P2G
- * round (192, 256, 384; 512: at most, chosen by the particle count); g2p_threads: threads per G2P/particle-update
- * workgroup (128, 256); block_wgs: workgroups of the per-block kernels, which
+ * round (192, 256, 384; 512: at most, chosen by the particle count); g2p_threads:
+ * 128 or 256, kept for callers (the waves of G2P work alone, in workgroups of one);
+ * block_wgs: workgroups of the per-block kernels (eight times as many of G2P's), which
  * loop over the active blocks (64..65536). Results do not depend on it beyond
  * summation order within a cell. slosh_autotune times `trial_steps` substeps of
  * a private copy of `data` per candidate (coordinate search, best of two

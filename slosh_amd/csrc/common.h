@@ -122,7 +122,7 @@ struct StepParams {
     float u_mass;
     // Launch shape (autotuned): particles staged in LDS per P2G round, threads per
     // G2P/update workgroup, workgroups of the per-block kernels.
-    uint32_t p2g_chunk, g2p_threads, block_wgs;
+    uint32_t p2g_chunk, block_wgs;
 };
 
 // ---------------------------------------------------------------------------

@@ -8,7 +8,7 @@
 //                    6x6x6 tile, the slabs summed per node, is written once to HBM. Same per-(node, particle) arithmetic as
 //                    p2g_scatter_style.slang:84-148; only the summation order
 //                    differs (and is fixed for a given particle order).
-//   k_grid_update    one wave per block: node momentum = own tile + the halo
+//   k_grid_update    one wave per block (in a workgroup of its own): node momentum = own tile + the halo
 //                    parts of the 7 "-1" neighbours' tiles, then
 //                    grid_update.slang:38-163 (gravity, clamp, collision
 //                    cache / collide(), boundary projection).
@@ -1852,14 +1852,13 @@ __device__ inline void reset_next_table(const NextTable &nt, uint32_t cap) {
 // mode 0: node momentum from tiles; mode 1: nodes already hold momentum (P2G hook).
 // do_update 0: only combine tiles (grid update disabled).
 template <bool MESH>
-__global__ __launch_bounds__(MESH ? 64 * MESH_WAVES : 256) void k_grid_update(StepParams P, const float4 *__restrict__ tiles,
+__global__ __launch_bounds__(MESH ? 64 * MESH_WAVES : 64) void k_grid_update(StepParams P, const float4 *__restrict__ tiles,
                                                      float4 *__restrict__ nodes, const uint32_t *__restrict__ nbr,
                                                      const uint32_t *__restrict__ keys, Colliders cs,
                                                      const NodeColl *__restrict__ coll_prev, NodeColl *__restrict__ coll_cur,
                                                      Members M, ItemLists L, NextTable nt, uint32_t mode,
                                                      uint32_t do_update) {
     const uint32_t *__restrict__ blk_cnt = M.blk_cnt;
-    reset_next_table(nt, P.cap);
     __shared__ float4 cbox[2 * SLOSH_MAX_COLLIDERS];
     if (threadIdx.x < cs.count) collider_box<MESH>(cs, threadIdx.x, 1.5f * P.h, &cbox[2 * threadIdx.x], &cbox[2 * threadIdx.x + 1]);
     __syncthreads();
@@ -1875,7 +1874,7 @@ __global__ __launch_bounds__(MESH ? 64 * MESH_WAVES : 256) void k_grid_update(St
     __shared__ typename std::conditional<MESH, MeshShared, char>::type shared;
     const uint32_t xcd = blockIdx.x & 7u, wg = blockIdx.x >> 3, wgs = gridDim.x >> 3;
     const bool owner = !MESH || wave == 0u;
-    for (uint32_t j = MESH ? wg : wg * 4u + wave;; j += MESH ? wgs : wgs * 4u) {
+    for (uint32_t j = wg;; j += wgs) {
         const uint32_t k = xcd_item(xcd, j, B);
         if (k >= B) break;
         const uint32_t hid = __builtin_amdgcn_readfirstlane(M.blist[k]);
@@ -2007,6 +2006,7 @@ __global__ __launch_bounds__(MESH ? 64 * MESH_WAVES : 256) void k_grid_update(St
         }
         nodes[(size_t)hid * NODES_PER_BLOCK + lane] = make_float4(v.x, v.y, v.z, mass);
     }
+    reset_next_table(nt, P.cap);
 }
 
 struct Bodies {
@@ -2126,17 +2126,19 @@ struct NextSort {
 // F64: the SVD-based steps refined to FP64 accuracy. The bounds keep that variant of
 // every material at three waves per SIMD (168 VGPRs), the others at four or more.
 //
-// One wave per item: 64 consecutive entries of a block's sequence, with the
-// block's node halo in an LDS tile of the wave's own, so that waves share no
-// barrier and a block's last, partly filled round holds one wave instead of a
-// workgroup. With one workgroup per block a second round of 256 entries cost a
-// block 3.8 us of serial latency, and a block of 50 particles kept four waves;
-// per wave (medians of the kernel, before and after): 2.1M sand and spheres (42k
-// blocks) 643 -> 280 us, 48 scenes of three materials (2.0M) 320 -> 168 us, sand on
-// a heightfield (85k) 43 -> 19 us, dam break of 131k 15.7 -> 13.1 us and of 1M
-// 66 -> 46 us once it moves. The small scenes are bound by
-// the chain of dependent loads and the ~1000 instructions of one particle, the
-// large ones by memory (188 MB per launch at 1M) and issue.
+// One wave per item, in a workgroup of its own: 64 consecutive entries of a block's
+// sequence, with the block's node halo in an LDS tile, so that waves share no barrier
+// and a block's last, partly filled round holds one wave instead of a workgroup. With
+// one workgroup per block a second round of 256 entries cost a block 3.8 us of serial
+// latency, and a block of 50 particles kept four waves; per wave (medians of the kernel,
+// before and after): 2.1M sand and spheres (42k blocks) 643 -> 252 us, 48 scenes of
+// three materials (2.0M) 320 -> 156 us, sand on a heightfield (85k) 43 -> 19 us, dam
+// break of 131k 15.7 -> 13.1 us and of 1M 66 -> 46 us once it moves. (Four items to a
+// workgroup kept the registers of its finished waves idle until the last one ended and
+// put a small scene's waves on a quarter of the CUs: 266, 168 and, 8k particles of four
+// materials, 29 us against 19.) The small scenes are bound by the chain of dependent
+// loads and the ~1000 instructions of one particle, 1M by memory (188 MB per launch),
+// FP64 materials by latency at three waves per SIMD and half by issue.
 //
 // Output order: a block's members take the output slots [start, start + total)
 // of the block in order of arrival of their waves (one atomic per wave, issued
@@ -2169,26 +2171,24 @@ __device__ inline const T &late_args() {
 }
 
 template <uint32_t MODELS, bool F64>
-__global__ __launch_bounds__(256, F64 && MODELS != 3u ? 3 : 4) void k_g2p_update(G2pArgs args, Members M,
+__global__ __launch_bounds__(64, F64 && MODELS != 3u ? 3 : 4) void k_g2p_update(G2pArgs args, Members M,
                                                     const uint32_t *__restrict__ items,
                                                     const float4 *__restrict__ nodes) {
-    extern __shared__ float4 halo[];  // TILE_NODES per wave
+    __shared__ float4 sh[TILE_NODES];
     // integrate_bodies: reads no particle or grid state (the impulses it applies
     // are only written by the host), so the last workgroup runs it alongside the
     // particle update.
-    if (blockIdx.x == gridDim.x - 1u) {  // (the eighth range's last workgroup takes no items)
+    if (blockIdx.x == gridDim.x - 1u) {  // (the one beyond the eight ranges' workgroups)
         if (threadIdx.x < args.bodies.count) integrate_body(args.P, args.bodies, threadIdx.x);
         return;
     }
     const uint32_t n_items = M.counters[CTR_ITEMS];
-    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), waves = blockDim.x >> 6;
-    float4 *sh = halo + wave * TILE_NODES;
-    for (uint32_t j = (blockIdx.x >> 3) * waves + wave;; j += (gridDim.x >> 3) * waves) {
+    for (uint32_t j = blockIdx.x >> 3;; j += gridDim.x >> 3) {
         const uint32_t i = xcd_item(blockIdx.x & 7u, j, n_items);
         if (i >= n_items) break;
         // An opaque copy: most waves take one item, so nothing is worth computing
         // ahead of the loop and holding in (spilled) registers.
-        uint32_t lane = threadIdx.x & 63u;
+        uint32_t lane = threadIdx.x;
         asm volatile("" : "+v"(lane));
         const uint32_t item = items[(size_t)i * ITEM_WORDS + (lane & 15u)];
         const uint32_t hid = __builtin_amdgcn_readlane(item, ITEM_HID);
@@ -2612,25 +2612,24 @@ static inline PBuf to_pbuf(const ParticleBuffers &b) {
     return p;
 }
 
-// Workgroups of a per-block kernel (a multiple of the XCDs): one block (per_wg
-// blocks) per workgroup up to the tuned persistent width; workgroups loop over the
+// Workgroups of a per-block kernel (a multiple of the XCDs): one block
+// per workgroup up to the tuned persistent width; workgroups loop over the
 // device-side block count. The count is not known here: dense scenes have a block per
 // 300 to 500 particles, so one per 256 leaves few workgroups without a block (an idle
 // one costs 0.2 ns of dispatch: 16384 of them 2.8 us), and 2048 fill the chip when
 // particles are sparse.
-static uint32_t block_grid(const StepParams &P, uint32_t per_wg) {
+static uint32_t block_grid(const StepParams &P) {
     const uint32_t likely = P.n / 256u > 2048u ? P.n / 256u : 2048u;
-    const uint32_t wgs = div_up_t(P.cap < likely ? P.cap : likely, per_wg);
-    return (min_t(wgs, P.block_wgs ? P.block_wgs : 8192u) + 7u) & ~7u;
+    return (min_t(P.cap < likely ? P.cap : likely, P.block_wgs) + 7u) & ~7u;
 }
 
-// Workgroups of `waves` items each (a multiple of the XCDs): every entry sequence is at
-// most its block's candidates and listed movers (together at most 2 n entries), in
-// 64s; dense scenes have an item per 55 particles.
-static uint32_t item_grid(const StepParams &P, uint32_t waves) {
-    const uint64_t likely = P.n / 48u > 4096u ? P.n / 48u : 4096u, most = max_items(P.n, P.cap);
-    const uint32_t wgs = div_up_t(likely < most ? likely : most, waves);
-    return (min_t(wgs, P.block_wgs ? P.block_wgs : 8192u) + 7u) & ~7u;
+// Workgroups of one item each (a multiple of the XCDs), looping beyond eight times the
+// persistent width: every entry sequence is at most its block's candidates and listed
+// movers (together at most 2 n entries), in 64s; dense scenes have an item per 55
+// particles, sparse ones (42k blocks of 50) one per 40.
+static uint32_t item_grid(const StepParams &P) {
+    const uint64_t likely = P.n / 32u > 4096u ? P.n / 32u : 4096u, most = max_items(P.n, P.cap);
+    return (min_t((uint32_t)(likely < most ? likely : most), 8u * P.block_wgs) + 7u) & ~7u;
 }
 
 static SortInputs sort_inputs(const TransferBuffers &t) {
@@ -2699,7 +2698,7 @@ hipError_t launch_p2g(const StepParams &P, const ParticleBuffers &pb, uint32_t p
                           : chunk == 256u ? k_p2g<256, false, 1>
                           : chunk == 384u ? k_p2g<384, false, 1>
                                           : k_p2g<512, false, 1>);
-    launch_kernel(ev, kern, dim3(block_grid(P, 1)), dim3(sub ? 384 : 192), 0, stream, P, (const float4 *)pb.pos,
+    launch_kernel(ev, kern, dim3(block_grid(P)), dim3(sub ? 384 : 192), 0, stream, P, (const float4 *)pb.pos,
                   (const float4 *)pb.vm, (const float *)pb.C, (const float *)t.fdt, pcap, members_of(t), sort_inputs(t),
                   t.keys, t.tiles, t.cell_cnt);
     return hipGetLastError();
@@ -2729,8 +2728,8 @@ hipError_t launch_grid_update(const StepParams &P, const TransferBuffers &t, con
     items.rshift = t.rshift;
     // Trimesh projection (a BVH walk) is compiled into its own instance so that
     // scenes without meshes keep the smaller kernel.
-    launch_kernel(ev, c.mesh_vtx ? k_grid_update<true> : k_grid_update<false>, dim3(block_grid(P, c.mesh_vtx ? 1 : 4)),
-                  dim3(c.mesh_vtx ? 64 * MESH_WAVES : 256), 0, stream, P,
+    launch_kernel(ev, c.mesh_vtx ? k_grid_update<true> : k_grid_update<false>, dim3(block_grid(P)),
+                  dim3(c.mesh_vtx ? 64 * MESH_WAVES : 64), 0, stream, P,
                   (const float4 *)t.tiles, t.nodes, t.nbr, t.keys, cs, (const NodeColl *)t.coll_prev,
                   (NodeColl *)t.coll_cur, members_of(t), items, next_table(next), mode, do_update);
     return hipGetLastError();
@@ -2768,17 +2767,15 @@ hipError_t launch_g2p_update(const StepParams &P, const ParticleBuffers &in, con
     auto kern = nh_only        ? k_g2p_update<2u, false>
                 : elastic_only ? (P.svd_f64 ? k_g2p_update<3u, true> : k_g2p_update<3u, false>)
                                : (P.svd_f64 ? k_g2p_update<15u, true> : k_g2p_update<15u, false>);
-    const uint32_t waves = P.g2p_threads == 128u ? 2u : 4u;
     // One more workgroup (the last) integrates the rigid bodies.
-    launch_kernel(ev, kern, dim3(item_grid(P, waves) + 1u), dim3(64u * waves),
-                  waves * TILE_NODES * (uint32_t)sizeof(float4), stream, args, members_of(t),
+    launch_kernel(ev, kern, dim3(item_grid(P) + 1u), dim3(64), 0, stream, args, members_of(t),
                   (const uint32_t *)t.items, (const float4 *)t.nodes);
     return hipGetLastError();
 }
 
 hipError_t launch_g2p(const StepParams &P, const ParticleBuffers &b, uint32_t pcap, const TransferBuffers &t,
                       const PassEvents *ev, hipStream_t stream) {
-    launch_kernel(ev, k_g2p, dim3(block_grid(P, 1)), dim3(256), 0, stream, P, to_pbuf(b), pcap, t.perm, t.blist,
+    launch_kernel(ev, k_g2p, dim3(block_grid(P)), dim3(256), 0, stream, P, to_pbuf(b), pcap, t.perm, t.blist,
                   (const uint32_t *)t.blk_start, (const uint32_t *)t.blk_cnt, t.nbr, (const float4 *)t.nodes,
                   t.counters);
     return hipGetLastError();

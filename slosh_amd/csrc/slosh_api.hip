@@ -989,7 +989,6 @@ static StepParams make_params(const slosh_data *d) {
                        ? 1u
                        : 0u;
     P.p2g_chunk = d->tuning.p2g_chunk;
-    P.g2p_threads = d->tuning.g2p_threads;
     P.block_wgs = d->tuning.block_wgs;
     P.u_prop = d->u_prop;
     P.u_model = d->u_model;
@@ -2762,9 +2761,8 @@ int slosh_autotune(slosh_pipeline *pl, slosh_data *d, slosh_stream stream, uint3
     float best_ms = 0.0f;
     int rc = run_step(pl, c, st, nullptr, nullptr, nullptr);
     if (rc == SLOSH_OK) rc = time_tuning(pl, c, st, best, steps, &best_ms);
-    // Coordinate search: P2G staging chunk, G2P workgroup size, persistent width.
+    // Coordinate search: P2G staging chunk, persistent width.
     const uint32_t chunks[] = {192u, 256u, 384u, 512u};
-    const uint32_t threads[] = {128u, 256u};
     const uint32_t widths[] = {2048u, 4096u, 8192u, 16384u, 32768u};
     auto consider = [&](slosh_tuning t) {
         if (rc != SLOSH_OK || std::memcmp(&t, &best, sizeof t) == 0) return;
@@ -2778,11 +2776,6 @@ int slosh_autotune(slosh_pipeline *pl, slosh_data *d, slosh_stream stream, uint3
     for (uint32_t v : chunks) {
         slosh_tuning t = best;
         t.p2g_chunk = v;
-        consider(t);
-    }
-    for (uint32_t v : threads) {
-        slosh_tuning t = best;
-        t.g2p_threads = v;
         consider(t);
     }
     for (uint32_t v : widths) {
