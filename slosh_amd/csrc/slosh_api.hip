@@ -710,13 +710,15 @@ static void stage_range(const slosh_particles *p, uint32_t id_base, S &s, size_t
 }
 
 // AoS reference records -> the internal SoA staging. The loop scatters each
-// particle into ~20 arrays (~40 ns per particle on one core), so large inputs
-// are split over up to 8 host threads; a range whose thread cannot be started
-// runs on the caller's.
-// Host threads for a pass over n particles (one below 2^17 particles).
-static size_t host_threads(size_t n) {
+// particle into ~20 arrays (~25 ns per particle on one core), so inputs are split
+// over up to 8 host threads; a range whose thread cannot be started runs on the
+// caller's.
+// Host threads for a pass over n particles at `each` per thread: 200 us of work, where
+// starting and joining a thread takes ~30 us.
+static constexpr size_t STAGE_EACH = 1 << 13, SCAN_EACH = 1 << 15;
+static size_t host_threads(size_t n, size_t each) {
     const size_t hw = std::max<size_t>(1, std::thread::hardware_concurrency() / 2);
-    return n < ((size_t)1 << 17) ? 1 : std::min<size_t>(std::min<size_t>(hw, 8), n >> 16);
+    return std::max<size_t>(1, std::min<size_t>(std::min<size_t>(hw, 8), n / each));
 }
 
 // One pass over an append's particles (in parallel for large ones): whether they
@@ -750,7 +752,7 @@ static AppendSummary summarize_range(const slosh_particles *p, size_t lo, size_t
 }
 
 static AppendSummary summarize(const slosh_particles *p) {
-    const size_t n = p->len, T = host_threads(n);
+    const size_t n = p->len, T = host_threads(n, SCAN_EACH);
     std::vector<AppendSummary> part(T);
     std::vector<std::thread> workers;
     for (size_t t = 1; t < T; t++) {
@@ -849,7 +851,7 @@ template <typename S>
 static int stage_particles(const slosh_particles *p, uint32_t id_base, S &s, bool *any_force, bool *any_sand) {
     const size_t n = p->len;
     s.resize(n);
-    const size_t T = host_threads(n);
+    const size_t T = host_threads(n, STAGE_EACH);
     std::vector<uint8_t> flags(3 * T, 0);
     std::vector<std::thread> workers;
     std::vector<size_t> inline_ranges;
@@ -1563,7 +1565,7 @@ static size_t first_out_of_range(const slosh_particles *p, size_t lo, size_t hi,
 }
 
 static int check_key_range(const slosh_particles *p, float h, uint32_t batched) {
-    const size_t n = p->len, T = host_threads(n);
+    const size_t n = p->len, T = host_threads(n, SCAN_EACH);
     std::vector<size_t> bad(T, n);
     std::vector<std::thread> workers;
     for (size_t t = 1; t < T; t++) {

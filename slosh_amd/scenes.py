@@ -209,13 +209,26 @@ def stir(scene, seed, rate=2.0):
     return scene
 
 
+def _column_extremes(a):
+    """Least and greatest value of each column. A reduction along rows of 3 or 4 values
+    costs numpy ~15 ns a row; 64 rows side by side make it a pass over memory."""
+    n, k = a.shape
+    whole = n - n % 64
+    parts = [a[whole:]] if whole < n else []
+    if whole:
+        wide = np.ascontiguousarray(a[:whole]).reshape(-1, 64 * k)
+        parts = [wide.min(axis=0).reshape(64, k), wide.max(axis=0).reshape(64, k)] + parts
+    return (np.min([p.min(axis=0) for p in parts], axis=0), np.max([p.max(axis=0) for p in parts], axis=0))
+
+
 def estimate_blocks(pos, cell_width):
     """Upper estimate of the active 4x4x4 blocks a particle cloud touches: its
     bounding box in blocks plus the +1 neighbour shell on every axis."""
     if len(pos) == 0:
         return 0
-    lo = np.floor(np.min(pos[:, :3], axis=0) / (4.0 * cell_width)) - 1
-    hi = np.floor(np.max(pos[:, :3], axis=0) / (4.0 * cell_width)) + 2
+    least, greatest = _column_extremes(np.asarray(pos))
+    lo = np.floor(least[:3] / (4.0 * cell_width)) - 1
+    hi = np.floor(greatest[:3] / (4.0 * cell_width)) + 2
     return int(np.prod(hi - lo + 1))
 
 
