@@ -697,7 +697,7 @@ struct Colliders {
     // The BVHs of the trimesh bodies as the walk reads them (see pack_meshes), and
     // each body's first node.
     const float4 *mesh_nodes, *mesh_leaves;
-    const uint32_t *mesh_base;
+    const uint32_t *mesh_base, *mesh_flat;
 };
 
 // triangle_project_local_point_and_get_location (trimesh.slang:304-377): closest
@@ -852,22 +852,26 @@ __device__ inline void trimesh_contact(const Colliders &cs, uint32_t i, uint32_t
 }
 
 // The closest triangles of a block's 64 nodes by a workgroup of MESH_WAVES waves,
-// for every trimesh collider: one wave collects the leaves near the block, a level of
-// the BVH at a time; then each wave tests its share of them for all nodes (lane =
-// node) and the closest wins by an LDS minimum over (distance, later leaf first),
-// the order the walk decides ties in.
+// for every trimesh collider: the leaves near the block are collected, of a small mesh
+// from all its nodes at once, else by one wave, a level of the BVH at a time; then each
+// wave tests its share of them for all nodes (lane = node), culled by the closest that
+// any wave has found, and the closest wins by an LDS minimum over (distance, later leaf
+// first), the order the walk decides ties in.
 //
 // Bound by latency: a block is 64 nodes with ~50 triangles in reach, and one triangle
 // test ~300 dependent instructions, so one wave per block left the chip idle. The
 // grid update of 85k particles over an 874-triangle heightfield (429 blocks): walked
-// per lane 110 us, walked by the wave together 114 us, shared by 8 waves 29 us (4 waves 37, 16 waves 48).
+// per lane 110 us, walked by the wave together 114 us, shared by 8 waves 28 us (4 waves
+// 37, 16 waves 48), with the leaves from all nodes at once 23 us, culled together 22 us.
+// The whole substep at finer heightfields (before: 512 leaves and 256 nodes of a level,
+// walked per lane beyond): 3690 triangles 287 -> 78 us, 7434 455 -> 106, 15834 770 -> 152.
 #define MESH_WAVES 8
-#define MESH_CAND 512  // leaves near a block that the workgroup shares; more are walked
-#define MESH_FRONT 256
+#define MESH_CAND 2048   // leaves near a block that the workgroup shares; more are walked
+#define MESH_FRONT 2048  // nodes of a level near a block
 struct MeshShared {
     uint32_t cand[MESH_CAND];
     uint32_t front[2][MESH_FRONT];
-    uint32_t n_cand;  // SLOSH_NONE: more than fit
+    uint32_t n_cand;  // above MESH_CAND: more than fit
     unsigned long long key[SLOSH_MAX_COLLIDERS][NODES_PER_BLOCK];  // all ones: none in reach
 };
 
@@ -913,6 +917,22 @@ __device__ inline void mesh_candidates(MeshShared &S, const float4 *__restrict__
         nf = next;
     }
     if (lane == 0) S.n_cand = fits ? n_cand : SLOSH_NONE;
+}
+
+// The same by the whole workgroup from all of a small mesh's nodes at once, without the
+// levels' chain of loads.
+__device__ inline void mesh_candidates_flat(MeshShared &S, const float4 *__restrict__ node, uint32_t count, float3 c,
+                                            float3 e, float reach) {
+    for (uint32_t k = threadIdx.x; k < count; k += 64u * MESH_WAVES) {
+        const float4 mn = node[2u * k], mx = node[2u * k + 1u];
+        const float gx = fmaxf(fmaxf(mn.x - (c.x + e.x), (c.x - e.x) - mx.x), 0.0f);
+        const float gy = fmaxf(fmaxf(mn.y - (c.y + e.y), (c.y - e.y) - mx.y), 0.0f);
+        const float gz = fmaxf(fmaxf(mn.z - (c.z + e.z), (c.z - e.z) - mx.z), 0.0f);
+        if (__float_as_uint(mn.w) == SLOSH_NONE && gx * gx + gy * gy + gz * gz <= reach * reach) {
+            const uint32_t at = atomicAdd(&S.n_cand, 1u);
+            if (at < MESH_CAND) S.cand[at] = k;
+        }
+    }
 }
 
 struct NodeColl {
@@ -1760,10 +1780,15 @@ __device__ inline void mesh_queries(const Colliders &cs, const float4 *box, Mesh
         if (wave == 0u) S.key[i][lane] = ~0ull;
         if (__ballot(on) == 0ull) continue;  // (every wave holds the same nodes)
         const float4 rot = cs.poses[2 * i], ts = cs.poses[2 * i + 1];
-        const uint32_t base = cs.mesh_base[i];
+        const uint32_t base = cs.mesh_base[i], count = __float_as_uint(a.z);
+        const bool flat = cs.mesh_flat[i] != 0u;
         const float4 *node = cs.mesh_nodes + 2u * (size_t)base, *leaf = cs.mesh_leaves + 3u * (size_t)base;
         const float3 pt = sim_inv_mul_pt(rot, ts, cell_pos);
-        if (wave == 0u) {
+        if (flat) {
+            if (threadIdx.x == 0u) S.n_cand = 0u;
+            __syncthreads();
+        }
+        if (flat || wave == 0u) {
             // The block's box in the mesh's frame, from its first node.
             const float3 w0 = make_float3(__shfl(cell_pos.x, 0), __shfl(cell_pos.y, 0), __shfl(cell_pos.z, 0));
             const float3 c = sim_inv_mul_pt(rot, ts, make_float3(w0.x + cap, w0.y + cap, w0.z + cap));
@@ -1776,34 +1801,32 @@ __device__ inline void mesh_queries(const Colliders &cs, const float4 *box, Mesh
                                          (fabsf(ix.y) + fabsf(iy.y) + fabsf(iz.y)) * s,
                                          (fabsf(ix.z) + fabsf(iy.z) + fabsf(iz.z)) * s);
             const float size = fmaxf(fmaxf(fabsf(c.x), fabsf(c.y)), fabsf(c.z));
-            mesh_candidates(S, node, c, e, 1.001f * cap + 1.0e-5f * size);
+            const float reach = 1.001f * cap + 1.0e-5f * size;
+            if (flat) mesh_candidates_flat(S, node, count, c, e, reach);
+            else mesh_candidates(S, node, c, e, reach);
         }
         __syncthreads();
         const uint32_t n = S.n_cand;
-        if (n == SLOSH_NONE) {
+        if (n > MESH_CAND) {
             if (wave == 0u && on) {
-                const uint32_t lf = trimesh_walk(node, leaf, __float_as_uint(a.z), pt, cap);
+                const uint32_t lf = trimesh_walk(node, leaf, count, pt, cap);
                 if (lf != SLOSH_NONE) S.key[i][lane] = (unsigned long long)~lf;
             }
         } else {
-            float best = cap;
-            unsigned long long key = ((unsigned long long)__float_as_uint(cap) << 32) | 0xffffffffull;
-            bool found = false;
+            // Every wave culls by the closest any of them has found so far.
+            volatile unsigned long long *closest = &S.key[i][lane];
             for (uint32_t q = wave; q < n; q += MESH_WAVES) {
                 const uint32_t lf = __builtin_amdgcn_readfirstlane(S.cand[q]);
+                const unsigned long long key = *closest;
+                const float best = key == ~0ull ? cap : __uint_as_float((uint32_t)(key >> 32));
                 if (on && box_distance(node[2u * lf], node[2u * lf + 1u], pt) <= best) {
                     float3 p;
                     uint32_t tri, feat, id;
                     const float dist = leaf_distance(leaf + 3u * (size_t)lf, pt, &p, &tri, &feat, &id);
                     const unsigned long long k = ((unsigned long long)__float_as_uint(dist) << 32) | (uint32_t)~lf;
-                    if (dist <= best && k < key) {
-                        best = dist;
-                        key = k;
-                        found = true;
-                    }
+                    if (dist <= best && k < key) atomicMin(&S.key[i][lane], k);
                 }
             }
-            if (found) atomicMin(&S.key[i][lane], key);
         }
         __syncthreads();
     }
@@ -2717,6 +2740,7 @@ hipError_t launch_grid_update(const StepParams &P, const TransferBuffers &t, con
     cs.mesh_nodes = c.mesh_nodes;
     cs.mesh_leaves = c.mesh_leaves;
     cs.mesh_base = c.mesh_base;
+    cs.mesh_flat = c.mesh_base ? c.mesh_base + SLOSH_MAX_COLLIDERS : nullptr;
     ItemLists items;
     items.items = t.items;
     items.rsum = t.rsum;

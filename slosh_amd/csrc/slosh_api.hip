@@ -1893,14 +1893,46 @@ void slosh_graph_destroy(slosh_graph *g) {
 // and for a leaf its triangle's vertices with the triangle index. A leaf's box is that
 // of its triangle (the reference never reads a leaf's own), grown by 1 % of its extent
 // and well above the rounding of its coordinates.
+// Whether a walk of the BVH visits every leaf whose triangle is near: each node's box
+// holds the triangles of the leaves below it, and every leaf is below the first node. Then
+// the leaves of a small mesh are tested directly.
+static bool walk_reaches_all(const float *vertices4, const uint32_t *indices, size_t vroot, size_t iroot,
+                             size_t count) {
+    size_t leaves = 0, reached = 0;
+    std::vector<size_t> open;  // nodes above the current one
+    for (size_t k = 0; k < count; k++) leaves += indices[iroot + 3 * k] == 0xffffffffu;
+    for (size_t k = 0; k < count;) {
+        const uint32_t *nd = indices + iroot + 3 * k;
+        while (!open.empty() && indices[iroot + 3 * open.back() + 1] <= k) open.pop_back();
+        if (nd[0] != 0xffffffffu) {
+            open.push_back(k);
+            k = nd[0];
+            continue;
+        }
+        reached++;
+        const uint32_t *t = indices + iroot + 3 * count + 3 * nd[2];
+        for (size_t up : open) {
+            const float *mn = vertices4 + 4 * (vroot + 2 * up), *mx = mn + 4;
+            for (int j = 0; j < 3; j++)
+                for (int c = 0; c < 3; c++) {
+                    const float x = vertices4[4 * (vroot + 2 * count + t[j]) + c];
+                    if (!(x >= mn[c] && x <= mx[c])) return false;
+                }
+        }
+        k = nd[1];
+    }
+    return reached == leaves;
+}
+
 static int pack_meshes(slosh_data *d, const float *vertices4, const uint32_t *indices) {
     std::vector<float4> nodes, leaves;
-    std::vector<uint32_t> base(SLOSH_MAX_COLLIDERS, 0u);
+    std::vector<uint32_t> base(2 * SLOSH_MAX_COLLIDERS, 0u);
     for (uint32_t b = 0; b < d->nbodies; b++) {
         const slosh_shape &sh = d->bodies_host[b].shape;
         if (f2u(sh.a[3]) != 6u) continue;
         const size_t vroot = f2u(sh.a[0]), iroot = f2u(sh.a[1]), count = f2u(sh.a[2]);
         base[b] = (uint32_t)(nodes.size() / 2);
+        base[SLOSH_MAX_COLLIDERS + b] = count <= MESH_FLAT && walk_reaches_all(vertices4, indices, vroot, iroot, count);
         for (size_t k = 0; k < count; k++) {
             const uint32_t *nd = indices + iroot + 3 * k;
             const float *mn = vertices4 + 4 * (vroot + 2 * k), *mx = mn + 4;
