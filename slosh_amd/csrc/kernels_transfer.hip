@@ -1722,7 +1722,7 @@ __global__ __launch_bounds__(192 * SUB, SUB == 1 && P2G_CHUNK <= 384 ? 4 : 1) vo
         __syncthreads();  // the staging's readers are done
         float4 *slab = S.slab[wave];
         for (uint32_t j = lane; j < P2G_SLAB_LDS; j += 64) slab[j] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-        __asm__ volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __asm__ volatile("" ::: "memory");
 #pragma unroll
         for (int ky = 0; ky < 3; ky++)
 #pragma unroll
@@ -1735,9 +1735,10 @@ __global__ __launch_bounds__(192 * SUB, SUB == 1 && P2G_CHUNK <= 384 ? 4 : 1) vo
                 t.z += acc[q][2];
                 t.w += acc[q][3];
                 slab[node] = t;
-                // The next round's nodes overlap other lanes' nodes of this
-                // round: complete this round's LDS writes first.
-                __asm__ volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+                // The next round's nodes overlap other lanes' nodes of this round: its
+                // reads come after this round's writes (a wave's LDS operations are
+                // carried out in their order).
+                __asm__ volatile("" ::: "memory");
             }
         __syncthreads();
         for (uint32_t j = threadIdx.x; j < TILE_NODES; j += T) {
