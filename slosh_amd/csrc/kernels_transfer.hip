@@ -2199,6 +2199,11 @@ __global__ __launch_bounds__(64, F64 && MODELS != 3u ? 3 : 4) void k_g2p_update(
                                                     const uint32_t *__restrict__ items,
                                                     const float4 *__restrict__ nodes) {
     __shared__ float4 sh[TILE_NODES];
+    // The FP64 corotated instance fits four waves per SIMD (128 VGPRs) without scratch
+    // memory, whose set-up alone costs more than the fourth wave gains, if it recomputes and
+    // stashes more (1.2M corotated particles 119.3 -> 114.3 us a substep; the neo-Hookean
+    // instance lost 2 us of 92 at 1M by the same).
+    constexpr bool TIGHT = F64 && MODELS == 3u;
     // integrate_bodies: reads no particle or grid state (the impulses it applies
     // are only written by the host), so the last workgroup runs it alongside the
     // particle update.
@@ -2210,11 +2215,12 @@ __global__ __launch_bounds__(64, F64 && MODELS != 3u ? 3 : 4) void k_g2p_update(
     for (uint32_t j = blockIdx.x >> 3;; j += gridDim.x >> 3) {
         const uint32_t i = xcd_item(blockIdx.x & 7u, j, n_items);
         if (i >= n_items) break;
-        // An opaque copy: most waves take one item, so nothing is worth computing
-        // ahead of the loop and holding in (spilled) registers.
-        uint32_t lane = threadIdx.x;
-        asm volatile("" : "+v"(lane));
-        const uint32_t item = items[(size_t)i * ITEM_WORDS + (lane & 15u)];
+        // Opaque copies of the lane, for the item and for each round over its entries:
+        // nearly every wave goes round once, so little is worth computing ahead of the
+        // loops and holding in registers (the halo's addresses alone took 15).
+        uint32_t lane1 = threadIdx.x;
+        asm volatile("" : "+v"(lane1));
+        const uint32_t item = items[(size_t)i * ITEM_WORDS + (lane1 & 15u)];
         const uint32_t hid = __builtin_amdgcn_readlane(item, ITEM_HID);
         const uint32_t first = __builtin_amdgcn_readlane(item, ITEM_FIRST);
         const uint32_t s0 = __builtin_amdgcn_readlane(item, ITEM_START);
@@ -2237,8 +2243,9 @@ __global__ __launch_bounds__(64, F64 && MODELS != 3u ? 3 : 4) void k_g2p_update(
             first == 0u && __builtin_amdgcn_readlane(item, ITEM_OVERFLOW) ? M.counters[CTR_OVERFLOW] : 0u;
         for (uint32_t o = 0; o < 64u + n_ovf; o += 64u) {
             const G2pArgs &A = late_args<G2pArgs>();
-            uint32_t l = lane;  // (opaque again: else the halo's addresses take 15 VGPRs throughout)
-            asm volatile("" : "+v"(l));
+            uint32_t lane2 = TIGHT ? threadIdx.x : lane1;
+            asm volatile("" : "+v"(lane2));
+            const uint32_t lane = TIGHT ? lane2 : lane1;
             bool entry;
             uint32_t p = 0u;
             if (o == 0u) {
@@ -2265,7 +2272,7 @@ __global__ __launch_bounds__(64, F64 && MODELS != 3u ? 3 : 4) void k_g2p_update(
                     oid = A.in.ids[p];
                 }
             }
-            load_halo_wave(sh, nodes, item, l);  // (the last iteration may have reused the tile)
+            load_halo_wave(sh, nodes, item, lane2);  // (the last iteration may have reused the tile)
             const uint32_t wbits = __float_as_uint(ps.w);
             const uint32_t scene = wbits >> 1;
             const Stencil at = stencil_of(A.P.h, ps.x, ps.y, ps.z);
@@ -2328,9 +2335,16 @@ __global__ __launch_bounds__(64, F64 && MODELS != 3u ? 3 : 4) void k_g2p_update(
                 // The FP64 steps need the registers: the velocity gradient waits in
                 // the wave's LDS tile, which the sums above no longer need.
                 float *keep = reinterpret_cast<float *>(sh) + lane;
+                float left_mass = mass, volume = prop.x;
                 if (F64) {
 #pragma unroll
                     for (int q = 0; q < 9; q++) keep[64 * q] = aff[q];
+                }
+                if (TIGHT) {
+                    keep[64 * 9] = mass;
+                    keep[64 * 10] = prop.x;
+                    keep[64 * 11] = __uint_as_float(next_key);
+                    keep[64 * 12] = __uint_as_float(p);
                 }
                 // Only Drucker-Prager particles read or write their plastic state
                 // (the other particles' state slots are never read).
@@ -2347,18 +2361,25 @@ __global__ __launch_bounds__(64, F64 && MODELS != 3u ? 3 : 4) void k_g2p_update(
                     for (int q = 0; q < 3; q++) out.dps[(size_t)q * pcap + slot] = dps[q];
                 }
                 ok = ok && det3(F) > 0.0f;
+                uint32_t from = p;
                 if (F64) {
 #pragma unroll
                     for (int q = 0; q < 9; q++) aff[q] = keep[64 * q];
                 }
-                finish_particle(P, ok, mass, prop.x, stress, aff, F);
+                if (TIGHT) {
+                    left_mass = keep[64 * 9];
+                    volume = keep[64 * 10];
+                    next_key = __float_as_uint(keep[64 * 11]);
+                    from = __float_as_uint(keep[64 * 12]);
+                }
+                finish_particle(P, ok, left_mass, volume, stress, aff, F);
 #pragma unroll
                 for (int q = 0; q < 9; q++) {
                     out.C[(size_t)q * pcap + slot] = aff[q];
                     out.F[(size_t)q * pcap + slot] = F[q];
                 }
                 if (!ok) {
-                    const float4 old = in.pos[p];
+                    const float4 old = in.pos[from];
                     out.pos[slot] = make_float4(old.x, old.y, old.z, __uint_as_float(wbits & ~1u));
                     out.vm[slot] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
                     next_key = block_key;
