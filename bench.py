@@ -73,9 +73,9 @@ def measured_traffic(workload, pass_name, tuning):
     path = os.path.join(ROOT, "profiles", files[workload])
     if not os.path.exists(path):
         return None
-    g2p = "k_g2p_update<2u,%d,false,true>" if workload == "dam_break" else "k_g2p_update<15u,%d,true,true>"
-    kernel = {"g2p": g2p % tuning["g2p_threads"], "p2g": "k_p2g<%d,true>" % tuning["p2g_chunk"],
-              "grid_update": "k_grid_update<false>"}.get(pass_name)
+    g2p = "k_g2p_update<2u,false>" if workload == "dam_break" else "k_g2p_update<15u,true>"
+    chunk = 384 if tuning["p2g_chunk"] == 512 else tuning["p2g_chunk"]  # (512: by size; both are large)
+    kernel = {"g2p": g2p, "p2g": "k_p2g<%d,true,1>" % chunk, "grid_update": "k_grid_update<false>"}.get(pass_name)
     for ln in open(path):
         f = ln.split()
         if len(f) == 4 and f[0] == "traffic" and f[1] == pass_name and f[2] == kernel:
