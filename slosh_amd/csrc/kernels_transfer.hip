@@ -30,6 +30,15 @@ namespace {
 constexpr int ASSOC[8][3] = {{0, 0, 0}, {0, 0, 1}, {0, 1, 0}, {0, 1, 1},
                              {1, 0, 0}, {1, 0, 1}, {1, 1, 0}, {1, 1, 1}};
 
+// A new, opaque address of the kernel's argument block: what is read through it is loaded
+// after that point, instead of held in scalar registers (and spilled) from the start.
+template <typename T>
+__device__ inline const T &late_args() {
+    auto p = (const __attribute__((address_space(4))) char *)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(p));
+    return *(const T *)p;
+}
+
 // ---------------------------------------------------------------------------
 // Quadratic B-spline (kernel.slang:160-174).
 
@@ -1608,9 +1617,9 @@ __device__ inline void finish_block(const StepParams &P, const SortInputs &in, c
 // the steady state it starts from the regional lists and the ranges the previous substep
 // left. A block takes ~6 us from its first dependent load (list entry, range, member
 // slots, particles) to its tile, so what counts with many blocks is how many are
-// resident: 512 members per chunk hold four workgroups to a CU (35 KB of LDS, 135 VGPRs),
-// 384 let in five (113 VGPRs): 1M particles 43 -> 39 us, 48 scenes 101 -> 88, 2.1M in 42k
-// blocks 248 -> 206. Chunks of 256 or 192 take no fewer registers than that and more
+// resident: 512 members per chunk hold four workgroups to a CU (35 KB of LDS, 128 VGPRs),
+// 384 let in five (106 VGPRs): 1M particles 43 -> 39 us, 48 scenes 101 -> 88, 2.1M in 42k
+// blocks 248 -> 206 (38.2, 84.5 and 201 by now; more waves per SIMD at 96 VGPRs gain nothing). Chunks of 256 or 192 take no fewer registers than that and more
 // rounds (2.1M: 204, 209; 1M: 42, 44).
 // While all blocks are resident at once, the longest one's latency counts instead: a
 // block of 512 then goes in one chunk (131k particles: 14.2 us against 15.3), and with a
@@ -1621,29 +1630,44 @@ __device__ inline void finish_block(const StepParams &P, const SortInputs &in, c
 #define P2G_SUB_N 98304u    // two sets of waves up to here
 #define P2G_WIDE_N 262144u  // chunks of 512 up to here
 
+// (read through late_args: 14 to 26 scalar registers spilled otherwise; 48 scenes 87 -> 84.5
+// us, 2.1M 206 -> 201)
+struct P2gArgs {
+    StepParams P;
+    const float4 *pos, *vm;
+    const float *C, *fdt;
+    uint32_t pcap;
+    Members M;
+    SortInputs in;
+    const uint32_t *keys;
+    float4 *tiles;
+    uint32_t *cell_cnt;
+};
+
 template <int P2G_CHUNK, bool FAST, int SUB>
-__global__ __launch_bounds__(192 * SUB, SUB == 1 && P2G_CHUNK <= 384 ? 4 : 1) void k_p2g(StepParams P, const float4 *__restrict__ pos,
-                                             const float4 *__restrict__ vm, const float *__restrict__ C,
-                                             const float *__restrict__ fdt, uint32_t pcap, Members M, SortInputs in,
-                                             const uint32_t *__restrict__ keys, float4 *__restrict__ tiles,
-                                             uint32_t *__restrict__ cell_cnt) {
+__global__ __launch_bounds__(192 * SUB, SUB == 1 && P2G_CHUNK <= 384 ? 4 : 1) void k_p2g(P2gArgs args) {
     __shared__ P2GShared<P2G_CHUNK, SUB> S;
     constexpr uint32_t T = 192 * SUB;
-    const uint32_t n_ovf = M.counters[CTR_OVERFLOW];
+    const uint32_t n_ovf = args.M.counters[CTR_OVERFLOW];
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63u;
     const int lx = lane & 3, ly = (lane >> 2) & 3, lz = lane >> 4;
     uint32_t B, upto = 0u;  // blocks; FAST: those of the regions up to the lane's
     if constexpr (FAST) {
-        upto = wave_inclusive_scan(in.rcnt[lane * RCNT_STRIDE]);
+        upto = wave_inclusive_scan(args.in.rcnt[lane * RCNT_STRIDE]);
         B = __builtin_amdgcn_readlane(upto, 63);
-        if (blockIdx.x == 0u && threadIdx.x == 0u) *in.num_blocks = B;
+        if (blockIdx.x == 0u && threadIdx.x == 0u) *args.in.num_blocks = B;
     } else {
-        B = M.counters[CTR_NUM_BLOCKS];
+        B = args.M.counters[CTR_NUM_BLOCKS];
     }
     if (threadIdx.x < 64) S.lcnt[threadIdx.x] = 0u;
     for (uint32_t j = blockIdx.x >> 3;; j += gridDim.x >> 3) {
         const uint32_t k = xcd_item(blockIdx.x & 7u, j, B);
         if (k >= B) break;
+        const P2gArgs &A = late_args<P2gArgs>();
+        const StepParams &P = A.P;
+        const Members &M = A.M;
+        const SortInputs &in = A.in;
+        const uint32_t *keys = A.keys;
         uint32_t hid, block_key;
         BlockRange br;
         uint4 range;
@@ -1676,7 +1700,7 @@ __global__ __launch_bounds__(192 * SUB, SUB == 1 && P2G_CHUNK <= 384 ? 4 : 1) vo
         const uint32_t n_main = br.cand_n + br.list_n;
         if (n_main == 0u) {
             if (wave == 0u) {
-                cell_cnt[(size_t)hid * NODES_PER_BLOCK + lane] = 0u;
+                A.cell_cnt[(size_t)hid * NODES_PER_BLOCK + lane] = 0u;
                 if constexpr (FAST) finish_block(P, in, keys, hid, block_key, lane, range, br.total, seen);
             }
             continue;
@@ -1687,8 +1711,8 @@ __global__ __launch_bounds__(192 * SUB, SUB == 1 && P2G_CHUNK <= 384 ? 4 : 1) vo
         uint32_t tot = 0u;
         for (uint32_t chunk = 0; chunk < n_main; chunk += P2G_CHUNK) {
             const uint32_t kn = n_main - chunk < (uint32_t)P2G_CHUNK ? n_main - chunk : (uint32_t)P2G_CHUNK;
-            p2g_chunk<P2G_CHUNK, SUB>(P, S, kn, [&](uint32_t t) { return entry_slot(br, chunk + t); }, pos, vm, C, fdt,
-                                 pcap, block_key, acc, tot);
+            p2g_chunk<P2G_CHUNK, SUB>(P, S, kn, [&](uint32_t t) { return entry_slot(br, chunk + t); }, A.pos, A.vm,
+                                      A.C, A.fdt, A.pcap, block_key, acc, tot);
         }
         if (br.overflow) {
             // This block's movers beyond its list: picked out of the overflow list,
@@ -1708,14 +1732,15 @@ __global__ __launch_bounds__(192 * SUB, SUB == 1 && P2G_CHUNK <= 384 ? 4 : 1) vo
                 }
                 if (mine) S.extra[before + (uint32_t)__popcll(mm & lanemask_lt())] = M.ovf_slot[i];
                 if (kn > 0)
-                    p2g_chunk<P2G_CHUNK, SUB>(P, S, kn, [&](uint32_t t) { return S.extra[t]; }, pos, vm, C, fdt, pcap,
-                                         block_key, acc, tot);
+                    p2g_chunk<P2G_CHUNK, SUB>(P, S, kn, [&](uint32_t t) { return S.extra[t]; }, A.pos, A.vm, A.C, A.fdt,
+                                              A.pcap, block_key, acc, tot);
             }
         }
+        const P2gArgs &E = late_args<P2gArgs>();
         // The block's place in its region's storage and items (stored below).
         unsigned long long rel = 0ull;
         if (threadIdx.x == 0u)
-            rel = atomicAdd(&in.rsum[(hid >> in.rshift) * RSUM_STRIDE], ((unsigned long long)br.total << 32) | item_count(br));
+            rel = atomicAdd(&E.in.rsum[(hid >> E.in.rshift) * RSUM_STRIDE], ((unsigned long long)br.total << 32) | item_count(br));
         // Each wave adds its registers into its own slab tile (sharing the staging's
         // LDS), in 9 rounds in which its 64 lanes touch 64 distinct nodes; then each
         // node is the sum of the slabs that cover it, in wave order.
@@ -1735,9 +1760,9 @@ __global__ __launch_bounds__(192 * SUB, SUB == 1 && P2G_CHUNK <= 384 ? 4 : 1) vo
                 t.z += acc[q][2];
                 t.w += acc[q][3];
                 slab[node] = t;
-                // The next round's nodes overlap other lanes' nodes of this round: its
-                // reads come after this round's writes (a wave's LDS operations are
-                // carried out in their order).
+                // The next step's nodes overlap other lanes' nodes of this one: its reads
+                // come after these writes (a wave's LDS operations are carried out in
+                // their order).
                 __asm__ volatile("" ::: "memory");
             }
         __syncthreads();
@@ -1756,12 +1781,12 @@ __global__ __launch_bounds__(192 * SUB, SUB == 1 && P2G_CHUNK <= 384 ? 4 : 1) vo
                     t.w += u.w;
                 }
             }
-            tiles[(size_t)hid * TILE_NODES + tile_index(x, y, z)] = t;
+            E.tiles[(size_t)hid * TILE_NODES + tile_index(x, y, z)] = t;
         }
-        if (wave == 0u) cell_cnt[(size_t)hid * NODES_PER_BLOCK + lane] = tot;
-        if (threadIdx.x == 0u) in.rel[hid] = make_uint2((uint32_t)(rel >> 32), (uint32_t)rel);
+        if (wave == 0u) E.cell_cnt[(size_t)hid * NODES_PER_BLOCK + lane] = tot;
+        if (threadIdx.x == 0u) E.in.rel[hid] = make_uint2((uint32_t)(rel >> 32), (uint32_t)rel);
         if constexpr (FAST)
-            if (wave == 0u) finish_block(P, in, keys, hid, block_key, lane, range, br.total, seen);
+            if (wave == 0u) finish_block(E.P, E.in, E.keys, hid, block_key, lane, range, br.total, seen);
     }
 }
 
@@ -2173,9 +2198,9 @@ struct NextSort {
 // The arguments, read where they are used: held in scalar registers from the start
 // 118 of them spilled to VGPR lanes. late_args() gives the compiler a new, opaque address
 // of the kernel's argument block, so that what is read through it is loaded after that
-// point: the neo-Hookean instance needs 93 instead of 108 VGPRs (five waves per SIMD
-// instead of four; 1M particles 53.0 -> 48.6 us), the FP32 one of every material 128
-// instead of 145 (four instead of three).
+// point: the neo-Hookean instance went from 108 to 93 VGPRs (now 77: six waves per SIMD
+// instead of four; 1M particles 53.0 -> 48.6 us), the FP32 one of every material from 145
+// to 128 (now 99).
 struct G2pArgs {
     StepParams P;
     PBuf in, out;
@@ -2186,13 +2211,6 @@ struct G2pArgs {
     NextSort ns;
     Bodies bodies;
 };
-
-template <typename T>
-__device__ inline const T &late_args() {
-    auto p = (const __attribute__((address_space(4))) char *)__builtin_amdgcn_kernarg_segment_ptr();
-    asm volatile("" : "+s"(p));
-    return *(const T *)p;
-}
 
 template <uint32_t MODELS, bool F64>
 __global__ __launch_bounds__(64, F64 && MODELS != 3u ? 3 : 4) void k_g2p_update(G2pArgs args, Members M,
@@ -2743,9 +2761,19 @@ hipError_t launch_p2g(const StepParams &P, const ParticleBuffers &pb, uint32_t p
                           : chunk == 256u ? k_p2g<256, false, 1>
                           : chunk == 384u ? k_p2g<384, false, 1>
                                           : k_p2g<512, false, 1>);
-    launch_kernel(ev, kern, dim3(block_grid(P)), dim3(sub ? 384 : 192), 0, stream, P, (const float4 *)pb.pos,
-                  (const float4 *)pb.vm, (const float *)pb.C, (const float *)t.fdt, pcap, members_of(t), sort_inputs(t),
-                  t.keys, t.tiles, t.cell_cnt);
+    P2gArgs args;
+    args.P = P;
+    args.pos = pb.pos;
+    args.vm = pb.vm;
+    args.C = pb.C;
+    args.fdt = t.fdt;
+    args.pcap = pcap;
+    args.M = members_of(t);
+    args.in = sort_inputs(t);
+    args.keys = t.keys;
+    args.tiles = t.tiles;
+    args.cell_cnt = t.cell_cnt;
+    launch_kernel(ev, kern, dim3(block_grid(P)), dim3(sub ? 384 : 192), 0, stream, args);
     return hipGetLastError();
 }
 
