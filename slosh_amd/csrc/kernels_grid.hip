@@ -64,6 +64,7 @@ __global__ __launch_bounds__(256) void k_reset_table(uint32_t *__restrict__ keys
         counters[CTR_NUM_BLOCKS] = 0u;
         counters[CTR_SORTED_ALLOC] = 0u;
         counters[CTR_OVERFLOW] = 0u;
+        counters[CTR_ITEMS] = 0u;
     }
     if (blockIdx.x == 0 && threadIdx.x < REGIONS) rsum[threadIdx.x * RSUM_STRIDE] = 0ull;
 }

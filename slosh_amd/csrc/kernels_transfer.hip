@@ -1899,7 +1899,7 @@ __device__ inline void reset_next_table(const NextTable &nt, uint32_t cap) {
 }
 
 // mode 0: node momentum from tiles; mode 1: nodes already hold momentum (P2G hook).
-// do_update 0: only combine tiles (grid update disabled).
+// do_update 0: only combine tiles (grid update disabled; nothing to do to the nodes in mode 1).
 template <bool MESH>
 __global__ __launch_bounds__(MESH ? 64 * MESH_WAVES : 64) void k_grid_update(StepParams P, const float4 *__restrict__ tiles,
                                                      float4 *__restrict__ nodes, const uint32_t *__restrict__ nbr,
@@ -1917,7 +1917,7 @@ __global__ __launch_bounds__(MESH ? 64 * MESH_WAVES : 64) void k_grid_update(Ste
     // Storage and items before the lane's region.
     const unsigned long long rs = L.rsum[lane * RSUM_STRIDE];
     const uint32_t up_p = wave_inclusive_scan((uint32_t)(rs >> 32)), up_i = wave_inclusive_scan((uint32_t)rs);
-    if (blockIdx.x == 0u && threadIdx.x == 0u) *L.n_items = __builtin_amdgcn_readlane(up_i, 63);
+    if (mode == 0 && blockIdx.x == 0u && threadIdx.x == 0u) *L.n_items = __builtin_amdgcn_readlane(up_i, 63);
     // With trimesh colliders a workgroup shares one block: every wave holds its nodes
     // (and takes part in mesh_queries), the first one writes them.
     __shared__ typename std::conditional<MESH, MeshShared, char>::type shared;
@@ -1931,14 +1931,23 @@ __global__ __launch_bounds__(MESH ? 64 * MESH_WAVES : 64) void k_grid_update(Ste
         // The neighbour table (lane l: entry l, see NBR_STRIDE).
         const uint32_t nb = lane < NBR_STRIDE ? nbr[(size_t)hid * NBR_STRIDE + lane] : SLOSH_NONE;
         const uint32_t prev = __builtin_amdgcn_readlane(nb, NBR_PREV);
-        if (mode == 0 && owner) {
+        if (owner) {
             const BlockRange br = M.fast ? block_range<true>(M, hid) : block_range<false>(M, hid);
             const uint32_t n = item_count(br), r = hid >> L.rshift;
             if (n) {
-                const uint2 rel = L.rel[hid];
-                const uint32_t item0 = rel.y + (r ? __builtin_amdgcn_readlane(up_i, r - 1u) : 0u);
-                const uint32_t start =
-                    M.fast ? rel.x + (r ? __builtin_amdgcn_readlane(up_p, r - 1u) : 0u) : M.blk_start[hid];
+                uint32_t item0, start;
+                if (mode == 0) {
+                    const uint2 rel = L.rel[hid];
+                    item0 = rel.y + (r ? __builtin_amdgcn_readlane(up_i, r - 1u) : 0u);
+                    start = M.fast ? rel.x + (r ? __builtin_amdgcn_readlane(up_p, r - 1u) : 0u) : M.blk_start[hid];
+                } else {
+                    // A hook did P2G after a full sort: the items in order of arrival (their
+                    // count was cleared by the sort).
+                    uint32_t at = 0u;
+                    if (lane == 0u) at = atomicAdd(L.n_items, n);
+                    item0 = __builtin_amdgcn_readfirstlane(at);
+                    start = M.blk_start[hid];
+                }
                 if (M.fast && lane == 0u) L.blk_start[hid] = start;
                 // Four items at a time, a word per lane.
                 const uint32_t w = lane & 15u;
@@ -2003,6 +2012,7 @@ __global__ __launch_bounds__(MESH ? 64 * MESH_WAVES : 64) void k_grid_update(Ste
                 }
             }
         } else {
+            if (!do_update) continue;
             acc = nodes[(size_t)hid * NODES_PER_BLOCK + lane];
         }
         if (MESH) __syncthreads();  // every wave has read the nodes (mode 1) and is done with the last block

@@ -1177,11 +1177,10 @@ static int run_step(slosh_pipeline *pl, slosh_data *d, hipStream_t st, const slo
     cb.mesh_nodes = d->mesh_nodes;
     cb.mesh_leaves = d->mesh_leaves;
     cb.mesh_base = d->mesh_base;
-    if (K.grid_update || !p2g_by_hook) {
-        const uint32_t mode = p2g_by_hook ? 1u : 0u;
-        HIP_TRY(launch_grid_update(P, t, cb, next, mode, K.grid_update ? 1u : 0u,
-                                   pass_events(ts, PASS_GRID_UPDATE, &pe), st));
-    }
+    // (The launch prepares the fused G2P kernel's items as well, whoever does the rest.)
+    const bool combine = K.grid_update || !p2g_by_hook;
+    HIP_TRY(launch_grid_update(P, t, cb, next, p2g_by_hook ? 1u : 0u, K.grid_update ? 1u : 0u,
+                               combine ? pass_events(ts, PASS_GRID_UPDATE, &pe) : nullptr, st));
     if (d->coll_cache) d->coll_prev_valid = 1;
     if (hooks && hooks->after_grid_update && hooks->after_grid_update(d, st, hs) != 0)
         return fail(SLOSH_E_HOOK, "after_grid_update hook failed");
@@ -1197,8 +1196,7 @@ static int run_step(slosh_pipeline *pl, slosh_data *d, hipStream_t st, const slo
     if (hooks && hooks->run_g2p && hooks->run_g2p(d, st, hs, &handled) != 0)
         return fail(SLOSH_E_HOOK, "run_g2p hook failed");
     const bool g2p_by_hook = handled != 0;
-    // (A P2G hook leaves the fused kernel's item starts unwritten.)
-    const bool split = g2p_by_hook || p2g_by_hook || (hooks && hooks->after_g2p) || !K.particles_update;
+    const bool split = g2p_by_hook || (hooks && hooks->after_g2p) || !K.particles_update;
     if (!g2p_by_hook && !K.builtin_transfers)
         return fail(SLOSH_E_NO_KERNELS, "pipeline built without builtin transfer kernels; a hook must handle run_g2p");
     if (!split) {
