@@ -268,8 +268,9 @@ __device__ inline void dp_project(float *state, const float4 hp, float lambda, f
 // Refined variants of the SVD-dependent steps. In FP32, F - R and log(sigma)
 // near sigma = 1 lose ~5 digits to cancellation, which is the size of the parity
 // tolerance. Here the quantities that cancel are computed to FP64 accuracy: the
-// polar rotation R by FP64 Newton iterations from F; the log strains and the
-// principal directions from the eigen-decomposition of F^T F - I.
+// polar rotation R by FP64 Newton iterations from F; the principal directions from
+// the eigen-decomposition of F^T F, less I near a rotation, and the log strains from its
+// eigenvalues there or from the stretches |F v| of the directions.
 
 // Orthogonal polar factor r of a (a = r s, s symmetric positive definite) by
 // Newton's iteration x <- (g x + x^-T / g) / 2 with determinant scaling
@@ -341,28 +342,48 @@ __device__ inline void jacobi_rotate(double &pp, double &qq, double &pq, double 
     }
 }
 
-// Eigenvalues (less 1, in e) and eigenvectors (the columns of v, a rotation) of
-// F^T F by cyclic Jacobi sweeps.
-__device__ inline void eigen_f64(const float *f32, double *e, double *v) {
+// Eigenvectors (the columns of v, a rotation) of F^T F by cyclic Jacobi sweeps. With
+// NEAR and where F^T F is near I, true is returned and e holds its eigenvalues less 1, which then lose
+// nothing to the 1. Elsewhere that difference would lose what is left of a matrix far
+// smaller than I: e orders the eigenvalues only (they are scaled to a trace of 1, which
+// also keeps the FP32 angles of tiny and huge gradients in range).
+template <bool NEAR>
+__device__ inline bool eigen_f64(const float *f32, double *e, double *v) {
     double e00, e11, e22, e01, e02, e12;
+    bool near;
     {
         // The products are exact in FP64, the sums lose only FP64 round-off.
         double f[9];
 #pragma unroll
         for (int k = 0; k < 9; k++) f[k] = f32[k];
-        e00 = f[0] * f[0] + f[3] * f[3] + f[6] * f[6] - 1.0;
-        e11 = f[1] * f[1] + f[4] * f[4] + f[7] * f[7] - 1.0;
-        e22 = f[2] * f[2] + f[5] * f[5] + f[8] * f[8] - 1.0;
+        e00 = f[0] * f[0] + f[3] * f[3] + f[6] * f[6];
+        e11 = f[1] * f[1] + f[4] * f[4] + f[7] * f[7];
+        e22 = f[2] * f[2] + f[5] * f[5] + f[8] * f[8];
         e01 = f[0] * f[1] + f[3] * f[4] + f[6] * f[7];
         e02 = f[0] * f[2] + f[3] * f[5] + f[6] * f[8];
         e12 = f[1] * f[2] + f[4] * f[5] + f[7] * f[8];
+        near = NEAR && fmax(fmax(fabs(e00 - 1.0), fabs(e11 - 1.0)), fabs(e22 - 1.0)) <= 0.5;
+        if (near) {
+            e00 -= 1.0;
+            e11 -= 1.0;
+            e22 -= 1.0;
+        } else {
+            const double k = 1.0 / (e00 + e11 + e22);
+            e00 *= k;
+            e11 *= k;
+            e22 *= k;
+            e01 *= k;
+            e02 *= k;
+            e12 *= k;
+        }
     }
 #pragma unroll
     for (int k = 0; k < 9; k++) v[k] = k % 4 == 0 ? 1.0 : 0.0;
 #pragma unroll 1
     for (int sweep = 0; sweep < 12; sweep++) {
         const double off = e01 * e01 + e02 * e02 + e12 * e12;
-        const double dg = (1.0 + e00) * (1.0 + e00) + (1.0 + e11) * (1.0 + e11) + (1.0 + e22) * (1.0 + e22);
+        const double one = near ? 1.0 : 0.0;
+        const double dg = (one + e00) * (one + e00) + (one + e11) * (one + e11) + (one + e22) * (one + e22);
         if (!(off > 1.0e-30 * dg)) break;
         jacobi_rotate(e00, e11, e01, e02, e12, v, 0, 1);
         jacobi_rotate(e00, e22, e02, e01, e12, v, 0, 2);
@@ -371,6 +392,18 @@ __device__ inline void eigen_f64(const float *f32, double *e, double *v) {
     e[0] = e00;
     e[1] = e11;
     e[2] = e22;
+    return near;
+}
+
+// |F v_i|^2 of column i of v.
+__device__ inline double stretch2(const float *f, const double *v, int i) {
+    double s = 0.0;
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        const double w = (double)f[3 * k] * v[i] + (double)f[3 * k + 1] * v[3 + i] + (double)f[3 * k + 2] * v[6 + i];
+        s += w * w;
+    }
+    return s;
 }
 
 __device__ inline double det3d(const float *a) {
@@ -384,7 +417,7 @@ __device__ inline double det3d(const float *a) {
 // their left vectors, the third is their cross product.
 __device__ inline void rotation_by_eigen(const float *f, double *r) {
     double e[3], v[9];
-    eigen_f64(f, e, v);
+    eigen_f64<false>(f, e, v);
     // The column of the smallest eigenvalue goes last (cyclically: v stays a rotation).
 #pragma unroll 1
     for (int turn = 0; turn < 2 && (e[0] < e[2] || e[1] < e[2]); turn++) {
@@ -403,9 +436,11 @@ __device__ inline void rotation_by_eigen(const float *f, double *r) {
     double u[2][3];
 #pragma unroll
     for (int j = 0; j < 2; j++) {
-        const double w = 1.0 / sqrt(1.0 + e[j]);
 #pragma unroll
-        for (int i = 0; i < 3; i++) u[j][i] = w * ((double)f[3 * i] * v[j] + (double)f[3 * i + 1] * v[3 + j] + (double)f[3 * i + 2] * v[6 + j]);
+        for (int i = 0; i < 3; i++) u[j][i] = (double)f[3 * i] * v[j] + (double)f[3 * i + 1] * v[3 + j] + (double)f[3 * i + 2] * v[6 + j];
+        const double w = 1.0 / sqrt(u[j][0] * u[j][0] + u[j][1] * u[j][1] + u[j][2] * u[j][2]);
+#pragma unroll
+        for (int i = 0; i < 3; i++) u[j][i] *= w;
     }
     const double c[3] = {u[0][1] * u[1][2] - u[0][2] * u[1][1], u[0][2] * u[1][0] - u[0][0] * u[1][2],
                          u[0][0] * u[1][1] - u[0][1] * u[1][0]};
@@ -440,14 +475,11 @@ __device__ inline void fc_stress_f64(float lambda, float mu, const float *f32, f
 }
 
 // log(1 + e) / 2, the log of a singular value from the eigenvalue 1 + e of
-// F^T F: atanh(e / (2 + e)) by its series for |e| <= 1/4 (relative error below
-// 1e-10), the library's FP64 function beyond.
+// F^T F, for |e| <= 1/4: atanh(e / (2 + e)) by its series (relative error below
+// 1e-10).
 __device__ inline double half_log1p(double e) {
-    if (fabs(e) <= 0.25) {
-        const double r = e / (2.0 + e), q = r * r;
-        return r + r * q * (1.0 / 3.0 + q * (1.0 / 5.0 + q * (1.0 / 7.0 + q * (1.0 / 9.0 + q * (1.0 / 11.0)))));
-    }
-    return 0.5 * log1p(e);
+    const double r = e / (2.0 + e), q = r * r;
+    return r + r * q * (1.0 / 3.0 + q * (1.0 / 5.0 + q * (1.0 / 7.0 + q * (1.0 / 9.0 + q * (1.0 / 11.0)))));
 }
 
 // exp(x) - 1: its Taylor series for |x| <= 1/4 (relative error below 1e-11), the
@@ -486,14 +518,19 @@ __device__ inline void dp_project_f64(float *state, const float4 hp, float lambd
         return;
     }
     double e[3], v[9];
-    eigen_f64(f32, e, v);
+    const bool near = eigen_f64<true>(f32, e, v);
     const float q = state[1];
     const float angle = hp.x + (hp.y * q - hp.w) * expf(-hp.z * q);
     const float sa = sinf(angle);
     const double alpha = (double)(sqrtf(2.0f / 3.0f) * (2.0f * sa) / (3.0f - sa));
     const double lambda = lambda_f, mu = mu_f, third = (double)state[2] / 3.0;
-    const double raw[3] = {half_log1p(e[0]), half_log1p(e[1]), half_log1p(e[2])};
-    double dev[3];
+    // The log of a singular value: beyond the series' range from the stretch of its
+    // direction, whose square keeps the digits that an eigenvalue far below the largest one
+    // (1e-16 of that one off) has lost.
+    double raw[3], dev[3];
+#pragma unroll
+    for (int i = 0; i < 3; i++)
+        raw[i] = (near & (fabs(e[i]) <= 0.25)) ? half_log1p(e[i]) : 0.5 * log(stretch2(f32, v, i));
     const double tr = raw[0] + raw[1] + raw[2] + 3.0 * third;
 #pragma unroll
     for (int i = 0; i < 3; i++) dev[i] = raw[i] + third - tr / 3.0;
