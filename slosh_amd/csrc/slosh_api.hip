@@ -246,6 +246,8 @@ struct slosh_data {
     // Readback staging, made at the first readback and grown to at most
     // READ_STAGE_MAX: device records of one pass, their pinned copy, and (the pinned
     // allocation's first bytes) the word a pass marks if the storage is inconsistent.
+    // Held for the length of a readback (host threads may read the same data at once).
+    std::mutex read_mu;
     uint8_t *read_dev = nullptr, *read_host = nullptr;
     size_t read_bytes = 0;
     uint32_t read_mark = 0;
@@ -1427,6 +1429,7 @@ static GatherArgs current_particles(slosh_data *d) {
 static int read_records(slosh_data *d, uint32_t kind, size_t rec, void *out, hipStream_t st) {
     const size_t n = d->n;
     if (n == 0) return SLOSH_OK;
+    std::lock_guard<std::mutex> lock(d->read_mu);
     TRY(reserve_read_staging(d, n * rec));
     uint32_t *bad = nullptr;
     HIP_TRY(hipHostGetDevicePointer((void **)&bad, d->read_host, 0));
@@ -2656,6 +2659,7 @@ int slosh_read_scene(slosh_data *d, slosh_stream stream, uint32_t scene_id, floa
     if (m == 0) return SLOSH_OK;
     if (m > max_count) return fail(SLOSH_E_INVALID, "output smaller than the scene");
     hipStream_t st = (hipStream_t)stream;
+    std::lock_guard<std::mutex> lock(d->read_mu);
     // Staging: the particle buffer the next substep writes (free between substeps).
     const PBufs &stg = d->pb[d->cur_p ^ 1];
     GatherArgs a = current_particles(d);
