@@ -215,14 +215,17 @@ __global__ __launch_bounds__(256) void k_scene_gather(PSet in, PSet out, uint32_
 // contiguous copy (27 us; 0.65 ms). A particle of a block is 16 to 96 bytes at a
 // scattered id, 4 bytes read per component in slot order; 12 us at 1M positions
 // against the 0.3 ms the copy then takes. An id outside [0, n) marks the storage
-// as inconsistent: *bad (host memory) becomes `mark`.
+// as inconsistent (bad[0] in host memory becomes `mark`), as does an overflow in the
+// error words of either table (bad[1]): then ids may be missing from it, or in it twice.
 __global__ __launch_bounds__(256) void k_read_records(PSet in, uint32_t n, uint32_t pcap, uint32_t kind, uint32_t lo,
                                                       uint32_t count, float4 *__restrict__ out,
-                                                      volatile uint32_t *bad, uint32_t mark) {
+                                                      const uint32_t *__restrict__ counters, volatile uint32_t *bad,
+                                                      uint32_t mark) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     const uint32_t id = in.ids[i];
-    if (id >= n) *bad = mark;
+    if (id >= n) bad[0] = mark;
+    if (i == 0u && ((counters[CTR_ERRORS] | counters[8 + CTR_ERRORS]) & (ERR_HASH_FULL | ERR_LOOKUP))) bad[1] = mark;
     if (id < lo || id - lo >= count || id >= n) return;
     if (kind == READ_POSITIONS) {
         const float4 p = in.pos[i];
@@ -297,10 +300,11 @@ hipError_t launch_scene_gather(const GatherArgs &a, uint32_t n, uint32_t pcap, u
 }
 
 hipError_t launch_read_records(const GatherArgs &a, uint32_t n, uint32_t pcap, uint32_t kind, uint32_t lo,
-                               uint32_t count, void *out, uint32_t *bad, uint32_t mark, hipStream_t st) {
+                               uint32_t count, void *out, const uint32_t *counters, uint32_t *bad, uint32_t mark,
+                               hipStream_t st) {
     if (n == 0 || count == 0) return hipSuccess;
     PSet in{a.pos, a.vm, a.C, a.F, a.vgd, a.dps, a.fdt, a.ids};
     hipLaunchKernelGGL(k_read_records, dim3(div_up_u(n, 256)), dim3(256), 0, st, in, n, pcap, kind, lo, count,
-                       (float4 *)out, bad, mark);
+                       (float4 *)out, counters, bad, mark);
     return hipGetLastError();
 }

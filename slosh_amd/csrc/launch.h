@@ -154,8 +154,10 @@ struct GatherArgs {
 hipError_t launch_scene_gather(const GatherArgs &a, uint32_t n, uint32_t pcap, uint32_t scene, uint32_t count,
                                uint32_t strip, hipStream_t st);
 // Reference records of the particles with ids [lo, lo + count) into `out`, in id
-// order; `bad` (mapped host memory) becomes `mark` if an id is not below n.
+// order; of `bad` (mapped host memory) word 0 becomes `mark` if an id is not below n,
+// word 1 if `counters` (both tables') report an overflow.
 enum { READ_POSITIONS = 0, READ_KINEMATICS, READ_DEF_GRAD };
 hipError_t launch_read_records(const GatherArgs &a, uint32_t n, uint32_t pcap, uint32_t kind, uint32_t lo,
-                               uint32_t count, void *out, uint32_t *bad, uint32_t mark, hipStream_t st);
+                               uint32_t count, void *out, const uint32_t *counters, uint32_t *bad, uint32_t mark,
+                               hipStream_t st);
 uint32_t scan_tiles(uint32_t n);

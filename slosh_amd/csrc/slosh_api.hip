@@ -25,6 +25,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
@@ -245,12 +246,14 @@ struct slosh_data {
     int *impulses = nullptr;
     // Readback staging, made at the first readback and grown to at most
     // READ_STAGE_MAX: device records of one pass, their pinned copy, and (the pinned
-    // allocation's first bytes) the word a pass marks if the storage is inconsistent.
+    // allocation's first bytes) the words a pass marks if the storage is inconsistent.
     // Held for the length of a readback (host threads may read the same data at once).
     std::mutex read_mu;
     uint8_t *read_dev = nullptr, *read_host = nullptr;
     size_t read_bytes = 0;
     uint32_t read_mark = 0;
+    // A grid overflow was seen: an id may be in two slots, or in none.
+    std::atomic<bool> lost{false};
     std::vector<hipEvent_t> read_done;
     // Captured runs of substeps: pairs, one per starting parity, then runs of
     // GRAPH_LONG (slots 4 to 7), each with the step parameters it was captured with (a
@@ -1358,8 +1361,16 @@ static int reserve_read_staging(slosh_data *d, size_t bytes) {
     return SLOSH_OK;
 }
 
-// Copies `bytes` (at most the staging's size) from device memory to `dst`.
-static int download(slosh_data *d, const void *src, size_t bytes, void *dst, hipStream_t st) {
+// Whether the pass marked `mark` found the storage inconsistent (word 0: an id out of
+// range; word 1: the grid has overflowed).
+static bool read_marked(const slosh_data *d, int word, uint32_t mark) {
+    return reinterpret_cast<const volatile uint32_t *>(d->read_host)[word] == mark;
+}
+
+// Copies `bytes` (at most the staging's size) from device memory to `dst`, unless the pass
+// before it on the stream, marked `mark`, found the storage inconsistent (mark 0: none).
+static int download(slosh_data *d, const void *src, size_t bytes, void *dst, hipStream_t st, uint32_t mark = 0) {
+    auto stop = [&] { return mark && (read_marked(d, 0, mark) || read_marked(d, 1, mark)); };
     uint8_t *stage = d->read_host + READ_HEAD;
     uint8_t *to = static_cast<uint8_t *>(dst);
     const uint8_t *from = static_cast<const uint8_t *>(src);
@@ -1368,7 +1379,7 @@ static int download(slosh_data *d, const void *src, size_t bytes, void *dst, hip
     if (T == 1) {
         HIP_TRY(hipMemcpyAsync(stage, from, bytes, hipMemcpyDeviceToHost, st));
         HIP_TRY(hipStreamSynchronize(st));
-        std::memcpy(to, stage, bytes);
+        if (!stop()) std::memcpy(to, stage, bytes);
         return SLOSH_OK;
     }
     const size_t pieces = (bytes + READ_PIECE - 1) / READ_PIECE;
@@ -1391,6 +1402,7 @@ static int download(slosh_data *d, const void *src, size_t bytes, void *dst, hip
                 err[t] = e;
                 return;
             }
+            if (stop()) return;
             std::memcpy(to + o, stage + o, len);
         }
     };
@@ -1424,12 +1436,45 @@ static GatherArgs current_particles(slosh_data *d) {
     return a;
 }
 
+// The same assembled on the host from a copy of the state, for a storage that a grid
+// overflow has left inconsistent: the last of an id's slots counts, an id without one
+// reads as zeros.
+static int read_records_host(slosh_data *d, uint32_t kind, size_t rec, void *out, hipStream_t st) {
+    Snapshot s;
+    TRY(download_current(d, st, s));
+    const size_t n = d->n;
+    std::memset(out, 0, n * rec);
+    for (size_t i = 0; i < n; i++) {
+        const uint32_t id = s.ids[i];
+        if (kind == READ_POSITIONS) {
+            std::memcpy(static_cast<float *>(out) + 4 * (size_t)id, &s.pos[4 * i], 12);
+        } else if (kind == READ_DEF_GRAD) {
+            slosh_matrix &m = static_cast<slosh_matrix *>(out)[id];
+            for (int r = 0; r < 3; r++)
+                for (int c = 0; c < 3; c++) m.m[r][c] = s.F[(size_t)(r * 3 + c) * n + i];
+        } else {
+            slosh_kinematics &k = static_cast<slosh_kinematics *>(out)[id];
+            for (int r = 0; r < 3; r++)
+                for (int c = 0; c < 3; c++) k.affine.m[r][c] = s.C[(size_t)(r * 3 + c) * n + i];
+            for (int c = 0; c < 3; c++) {
+                k.velocity[c] = s.vm[4 * i + c];
+                k.force_dt[c] = s.fdt[(size_t)c * n + i];
+            }
+            k.vel_grad_det = s.vgd[i];
+            k.mass = s.vm[4 * i + 3];
+            k.enabled = f2u(s.pos[4 * i + 3]) & 1u;
+        }
+    }
+    return SLOSH_OK;
+}
+
 // Every particle's record of `kind` (`rec` bytes) in id order, through the staging,
 // as many ids per pass as it holds.
 static int read_records(slosh_data *d, uint32_t kind, size_t rec, void *out, hipStream_t st) {
     const size_t n = d->n;
     if (n == 0) return SLOSH_OK;
     std::lock_guard<std::mutex> lock(d->read_mu);
+    if (d->lost) return read_records_host(d, kind, rec, out, st);
     TRY(reserve_read_staging(d, n * rec));
     uint32_t *bad = nullptr;
     HIP_TRY(hipHostGetDevicePointer((void **)&bad, d->read_host, 0));
@@ -1438,11 +1483,12 @@ static int read_records(slosh_data *d, uint32_t kind, size_t rec, void *out, hip
     for (size_t lo = 0; lo < n; lo += per) {
         const size_t count = std::min(per, n - lo);
         HIP_TRY(launch_read_records(current_particles(d), (uint32_t)n, (uint32_t)d->pcap, kind, (uint32_t)lo,
-                                    (uint32_t)count, d->read_dev, bad, mark, st));
-        TRY(download(d, d->read_dev, count * rec, static_cast<uint8_t *>(out) + lo * rec, st));
+                                    (uint32_t)count, d->read_dev, d->counters, bad, mark, st));
+        TRY(download(d, d->read_dev, count * rec, static_cast<uint8_t *>(out) + lo * rec, st, mark));
+        if (read_marked(d, 0, mark))
+            return fail(SLOSH_E_GRID_OVERFLOW, "particle storage inconsistent (grid overflow?)");
+        if (read_marked(d, 1, mark)) return read_records_host(d, kind, rec, out, st);
     }
-    if (*reinterpret_cast<volatile uint32_t *>(d->read_host) == mark)
-        return fail(SLOSH_E_GRID_OVERFLOW, "particle storage inconsistent (grid overflow?)");
     return SLOSH_OK;
 }
 
@@ -2116,6 +2162,7 @@ int slosh_check_errors(slosh_data *d, slosh_stream stream) {
     HIP_TRY(hipStreamSynchronize(st));
     const uint32_t err = c[CTR_ERRORS] | c[8 + CTR_ERRORS];
     if (err != 0u) {
+        if (err & (ERR_HASH_FULL | ERR_LOOKUP)) d->lost = true;
         uint32_t zero = 0;
         HIP_TRY(hipMemcpy(d->counters + CTR_ERRORS, &zero, 4, hipMemcpyHostToDevice));
         HIP_TRY(hipMemcpy(d->counters + 8 + CTR_ERRORS, &zero, 4, hipMemcpyHostToDevice));
