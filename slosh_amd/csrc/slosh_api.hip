@@ -245,12 +245,13 @@ struct slosh_data {
     uint2 *mats = nullptr;
     int *impulses = nullptr;
     // Readback staging, made at the first readback and grown to at most
-    // READ_STAGE_MAX: device records of one pass, their pinned copy, and (the pinned
-    // allocation's first bytes) the words a pass marks if the storage is inconsistent.
+    // READ_STAGE_MAX: device records of one pass (a scene's readback has none), their
+    // pinned copy, and (the pinned allocation's first bytes) the words a pass marks if the
+    // storage is inconsistent.
     // Held for the length of a readback (host threads may read the same data at once).
     std::mutex read_mu;
     uint8_t *read_dev = nullptr, *read_host = nullptr;
-    size_t read_bytes = 0;
+    size_t read_bytes = 0, read_dev_bytes = 0;
     uint32_t read_mark = 0;
     // A grid overflow was seen: an id may be in two slots, or in none.
     std::atomic<bool> lost{false};
@@ -1333,31 +1334,55 @@ static int ring_commit(slosh_data *d, size_t off, size_t need, hipStream_t st) {
 // way: a direct copy into pageable memory runs at 2.4 GB/s for 2 MiB and page-faults
 // on one thread (4.5 ms for 16 MiB), pinned at 56 GB/s and the faults of four threads
 // side by side 0.3 ms.
-static constexpr size_t READ_STAGE_MAX = (size_t)64 << 20, READ_PIECE = (size_t)1 << 20, READ_HEAD = 64;
+static constexpr size_t READ_STAGE_MAX = (size_t)64 << 20, READ_STAGE_MIN = (size_t)64 << 10;
+static constexpr size_t READ_PIECE = (size_t)1 << 20, READ_HEAD = 64;
 
 static void release_read_staging(slosh_data *d) {
     if (d->read_dev) (void)hipFree(d->read_dev);
     if (d->read_host) (void)hipHostFree(d->read_host);
     d->read_dev = d->read_host = nullptr;
-    d->read_bytes = 0;
+    d->read_bytes = d->read_dev_bytes = 0;
     for (hipEvent_t e : d->read_done) (void)hipEventDestroy(e);
     d->read_done.clear();
 }
 
-// Staging for `bytes` (or READ_STAGE_MAX of them).
+// Pinned staging for `bytes` (or READ_STAGE_MAX of them; where so much is not to be had,
+// for less, in more passes).
 static int reserve_read_staging(slosh_data *d, size_t bytes) {
     bytes = std::min(bytes, READ_STAGE_MAX);
     if (bytes <= d->read_bytes) return SLOSH_OK;
     release_read_staging(d);  // (every readback waits for its copies)
-    if (hipMalloc((void **)&d->read_dev, bytes) != hipSuccess ||
-        hipHostMalloc((void **)&d->read_host, READ_HEAD + bytes, hipHostMallocDefault) != hipSuccess) {
+    while (hipHostMalloc((void **)&d->read_host, READ_HEAD + bytes, hipHostMallocDefault) != hipSuccess) {
         (void)hipGetLastError();
-        release_read_staging(d);
-        return fail(SLOSH_E_NO_MEMORY, "readback staging");
+        d->read_host = nullptr;
+        if (bytes <= READ_STAGE_MIN) return fail(SLOSH_E_NO_MEMORY, "readback staging");
+        bytes /= 2;
     }
     std::memset(d->read_host, 0, READ_HEAD);
     d->read_mark = 0;
     d->read_bytes = bytes;
+    return SLOSH_OK;
+}
+
+// Where a pass's records of up to `bytes` (as many as the pinned staging holds at most) are
+// written: device memory, or the pinned staging itself if there is none left.
+static int reserve_read_records(slosh_data *d, size_t bytes, uint8_t **records) {
+    bytes = std::min(bytes, d->read_bytes);
+    if (bytes > d->read_dev_bytes) {
+        if (d->read_dev) (void)hipFree(d->read_dev);
+        d->read_dev = nullptr;
+        d->read_dev_bytes = 0;
+        if (hipMalloc((void **)&d->read_dev, bytes) == hipSuccess) {
+            d->read_dev_bytes = bytes;
+        } else {
+            (void)hipGetLastError();
+            d->read_dev = nullptr;
+            HIP_TRY(hipHostGetDevicePointer((void **)records, d->read_host, 0));
+            *records += READ_HEAD;
+            return SLOSH_OK;
+        }
+    }
+    *records = d->read_dev;
     return SLOSH_OK;
 }
 
@@ -1367,12 +1392,18 @@ static bool read_marked(const slosh_data *d, int word, uint32_t mark) {
     return reinterpret_cast<const volatile uint32_t *>(d->read_host)[word] == mark;
 }
 
-// Copies `bytes` (at most the staging's size) from device memory to `dst`, unless the pass
+// Copies `bytes` (at most the staging's size) from device memory (null: what is in the
+// pinned staging once the stream is done) to `dst`, unless the pass
 // before it on the stream, marked `mark`, found the storage inconsistent (mark 0: none).
 static int download(slosh_data *d, const void *src, size_t bytes, void *dst, hipStream_t st, uint32_t mark = 0) {
     auto stop = [&] { return mark && (read_marked(d, 0, mark) || read_marked(d, 1, mark)); };
     uint8_t *stage = d->read_host + READ_HEAD;
     uint8_t *to = static_cast<uint8_t *>(dst);
+    if (!src) {  // the records were written there
+        HIP_TRY(hipStreamSynchronize(st));
+        if (!stop()) std::memcpy(to, stage, bytes);
+        return SLOSH_OK;
+    }
     const uint8_t *from = static_cast<const uint8_t *>(src);
     const size_t T = std::min<size_t>({4, std::max<size_t>(1, std::thread::hardware_concurrency() / 2),
                                        bytes / (2 * READ_PIECE) + 1});
@@ -1477,13 +1508,15 @@ static int read_records(slosh_data *d, uint32_t kind, size_t rec, void *out, hip
     if (d->lost) return read_records_host(d, kind, rec, out, st);
     TRY(reserve_read_staging(d, n * rec));
     uint32_t *bad = nullptr;
+    uint8_t *records = nullptr;
     HIP_TRY(hipHostGetDevicePointer((void **)&bad, d->read_host, 0));
+    TRY(reserve_read_records(d, n * rec, &records));
     const uint32_t mark = ++d->read_mark;
     const size_t per = d->read_bytes / rec;
     for (size_t lo = 0; lo < n; lo += per) {
         const size_t count = std::min(per, n - lo);
         HIP_TRY(launch_read_records(current_particles(d), (uint32_t)n, (uint32_t)d->pcap, kind, (uint32_t)lo,
-                                    (uint32_t)count, d->read_dev, d->counters, bad, mark, st));
+                                    (uint32_t)count, records, d->counters, bad, mark, st));
         TRY(download(d, d->read_dev, count * rec, static_cast<uint8_t *>(out) + lo * rec, st, mark));
         if (read_marked(d, 0, mark))
             return fail(SLOSH_E_GRID_OVERFLOW, "particle storage inconsistent (grid overflow?)");
