@@ -68,6 +68,15 @@ static void dfree(T *&p) {
     p = nullptr;
 }
 
+// A device copy of n elements at *p.
+template <typename T>
+static int upload(T **p, const std::remove_cv_t<T> *src, size_t n) {
+    const int rc = dalloc(p, n);
+    if (rc != SLOSH_OK || n == 0) return rc;
+    const hipError_t e = hipMemcpy((void *)*p, src, sizeof(T) * n, hipMemcpyHostToDevice);
+    return e == hipSuccess ? SLOSH_OK : fail(SLOSH_E_HIP, std::string("hipMemcpy: ") + hipGetErrorString(e));
+}
+
 #define TRY(expr)                    \
     do {                             \
         int r_ = (expr);             \
@@ -1055,7 +1064,7 @@ static const PassEvents *pass_events(slosh_timestamps *ts, int pass, PassEvents 
 // ---- one substep --------------------------------------------------------------
 static int run_step(slosh_pipeline *pl, slosh_data *d, hipStream_t st, const slosh_hooks *hooks, void *hs,
                     slosh_timestamps *ts) {
-    if (d->has_trimesh && !d->mesh_vtx)
+    if (d->has_trimesh && !(d->mesh_vtx && d->mesh_nodes && d->mesh_leaves && d->mesh_base))
         return fail(SLOSH_E_INVALID, "trimesh colliders need slosh_data_set_collision_mesh before stepping");
     const slosh_kernels &K = pl->kernels;
     const bool any_hook = hooks && (hooks->after_particle_sort || hooks->run_p2g || hooks->run_g2p || hooks->after_p2g ||
@@ -2018,9 +2027,15 @@ static bool walk_reaches_all(const float *vertices4, const uint32_t *indices, si
     return reached == leaves;
 }
 
-static int pack_meshes(slosh_data *d, const float *vertices4, const uint32_t *indices) {
+struct PackedMeshes {
     std::vector<float4> nodes, leaves;
-    std::vector<uint32_t> base(2 * SLOSH_MAX_COLLIDERS, 0u);
+    std::vector<uint32_t> base;
+};
+
+static void pack_meshes(const slosh_data *d, const float *vertices4, const uint32_t *indices, PackedMeshes &out) {
+    std::vector<float4> &nodes = out.nodes, &leaves = out.leaves;
+    std::vector<uint32_t> &base = out.base;
+    base.assign(2 * SLOSH_MAX_COLLIDERS, 0u);
     for (uint32_t b = 0; b < d->nbodies; b++) {
         const slosh_shape &sh = d->bodies_host[b].shape;
         if (f2u(sh.a[3]) != 6u) continue;
@@ -2058,19 +2073,10 @@ static int pack_meshes(slosh_data *d, const float *vertices4, const uint32_t *in
             leaves.insert(leaves.end(), v, v + 3);
         }
     }
-    dfree(d->mesh_nodes);
-    dfree(d->mesh_leaves);
-    dfree(d->mesh_base);
-    TRY(dalloc(&d->mesh_nodes, std::max<size_t>(nodes.size(), 2)));
-    TRY(dalloc(&d->mesh_leaves, std::max<size_t>(leaves.size(), 3)));
-    TRY(dalloc(&d->mesh_base, base.size()));
-    if (!nodes.empty()) {
-        HIP_TRY(hipMemcpy(d->mesh_nodes, nodes.data(), 16 * nodes.size(), hipMemcpyHostToDevice));
-        HIP_TRY(hipMemcpy(d->mesh_leaves, leaves.data(), 16 * leaves.size(), hipMemcpyHostToDevice));
-    }
-    HIP_TRY(hipMemcpy(d->mesh_base, base.data(), 4 * base.size(), hipMemcpyHostToDevice));
-    return SLOSH_OK;
+    nodes.resize(std::max<size_t>(nodes.size(), 2));
+    leaves.resize(std::max<size_t>(leaves.size(), 3));
 }
+
 
 int slosh_data_set_collision_mesh(slosh_data *d, const float *vertices4, size_t num_vertices,
                                   const uint32_t *indices, size_t num_indices) {
@@ -2108,18 +2114,38 @@ int slosh_data_set_collision_mesh(slosh_data *d, const float *vertices4, size_t 
                                                      ": the root BVH box does not hold every triangle");
         }
     }
-    invalidate_graphs(d);
-    TRY(pack_meshes(d, vertices4, indices));
-    dfree(d->mesh_vtx);
-    dfree(d->mesh_idx);
-    TRY(dalloc(&d->mesh_vtx, 4 * std::max<size_t>(num_vertices, 1)));
-    TRY(dalloc(&d->mesh_idx, std::max<size_t>(num_indices, 1)));
-    if (num_vertices) HIP_TRY(hipMemcpy(d->mesh_vtx, vertices4, 16 * num_vertices, hipMemcpyHostToDevice));
-    if (num_indices) HIP_TRY(hipMemcpy(d->mesh_idx, indices, 4 * num_indices, hipMemcpyHostToDevice));
-    d->mesh_nv = num_vertices;
-    d->mesh_ni = num_indices;
-    invalidate_graphs(d);
-    return SLOSH_OK;
+    // All of the new buffers, then the exchange: without memory for them the data keeps the
+    // ones it has.
+    PackedMeshes packed;
+    try {
+        pack_meshes(d, vertices4, indices, packed);
+    } catch (const std::bad_alloc &) {
+        return fail(SLOSH_E_NO_MEMORY, "collision mesh");
+    }
+    float *vtx = nullptr;
+    uint32_t *idx = nullptr, *base = nullptr;
+    float4 *nodes = nullptr, *leaves = nullptr;
+    int rc = upload(&vtx, vertices4, 4 * num_vertices);
+    if (rc == SLOSH_OK) rc = upload(&idx, indices, num_indices);
+    if (rc == SLOSH_OK) rc = upload(&nodes, packed.nodes.data(), packed.nodes.size());
+    if (rc == SLOSH_OK) rc = upload(&leaves, packed.leaves.data(), packed.leaves.size());
+    if (rc == SLOSH_OK) rc = upload(&base, packed.base.data(), packed.base.size());
+    if (rc == SLOSH_OK) {
+        invalidate_graphs(d);
+        std::swap(vtx, d->mesh_vtx);
+        std::swap(idx, d->mesh_idx);
+        std::swap(nodes, d->mesh_nodes);
+        std::swap(leaves, d->mesh_leaves);
+        std::swap(base, d->mesh_base);
+        d->mesh_nv = num_vertices;
+        d->mesh_ni = num_indices;
+    }
+    dfree(vtx);
+    dfree(idx);
+    dfree(nodes);
+    dfree(leaves);
+    dfree(base);
+    return rc;
 }
 
 int slosh_set_svd_fp64(slosh_data *d, int enable) {
