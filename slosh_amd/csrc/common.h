@@ -80,10 +80,15 @@ __device__ __host__ inline uint32_t tile_index(uint32_t x, uint32_t y, uint32_t 
 #define ITEM_TOTAL 14      // members
 #define ITEM_OVERFLOW 15   // nonzero: some of the block's movers are in the overflow list
 
-// Most BVH nodes of a trimesh whose leaves the grid update tests without a walk (substep
-// of 85k particles over a heightfield of 1747 nodes 55.1 us, walked by levels 60.0; 7379
-// nodes 78.5 and 81.9; 14867 nodes 107 and 105).
-#define MESH_FLAT 8192
+// How the grid update finds a mesh's closest triangles: by the BVH walk of each node; or, if
+// that finds the closest of them all, from the leaves near the block, found by levels of
+// the tree or, of a tree of up to MESH_FLAT_NODES, among all of its leaves (substep of 85k
+// particles over a heightfield of 1747 nodes 55.1 us, by levels 60.0; 7379 nodes 78.5 and
+// 81.9; 14867 nodes 107 and 105).
+#define MESH_WALK 0u
+#define MESH_LEVELS 1u
+#define MESH_FLAT 2u
+#define MESH_FLAT_NODES 8192
 
 // Particles per workgroup of the two-pass timestep bound (one partial minimum each).
 #define TSB_CHUNK 2048u

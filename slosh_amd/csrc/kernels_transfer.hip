@@ -742,10 +742,11 @@ struct Colliders {
     uint32_t count;
     const float4 *mesh_vtx;   // trimesh collision vertices: BVH AABBs, vertices, pseudo-normals
     const uint32_t *mesh_idx; // trimesh collision indices: BVH topology, triangles
-    // The BVHs of the trimesh bodies as the walk reads them (see pack_meshes), and
-    // each body's first node.
+    // The BVHs of the trimesh bodies as the walk reads them (see pack_meshes), each
+    // body's first node, and how its closest triangles are found (MESH_*).
     const float4 *mesh_nodes, *mesh_leaves;
-    const uint32_t *mesh_base, *mesh_flat;
+    const uint32_t *mesh_base, *mesh_search;
+    const float *mesh_size;  // largest coordinate
 };
 
 // triangle_project_local_point_and_get_location (trimesh.slang:304-377): closest
@@ -827,46 +828,42 @@ __device__ inline float leaf_distance(const float4 *__restrict__ leaf, float3 pt
     return sqrtf(dx * dx + dy * dy + dz * dz);
 }
 
+// Distance of a point from the box of the triangle of `leaf`.
+__device__ inline float leaf_box_distance(const float4 *__restrict__ leaf, float3 pt) {
+    const float4 a = leaf[0], b = leaf[1], c = leaf[2];
+    return box_distance(make_float4(fminf(fminf(a.x, b.x), c.x), fminf(fminf(a.y, b.y), c.y), fminf(fminf(a.z, b.z), c.z), 0.0f),
+                        make_float4(fmaxf(fmaxf(a.x, b.x), c.x), fmaxf(fmaxf(a.y, b.y), c.y), fmaxf(fmaxf(a.z, b.z), c.z), 0.0f),
+                        pt);
+}
+
 // TriMesh::project_local_point (trimesh.slang:111-154): the leaf of the closest
 // triangle within max_dist by the stackless BVH walk (SLOSH_NONE: none; links point
-// forward, checked on the host, so the walk ends). The lanes of a wave hold
-// neighbouring nodes and visit mostly the same BVH nodes, so they walk together: each
-// step takes the first node any lane is at, which makes its record one scalar load,
-// and the lanes that are there test it. Every lane still visits its own nodes in its
-// own order. A lane skips a leaf whose box (grown by 1 % on the host, far above
-// rounding) is farther than its best so far, which the reference tests all the same;
-// its triangle cannot win.
+// forward, checked on the host, so the walk ends), each lane for its own point. With `cull`,
+// a leaf whose box (grown by 1 % on the host, far above rounding) is farther than the best
+// so far is skipped, which the reference tests all the same: no triangle but a degenerate
+// one can win from there.
 __device__ inline uint32_t trimesh_walk(const float4 *__restrict__ node, const float4 *__restrict__ leaf,
-                                        uint32_t nodes, float3 pt, float max_dist) {
+                                        uint32_t nodes, float3 pt, float max_dist, bool cull) {
     float best = max_dist;
     uint32_t best_leaf = SLOSH_NONE;
-    uint32_t cur = 0u, at = 0u;  // this lane's next node, the wave's
-    while (at < nodes) {
+    for (uint32_t at = 0u; at < nodes;) {
         const float4 mn = node[2u * at], mx = node[2u * at + 1u];
         const uint32_t entry = __float_as_uint(mn.w), exit_ = __float_as_uint(mx.w);
-        if (cur == at) {
-            const float dbox = box_distance(mn, mx, pt);
-            const bool is_leaf = entry == SLOSH_NONE;
-            cur = !is_leaf && dbox < best ? entry : exit_;
-            if (is_leaf && dbox <= best) {
-                float3 p;
-                uint32_t tri, feat, id;
-                const float dist = leaf_distance(leaf + 3u * (size_t)at, pt, &p, &tri, &feat, &id);
-                if (dist <= best) {
-                    best = dist;
-                    best_leaf = at;
-                }
+        const float dbox = box_distance(mn, mx, pt);
+        if (entry != SLOSH_NONE) {
+            at = dbox < best ? entry : exit_;
+            continue;
+        }
+        if (!cull || dbox <= best) {
+            float3 p;
+            uint32_t tri, feat, id;
+            const float dist = leaf_distance(leaf + 3u * (size_t)at, pt, &p, &tri, &feat, &id);
+            if (dist <= best) {
+                best = dist;
+                best_leaf = at;
             }
         }
-        // The first node a lane is at now: usually the next one.
-        if (__ballot(cur == at + 1u)) {
-            at = at + 1u;
-        } else {
-            uint32_t m = __builtin_amdgcn_readfirstlane(cur);
-            for (uint64_t less = __ballot(cur < m); less; less = __ballot(cur < m))
-                m = __builtin_amdgcn_readlane(cur, __ffsll((unsigned long long)less) - 1);
-            at = m;
-        }
+        at = exit_;
     }
     return best_leaf;
 }
@@ -903,17 +900,25 @@ __device__ inline void trimesh_contact(const Colliders &cs, uint32_t i, uint32_t
 // for every trimesh collider: the leaves near the block are collected, of a small mesh
 // from all its nodes at once, else by one wave, a level of the BVH at a time; then each
 // wave tests its share of them for all nodes (lane = node), culled by the closest that
-// any wave has found, and the closest wins by an LDS minimum over (distance, later leaf
-// first), the order the walk decides ties in.
+// any wave has found, and the closest wins by an LDS minimum over (distance, leaf).
+//
+// The walk (trimesh_walk) defines the result. It finds the same point, but for rounding, if
+// every triangle lies in the boxes above it (the host says which meshes are such; MESH_WALK:
+// not) and it cannot miss the closest one: a triangle farther than its own box is surely
+// met, as the boxes above are nearer still. One at its box's distance (it lies along an
+// axis, say) may be left out when another point is as far, or when the reach is, by the
+// strict comparison with the boxes: such nodes are walked after all.
 //
 // Bound by latency: a block is 64 nodes with ~50 triangles in reach, and one triangle
 // test ~300 dependent instructions, so one wave per block left the chip idle. The
 // grid update of 85k particles over an 874-triangle heightfield (429 blocks): walked
-// per lane 110 us, walked by the wave together 114 us, shared by 8 waves 28 us (4 waves
-// 37, 16 waves 48), with the leaves from all nodes at once 23 us, culled together 22 us.
-// The whole substep at finer heightfields (before: 512 leaves and 256 nodes of a level,
-// walked per lane beyond): 3690 triangles 287 -> 78 us, 7434 455 -> 106, 15834 770 -> 152.
-#define MESH_WAVES 8
+// per lane 110 us, shared by 8 waves 28 us (4 waves 37, 16 waves 48), with the leaves from
+// all nodes at once 23 us, culled together and the undecided nodes walked 23.5 us. Over
+// finer heightfields, walked per lane and now: 3698 triangles 180 -> 48 us, 15842 329 ->
+// 127, 178802 (too many near a block: walked, eight nodes to a wave) 1213 -> 812; over a flat
+// aligned floor of 2048, most of whose nodes are walked after all, 41 -> 37; a tree with
+// short boxes over 3698 triangles 181 -> 125.
+#define MESH_WAVES 8  // (each has eight of the 64 nodes where they are walked)
 #define MESH_CAND 2048   // leaves near a block that the workgroup shares; more are walked
 #define MESH_FRONT 2048  // nodes of a level near a block
 struct MeshShared {
@@ -921,7 +926,17 @@ struct MeshShared {
     uint32_t front[2][MESH_FRONT];
     uint32_t n_cand;  // above MESH_CAND: more than fit
     unsigned long long key[SLOSH_MAX_COLLIDERS][NODES_PER_BLOCK];  // all ones: none in reach
+    float point[3][NODES_PER_BLOCK];  // on the closest
+    uint32_t tie[NODES_PER_BLOCK];    // least distance that the walk has to decide (float bits)
 };
+
+// MeshShared::key: the distance (float bits), the leaf (the later one first, as the walk
+// decides ties).
+__device__ inline unsigned long long mesh_key(float dist, uint32_t leaf) {
+    return ((unsigned long long)__float_as_uint(dist) << 32) | ~leaf;
+}
+__device__ inline uint32_t key_leaf(unsigned long long key) { return ~(uint32_t)key; }
+__device__ inline float key_distance(unsigned long long key) { return __uint_as_float((uint32_t)(key >> 32)); }
 
 // Appends `v` of the lanes in `on` to list[0, *n) (wave-uniform *n); false if it does not fit.
 __device__ inline bool push(uint32_t *list, uint32_t cap, uint32_t *n, bool on, uint32_t v) {
@@ -1068,7 +1083,7 @@ __device__ inline NodeColl collide(const Colliders &cs, const float4 *box, float
             const unsigned long long key = keys[i][lane];
             if (key == ~0ull) continue;
             float3 lproj;
-            trimesh_contact(cs, i, ~(uint32_t)key, sim_inv_mul_pt(rot, ts, point), &lproj, &inside);
+            trimesh_contact(cs, i, key_leaf(key), sim_inv_mul_pt(rot, ts, point), &lproj, &inside);
             proj = sim_mul_pt(rot, ts, lproj);
         } else if (ty <= 4u) {
             float3 lp = sim_inv_mul_pt(rot, ts, point);
@@ -1842,18 +1857,24 @@ __device__ inline void mesh_queries(const Colliders &cs, const float4 *box, Mesh
         const float4 lo = box[2 * i], hi = box[2 * i + 1];
         const bool on = need && cell_pos.x >= lo.x && cell_pos.x <= hi.x && cell_pos.y >= lo.y && cell_pos.y <= hi.y &&
                         cell_pos.z >= lo.z && cell_pos.z <= hi.z;
-        if (wave == 0u) S.key[i][lane] = ~0ull;
+        if (wave == 0u) {
+            S.key[i][lane] = ~0ull;
+            S.tie[lane] = ~0u;
+        }
         if (__ballot(on) == 0ull) continue;  // (every wave holds the same nodes)
         const float4 rot = cs.poses[2 * i], ts = cs.poses[2 * i + 1];
         const uint32_t base = cs.mesh_base[i], count = __float_as_uint(a.z);
-        const bool flat = cs.mesh_flat[i] != 0u;
+        const uint32_t search = cs.mesh_search[i];
+        const bool flat = search == MESH_FLAT;
         const float4 *node = cs.mesh_nodes + 2u * (size_t)base, *leaf = cs.mesh_leaves + 3u * (size_t)base;
         const float3 pt = sim_inv_mul_pt(rot, ts, cell_pos);
         if (flat) {
             if (threadIdx.x == 0u) S.n_cand = 0u;
             __syncthreads();
         }
-        if (flat || wave == 0u) {
+        if (search == MESH_WALK) {
+            if (threadIdx.x == 0u) S.n_cand = SLOSH_NONE;
+        } else if (flat || wave == 0u) {
             // The block's box in the mesh's frame, from its first node.
             const float3 w0 = make_float3(__shfl(cell_pos.x, 0), __shfl(cell_pos.y, 0), __shfl(cell_pos.z, 0));
             const float3 c = sim_inv_mul_pt(rot, ts, make_float3(w0.x + cap, w0.y + cap, w0.z + cap));
@@ -1871,25 +1892,61 @@ __device__ inline void mesh_queries(const Colliders &cs, const float4 *box, Mesh
             else mesh_candidates(S, node, c, e, reach);
         }
         __syncthreads();
+        // Nodes that are walked: 4 x 2 of them per wave (side by side, so that they visit much
+        // the same).
+        const bool mine = lane >> 3 == wave;
         const uint32_t n = S.n_cand;
         if (n > MESH_CAND) {
-            if (wave == 0u && on) {
-                const uint32_t lf = trimesh_walk(node, leaf, count, pt, cap);
-                if (lf != SLOSH_NONE) S.key[i][lane] = (unsigned long long)~lf;
+            if (on && mine) {
+                const uint32_t lf = trimesh_walk(node, leaf, count, pt, cap, search != MESH_WALK);
+                if (lf != SLOSH_NONE) S.key[i][lane] = mesh_key(0.0f, lf);
             }
         } else {
-            // Every wave culls by the closest any of them has found so far.
+            // Every wave culls by the closest any of them has found so far. `eps`: above the
+            // rounding of distances between numbers of the mesh's size.
+            const float size = cs.mesh_size[i] + cap, eps = 3.0e-7f * size;
             volatile unsigned long long *closest = &S.key[i][lane];
             for (uint32_t q = wave; q < n; q += MESH_WAVES) {
                 const uint32_t lf = __builtin_amdgcn_readfirstlane(S.cand[q]);
                 const unsigned long long key = *closest;
-                const float best = key == ~0ull ? cap : __uint_as_float((uint32_t)(key >> 32));
+                const float best = key == ~0ull ? cap : key_distance(key) + eps;
                 if (on && box_distance(node[2u * lf], node[2u * lf + 1u], pt) <= best) {
                     float3 p;
                     uint32_t tri, feat, id;
-                    const float dist = leaf_distance(leaf + 3u * (size_t)lf, pt, &p, &tri, &feat, &id);
-                    const unsigned long long k = ((unsigned long long)__float_as_uint(dist) << 32) | (uint32_t)~lf;
-                    if (dist <= best && k < key) atomicMin(&S.key[i][lane], k);
+                    const float4 *lv = leaf + 3u * (size_t)lf;
+                    const float dist = leaf_distance(lv, pt, &p, &tri, &feat, &id);
+                    if (dist <= fminf(best, cap)) {
+                        const unsigned long long k = mesh_key(dist, lf);
+                        // What was the closest before: of waves that come at once, each sees
+                        // the one before it. (Its point may not be stored yet: then a node
+                        // counts as tied without need, and is walked to the same result.)
+                        const unsigned long long old = k < key ? atomicMin(&S.key[i][lane], k) : key;
+                        volatile float *px = &S.point[0][lane], *py = &S.point[1][lane], *pz = &S.point[2][lane];
+                        const float d = key_distance(old);  // (a NaN if there was none)
+                        if (fabsf(d - dist) <= eps &&
+                            fmaxf(fmaxf(fabsf(*px - p.x), fabsf(*py - p.y)), fabsf(*pz - p.z)) > eps) {
+                            if (fmaxf(leaf_box_distance(lv, pt),
+                                      leaf_box_distance(leaf + 3u * (size_t)key_leaf(old), pt)) >= dist - 2.0f * eps)
+                                atomicMin(&S.tie[lane], __float_as_uint(fminf(d, dist)));
+                        }
+                        if (k < old) {
+                            *px = p.x;
+                            *py = p.y;
+                            *pz = p.z;
+                        }
+                    }
+                }
+            }
+            __syncthreads();
+            if (on && mine) {
+                const unsigned long long key = *closest;
+                const float d = key_distance(key);
+                bool decide = __uint_as_float(S.tie[lane]) <= d + eps;
+                if (d + eps >= cap)
+                    decide = decide || leaf_box_distance(leaf + 3u * (size_t)key_leaf(key), pt) >= d - eps;
+                if (decide) {
+                    const uint32_t lf = trimesh_walk(node, leaf, count, pt, fminf(cap, d + 4.0f * eps), true);
+                    S.key[i][lane] = lf != SLOSH_NONE ? mesh_key(0.0f, lf) : ~0ull;
                 }
             }
         }
@@ -2839,7 +2896,8 @@ hipError_t launch_grid_update(const StepParams &P, const TransferBuffers &t, con
     cs.mesh_nodes = c.mesh_nodes;
     cs.mesh_leaves = c.mesh_leaves;
     cs.mesh_base = c.mesh_base;
-    cs.mesh_flat = c.mesh_base ? c.mesh_base + SLOSH_MAX_COLLIDERS : nullptr;
+    cs.mesh_search = c.mesh_base ? c.mesh_base + SLOSH_MAX_COLLIDERS : nullptr;
+    cs.mesh_size = c.mesh_base ? (const float *)(c.mesh_base + 2 * SLOSH_MAX_COLLIDERS) : nullptr;
     ItemLists items;
     items.items = t.items;
     items.rsum = t.rsum;

@@ -71,8 +71,8 @@ struct ColliderBuffers {
     const float4 *mesh_vtx;    // trimesh collision vertices (x, y, z, pad)
     const uint32_t *mesh_idx;  // trimesh collision indices
     // Per node of every trimesh body: its box, entry and exit (2 float4), and a leaf's
-    // triangle and its index (3 float4); per collider its first node, then per collider
-    // whether its leaves may be taken without a walk (MESH_FLAT nodes at most).
+    // triangle and its index (3 float4); per collider its first node, then per
+    // collider how its closest triangles are found (MESH_*) and its largest coordinate.
     const float4 *mesh_nodes, *mesh_leaves;
     const uint32_t *mesh_base;
 };

@@ -30,6 +30,7 @@
 #include <cstdio>
 #include <cstring>
 #include <deque>
+#include <limits>
 #include <memory>
 #include <mutex>
 #include <string>
@@ -1991,42 +1992,79 @@ void slosh_graph_destroy(slosh_graph *g) {
     delete g;
 }
 
-// The trimesh bodies' BVHs in the layout of the grid update's walk: per node its box
-// with the entry link (all ones: a leaf) and the exit link in the spare components,
-// and for a leaf its triangle's vertices with the triangle index. A leaf's box is that
-// of its triangle (the reference never reads a leaf's own), grown by 1 % of its extent
-// and well above the rounding of its coordinates.
-// Whether a walk of the BVH visits every leaf whose triangle is near: each node's box
-// holds the triangles of the leaves below it, and every leaf is below the first node. Then
-// the leaves of a small mesh are tested directly.
-static bool walk_reaches_all(const float *vertices4, const uint32_t *indices, size_t vroot, size_t iroot,
-                             size_t count) {
-    size_t leaves = 0, reached = 0;
-    std::vector<size_t> open;  // nodes above the current one
-    for (size_t k = 0; k < count; k++) leaves += indices[iroot + 3 * k] == 0xffffffffu;
+// Whether the walk of a BVH (trimesh_walk, from any point) finds the closest of its
+// triangles, rounding aside, and all of them can be found by the tree's levels: each node's
+// children follow one another up to its exit, its box holds the triangles below it, and no
+// triangle is so thin that the projection on it may end in the degenerate case (the point
+// itself, at distance 0). `leaves`: whether every leaf is below the first node as well, so
+// that all may be taken without the tree. `h`: the cell width.
+static bool walk_finds_closest(const float *vertices4, const uint32_t *indices, size_t vroot, size_t iroot,
+                               size_t count, float h, bool *leaves) {
+    struct Open {
+        size_t node;
+        float lo[3], hi[3];  // of the triangles below it so far
+    };
+    std::vector<Open> open;
+    const float inf = std::numeric_limits<float>::infinity();
+    auto enclose = [&](const float *lo, const float *hi) {  // in the innermost open node
+        if (open.empty()) return;
+        for (int c = 0; c < 3; c++) {
+            open.back().lo[c] = std::min(open.back().lo[c], lo[c]);
+            open.back().hi[c] = std::max(open.back().hi[c], hi[c]);
+        }
+    };
+    auto close = [&] {
+        const Open n = open.back();
+        open.pop_back();
+        const float *mn = vertices4 + 4 * (vroot + 2 * n.node), *mx = mn + 4;
+        for (int c = 0; c < 3; c++)
+            if (n.lo[c] <= n.hi[c] && !(mn[c] <= n.lo[c] && n.hi[c] <= mx[c])) return false;
+        enclose(n.lo, n.hi);
+        return true;
+    };
+    size_t all = 0, reached = 0;
+    for (size_t k = 0; k < count; k++) all += indices[iroot + 3 * k] == 0xffffffffu;
     for (size_t k = 0; k < count;) {
         const uint32_t *nd = indices + iroot + 3 * k;
-        while (!open.empty() && indices[iroot + 3 * open.back() + 1] <= k) open.pop_back();
+        while (!open.empty() && indices[iroot + 3 * open.back().node + 1] <= k)
+            if (!close()) return false;
+        if (!open.empty() && nd[1] > indices[iroot + 3 * open.back().node + 1]) return false;
         if (nd[0] != 0xffffffffu) {
-            open.push_back(k);
+            open.push_back({k, {inf, inf, inf}, {-inf, -inf, -inf}});
             k = nd[0];
             continue;
         }
         reached++;
         const uint32_t *t = indices + iroot + 3 * count + 3 * nd[2];
-        for (size_t up : open) {
-            const float *mn = vertices4 + 4 * (vroot + 2 * up), *mx = mn + 4;
-            for (int j = 0; j < 3; j++)
-                for (int c = 0; c < 3; c++) {
-                    const float x = vertices4[4 * (vroot + 2 * count + t[j]) + c];
-                    if (!(x >= mn[c] && x <= mx[c])) return false;
-                }
+        float lo[3], hi[3], e[2][3], longest = 0.0f;
+        const float *v[3];
+        for (int j = 0; j < 3; j++) v[j] = vertices4 + 4 * (vroot + 2 * count + t[j]);
+        for (int c = 0; c < 3; c++) {
+            lo[c] = std::min({v[0][c], v[1][c], v[2][c]});
+            hi[c] = std::max({v[0][c], v[1][c], v[2][c]});
+            longest = std::max(longest, hi[c] - lo[c]);
+            for (int j = 0; j < 2; j++) e[j][c] = v[j + 1][c] - v[0][c];
         }
+        const float n[3] = {e[0][1] * e[1][2] - e[0][2] * e[1][1], e[0][2] * e[1][0] - e[0][0] * e[1][2],
+                            e[0][0] * e[1][1] - e[0][1] * e[1][0]};
+        // Its numerators cancel to rounding (6e-8) of edge times distance to the point, which
+        // is a few cells at most.
+        if (!(std::sqrt(n[0] * n[0] + n[1] * n[1] + n[2] * n[2]) > 1.0e-5f * longest * std::max(longest, 10.0f * h)))
+            return false;
+        enclose(lo, hi);
         k = nd[1];
     }
-    return reached == leaves;
+    while (!open.empty())
+        if (!close()) return false;
+    *leaves = reached == all;
+    return true;
 }
 
+// The trimesh bodies' BVHs in the layout of the grid update: per node its box with the
+// entry link (all ones: a leaf) and the exit link in the spare components, and for a leaf
+// its triangle's vertices with the triangle's index. A leaf's box is that of its triangle (the
+// walk never reads a leaf's own), grown by 1 % of its extent and well above the rounding of
+// its coordinates.
 struct PackedMeshes {
     std::vector<float4> nodes, leaves;
     std::vector<uint32_t> base;
@@ -2035,13 +2073,19 @@ struct PackedMeshes {
 static void pack_meshes(const slosh_data *d, const float *vertices4, const uint32_t *indices, PackedMeshes &out) {
     std::vector<float4> &nodes = out.nodes, &leaves = out.leaves;
     std::vector<uint32_t> &base = out.base;
-    base.assign(2 * SLOSH_MAX_COLLIDERS, 0u);
+    base.assign(3 * SLOSH_MAX_COLLIDERS, 0u);
     for (uint32_t b = 0; b < d->nbodies; b++) {
         const slosh_shape &sh = d->bodies_host[b].shape;
         if (f2u(sh.a[3]) != 6u) continue;
         const size_t vroot = f2u(sh.a[0]), iroot = f2u(sh.a[1]), count = f2u(sh.a[2]);
         base[b] = (uint32_t)(nodes.size() / 2);
-        base[SLOSH_MAX_COLLIDERS + b] = count <= MESH_FLAT && walk_reaches_all(vertices4, indices, vroot, iroot, count);
+        bool flat = false;
+        base[SLOSH_MAX_COLLIDERS + b] = !walk_finds_closest(vertices4, indices, vroot, iroot, count, d->h, &flat) ? MESH_WALK
+                                        : flat && count <= MESH_FLAT_NODES                                    ? MESH_FLAT
+                                                                                                              : MESH_LEVELS;
+        float largest = 0.0f;  // (the first box holds every triangle)
+        for (int c = 0; c < 8; c++) largest = std::max(largest, c % 4 < 3 ? std::fabs(vertices4[4 * vroot + c]) : 0.0f);
+        base[2 * SLOSH_MAX_COLLIDERS + b] = f2u(largest);
         for (size_t k = 0; k < count; k++) {
             const uint32_t *nd = indices + iroot + 3 * k;
             const float *mn = vertices4 + 4 * (vroot + 2 * k), *mx = mn + 4;
