@@ -2030,12 +2030,14 @@ __global__ __launch_bounds__(MESH ? 64 * MESH_WAVES : 64) void k_grid_update(Ste
         if (owner) {
             const BlockRange br = M.fast ? block_range<true>(M, hid) : block_range<false>(M, hid);
             const uint32_t n = item_count(br), r = hid >> L.rshift;
+            // (Where its particles begin; a block without any, where its region's do.)
+            uint32_t start = r ? __builtin_amdgcn_readlane(up_p, r - 1u) : 0u;
             if (n) {
-                uint32_t item0, start;
+                uint32_t item0;
                 if (mode == 0) {
                     const uint2 rel = L.rel[hid];
                     item0 = rel.y + (r ? __builtin_amdgcn_readlane(up_i, r - 1u) : 0u);
-                    start = M.fast ? rel.x + (r ? __builtin_amdgcn_readlane(up_p, r - 1u) : 0u) : M.blk_start[hid];
+                    start = M.fast ? start + rel.x : M.blk_start[hid];
                 } else {
                     // A hook did P2G after a full sort: the items in order of arrival (their
                     // count was cleared by the sort).
@@ -2044,7 +2046,6 @@ __global__ __launch_bounds__(MESH ? 64 * MESH_WAVES : 64) void k_grid_update(Ste
                     item0 = __builtin_amdgcn_readfirstlane(at);
                     start = M.blk_start[hid];
                 }
-                if (M.fast && lane == 0u) L.blk_start[hid] = start;
                 // Four items at a time, a word per lane.
                 const uint32_t w = lane & 15u;
                 uint32_t v = (uint32_t)__shfl((int)nb, (int)w);
@@ -2060,6 +2061,7 @@ __global__ __launch_bounds__(MESH ? 64 * MESH_WAVES : 64) void k_grid_update(Ste
                     L.items[(size_t)(item0 + c) * ITEM_WORDS + w] = w == ITEM_FIRST ? 64u * c : v;
             }
             if (lane == 0u) {
+                if (M.fast) L.blk_start[hid] = start;
                 L.taken[hid] = 0u;
                 L.stay[hid] = 0u;
             }
