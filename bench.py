@@ -47,19 +47,30 @@ HBM_PEAK_GBS = 8000.0
 
 
 def pass_bytes(n, n_blk, n_dp=0):
-    """Algorithmic HBM bytes per launch of each pass (FP32 fields, each moved once):
-    grid_sort: block key write + read, 8 B/particle;
+    """Algorithmic HBM bytes per launch of each pass (FP32 fields, each moved once; a
+    steady-state substep launches no sort):
     p2g: read x, v, m, C (64 B/particle) + write 64 nodes x 16 B per block;
     grid_update: read + write 64 nodes x 16 B per block;
     g2p (fused with the particle update): read x, m, F, V0, tag, lambda, mu (68 B)
       and write x, v, C, F, force_dt (108 B) per particle + read 64 nodes x 16 B
       per block; Drucker-Prager particles add 16 B of parameters and 12 + 12 B of state."""
     return {
-        "grid_sort": 8.0 * n,
         "p2g": 64.0 * n + 1024.0 * n_blk,
         "grid_update": 2048.0 * n_blk,
         "g2p": 176.0 * n + 40.0 * n_dp + 1024.0 * n_blk,
     }
+
+
+def pass_times(per_pass, nbytes):
+    """Mean time, launches and bandwidth of the timed passes. The sort is left out: in a
+    steady-state substep an empty kernel stands for it while passes are timed."""
+    passes = {k: {"mean_us": 1e3 * v[0] / max(v[1], 1), "launches": v[1]} for k, v in per_pass.items()
+              if v[1] and k != "grid_sort"}
+    for k, v in passes.items():
+        if k in nbytes:
+            v["alg_bytes"] = nbytes[k]
+            v["GBps"] = nbytes[k] / (v["mean_us"] * 1e-6) / 1e9
+    return passes
 
 
 def measured_traffic(workload, pass_name, tuning):
@@ -156,17 +167,11 @@ def run_plain(args):
     per_pass = ts.read()
     data.check_errors(st)
     nbytes = pass_bytes(n, n_blk)
-    passes = {k: {"mean_us": 1e3 * v[0] / max(v[1], 1), "launches": v[1]} for k, v in per_pass.items() if v[1]}
-    for k, v in passes.items():
-        if k in nbytes:
-            v["alg_bytes"] = nbytes[k]
-            v["GBps"] = nbytes[k] / (v["mean_us"] * 1e-6) / 1e9
-    # The dominant kernel: the grid-sort pass is a chain of short kernels (each far
-    # below the single-kernel passes), so the candidates are P2G, the grid update
-    # and G2P + particle update.
-    dom = max((k for k in passes if k in nbytes and k != "grid_sort"), key=lambda k: passes[k]["mean_us"])
+    passes = pass_times(per_pass, nbytes)
+    # The dominant kernel: P2G, the grid update or G2P + particle update.
+    dom = max((k for k in passes if k in nbytes), key=lambda k: passes[k]["mean_us"])
     achieved = passes[dom]["GBps"]
-    timed_ms = sum(v[0] for v in per_pass.values()) / rsteps
+    timed_ms = sum(v["mean_us"] * v["launches"] for v in passes.values()) * 1e-3 / rsteps
     line = {
         "metric": METRIC,
         "value": value,
@@ -250,12 +255,8 @@ def run_batched(args):
     tags = batch.particles["models"][:, 0]
     n_dp = int(np.count_nonzero((tags == 2) | (tags == 3)))
     nbytes = pass_bytes(batch.n, n_blk, n_dp)
-    passes = {k: {"mean_us": 1e3 * v[0] / max(v[1], 1), "launches": v[1]} for k, v in per_pass.items() if v[1]}
-    for k, v in passes.items():
-        if k in nbytes:
-            v["alg_bytes"] = nbytes[k]
-            v["GBps"] = nbytes[k] / (v["mean_us"] * 1e-6) / 1e9
-    dom = max((k for k in passes if k in nbytes and k != "grid_sort"), key=lambda k: passes[k]["mean_us"])
+    passes = pass_times(per_pass, nbytes)
+    dom = max((k for k in passes if k in nbytes), key=lambda k: passes[k]["mean_us"])
     out = {
         "workload": f"{len(scs)} scenes, {batch.n} particles (N log-uniform [2e3, 2e5]; NH / FC / DP)",
         "value": batched,
