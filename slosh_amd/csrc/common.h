@@ -39,7 +39,6 @@ __device__ __host__ inline uint32_t tile_index(uint32_t x, uint32_t y, uint32_t 
 // Counter slots of one substep's counter set (two sets alternate with the hash
 // tables so a substep can prepare the next one's).
 #define CTR_NUM_BLOCKS 0
-#define CTR_SORTED_ALLOC 1
 #define CTR_ERRORS 2
 #define CTR_OVERFLOW 4   // movers beyond a block's MOVER_CAP list slots
 #define CTR_ITEMS 5      // items of the fused G2P kernel
@@ -130,8 +129,8 @@ struct StepParams {
     // disabled particles since (it zeroes their mass): mass = enabled ? u_mass : 0.
     uint32_t mass_uniform;
     float u_mass;
-    // Launch shape (autotuned): particles staged in LDS per P2G round, threads per
-    // G2P/update workgroup, workgroups of the per-block kernels.
+    // Launch shape (autotuned): particles staged in LDS per P2G round, workgroups of the
+    // per-block kernels.
     uint32_t p2g_chunk, block_wgs;
 };
 

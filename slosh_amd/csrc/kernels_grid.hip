@@ -62,7 +62,6 @@ __global__ __launch_bounds__(256) void k_reset_table(uint32_t *__restrict__ keys
             reinterpret_cast<uint4 *>(cell_cnt)[s] = make_uint4(0u, 0u, 0u, 0u);
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         counters[CTR_NUM_BLOCKS] = 0u;
-        counters[CTR_SORTED_ALLOC] = 0u;
         counters[CTR_OVERFLOW] = 0u;
         counters[CTR_ITEMS] = 0u;
     }
@@ -119,7 +118,7 @@ struct BlockCounts {
 
 // Exclusive scan of the particle counts of all slots (cap a power of two up to INDEX_CAP)
 // by a workgroup of 256 threads, each with consecutive slots.
-__device__ inline void scan_slots(const BlockCounts &b, uint32_t cap, uint32_t *counters, uint32_t *wsum) {
+__device__ inline void scan_slots(const BlockCounts &b, uint32_t cap, uint32_t *wsum) {
     const uint32_t tid = threadIdx.x, wave = tid >> 6, lane = tid & 63u;
     const uint32_t each = cap > 256u ? cap >> 8 : 1u, lo = tid * each;
     uint32_t sum = 0u;
@@ -150,7 +149,6 @@ __device__ inline void scan_slots(const BlockCounts &b, uint32_t cap, uint32_t *
             at += b.blk_cnt[lo + k];
         }
     }
-    if (tid == 255u) counters[CTR_SORTED_ALLOC] = at;
 }
 
 template <uint32_t ITEMS>
@@ -205,7 +203,7 @@ __global__ __launch_bounds__(256) void k_block_list(const uint32_t *__restrict__
         return;
     }
     if (blockIdx.x == cmp_wgs + nbr_wgs) {
-        scan_slots(counts, cap, counters, wsum);
+        scan_slots(counts, cap, wsum);
         return;
     }
     const uint32_t s0 = ((blockIdx.x - cmp_wgs - nbr_wgs - 1u) * 4u + wave) * 16u;
@@ -382,14 +380,13 @@ __global__ __launch_bounds__(1024) void k_block_scan_tiles(const uint32_t *__res
 }
 
 __global__ __launch_bounds__(1024) void k_block_scan_top(uint32_t *__restrict__ tile_sums,
-                                                         uint32_t *__restrict__ counters) {
+                                                         const uint32_t *__restrict__ counters) {
     __shared__ uint32_t wsum[16];
     const uint32_t B = counters[CTR_NUM_BLOCKS];
     const uint32_t ntiles = (B + 4095u) / 4096u;
     uint32_t carry = 0;
     for (uint32_t base = 0; base < ntiles; base += 4096u)
         carry += scan_tile(nullptr, tile_sums, tile_sums, base, ntiles, carry, wsum);
-    if (threadIdx.x == 0) counters[CTR_SORTED_ALLOC] = carry;
 }
 
 __global__ __launch_bounds__(256) void k_block_scan_add(const uint32_t *__restrict__ blist,
@@ -470,7 +467,8 @@ hipError_t launch_grid_build(const GridBuffers &g, const float4 *pos, uint32_t n
         launch_kernel(nullptr, k_block_scan_tiles, dim3(tile_wgs + cell_wgs), dim3(1024), 0, stream,
                       (const uint32_t *)g.blist, (const uint32_t *)g.blk_cnt, g.blk_start, g.tile_sums,
                       (const uint32_t *)g.counters, tile_wgs, (const uint32_t *)g.cell_cnt, g.cell_start);
-        launch_kernel(nullptr, k_block_scan_top, dim3(1), dim3(1024), 0, stream, g.tile_sums, g.counters);
+        launch_kernel(nullptr, k_block_scan_top, dim3(1), dim3(1024), 0, stream, g.tile_sums,
+                      (const uint32_t *)g.counters);
         launch_kernel(nullptr, k_block_scan_add, dim3(min_u(div_up(cap, 256), 4096)), dim3(256), 0, stream,
                       (const uint32_t *)g.blist, g.blk_start, (const uint32_t *)g.tile_sums,
                       (const uint32_t *)g.counters);

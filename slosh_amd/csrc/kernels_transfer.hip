@@ -1366,7 +1366,6 @@ __device__ inline void finish_particle(const StepParams &P, bool ok, float mass,
 struct Members {
     uint32_t fast;
     const uint32_t *blist;                   // block list (header ids = table slots)
-    const uint32_t *nbr;                     // neighbour tables
     const uint4 *bin;                        // per block: its previous-table block's range (start, count) and
                                              // stayers, the movers it received
     const uint32_t *mlist;                   // the first MOVER_CAP of them
@@ -1673,14 +1672,17 @@ __device__ inline void finish_block(const StepParams &P, const SortInputs &in, c
 // slots, particles) to its tile, so what counts with many blocks is how many are
 // resident: 512 members per chunk hold four workgroups to a CU (35 KB of LDS, 128 VGPRs),
 // 384 let in five (106 VGPRs): 1M particles 43 -> 39 us, 48 scenes 101 -> 88, 2.1M in 42k
-// blocks 248 -> 206 (38.2, 84.5 and 201 by now; more waves per SIMD at 96 VGPRs gain nothing). Chunks of 256 or 192 take no fewer registers than that and more
-// rounds (2.1M: 204, 209; 1M: 42, 44).
+// blocks 248 -> 206 (36, 77 and 200 by now; more waves per SIMD at 96 VGPRs gain nothing).
+// Chunks of 256 or 192 take more rounds (by now: 1M 36, 42; 48 scenes 82, 79; 131k 15, 20),
+// which only the sparse blocks of the 2.1M do not have (203, 186).
 // While all blocks are resident at once, the longest one's latency counts instead: a
 // block of 512 then goes in one chunk (131k particles: 14.2 us against 15.3), and with a
 // CU for each, in six waves that halve its longest cells and its loads per thread (2k
 // particles 11.8 -> 9.7 us, 33k 12.2 -> 10.4, 80k 12.6 -> 12.2; but 131k 14.2 -> 16.6,
 // 2.1M 248 -> 437). The count of blocks is not known to the host; scenes have one (with
-// the empty neighbours) per 150 to 300 particles.
+// the empty neighbours) per 150 to 300 particles. Sprays of fewer have many more blocks and
+// would do better with three waves: the substep of 90k particles, 6 to a block 101 us
+// instead of 119, 2 to a block 244 instead of 312.
 #define P2G_SUB_N 98304u    // two sets of waves up to here
 #define P2G_WIDE_N 262144u  // chunks of 512 up to here
 
@@ -1989,7 +1991,6 @@ __device__ inline void reset_next_table(const NextTable &nt, uint32_t cap) {
     }
     if (i == 0u) {
         nt.counters[CTR_NUM_BLOCKS] = 0u;
-        nt.counters[CTR_SORTED_ALLOC] = 0u;
         nt.counters[CTR_OVERFLOW] = 0u;
     }
 }
@@ -2841,7 +2842,6 @@ static Members members_of(const TransferBuffers &t) {
     Members M;
     M.fast = t.fast;
     M.blist = t.blist;
-    M.nbr = t.nbr;
     M.bin = t.bin;
     M.mlist = t.mlist;
     M.ovf_slot = t.ovf_slot;
