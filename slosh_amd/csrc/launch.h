@@ -104,6 +104,10 @@ hipError_t launch_p2g(const StepParams &P, const ParticleBuffers &pb, uint32_t p
 hipError_t launch_grid_update(const StepParams &P, const TransferBuffers &t, const ColliderBuffers &c,
                               const NextTableBuffers &next, uint32_t mode, uint32_t do_update, const PassEvents *ev,
                               hipStream_t stream);
+// The BVH of one trimesh body (its `count` nodes' boxes and vertices at vtx, links and
+// triangles at idx) in the layout of the grid update: ColliderBuffers::mesh_nodes, mesh_leaves.
+hipError_t launch_pack_mesh(const float4 *vtx, const uint32_t *idx, uint32_t count, float4 *nodes, float4 *leaves,
+                            hipStream_t stream);
 hipError_t launch_g2p_update(const StepParams &P, const ParticleBuffers &in, const ParticleBuffers &out,
                              const StaticBuffers &s, uint32_t pcap, const TransferBuffers &t,
                              const NextTableBuffers &next, const BodyBuffers &bb, const PassEvents *ev,

@@ -2036,21 +2036,23 @@ static bool walk_finds_closest(const float *vertices4, const uint32_t *indices, 
         }
         reached++;
         const uint32_t *t = indices + iroot + 3 * count + 3 * nd[2];
-        float lo[3], hi[3], e[2][3], longest = 0.0f;
-        const float *v[3];
-        for (int j = 0; j < 3; j++) v[j] = vertices4 + 4 * (vroot + 2 * count + t[j]);
+        const float *va = vertices4 + 4 * (vroot + 2 * count + t[0]);
+        const float *vb = vertices4 + 4 * (vroot + 2 * count + t[1]);
+        const float *vc = vertices4 + 4 * (vroot + 2 * count + t[2]);
+        float lo[3], hi[3], ab[3], ac[3], longest = 0.0f;
         for (int c = 0; c < 3; c++) {
-            lo[c] = std::min({v[0][c], v[1][c], v[2][c]});
-            hi[c] = std::max({v[0][c], v[1][c], v[2][c]});
+            lo[c] = std::min(std::min(va[c], vb[c]), vc[c]);
+            hi[c] = std::max(std::max(va[c], vb[c]), vc[c]);
             longest = std::max(longest, hi[c] - lo[c]);
-            for (int j = 0; j < 2; j++) e[j][c] = v[j + 1][c] - v[0][c];
+            ab[c] = vb[c] - va[c];
+            ac[c] = vc[c] - va[c];
         }
-        const float n[3] = {e[0][1] * e[1][2] - e[0][2] * e[1][1], e[0][2] * e[1][0] - e[0][0] * e[1][2],
-                            e[0][0] * e[1][1] - e[0][1] * e[1][0]};
-        // Its numerators cancel to rounding (6e-8) of edge times distance to the point, which
-        // is a few cells at most.
-        if (!(std::sqrt(n[0] * n[0] + n[1] * n[1] + n[2] * n[2]) > 1.0e-5f * longest * std::max(longest, 10.0f * h)))
-            return false;
+        const double n[3] = {(double)ab[1] * ac[2] - (double)ab[2] * ac[1], (double)ab[2] * ac[0] - (double)ab[0] * ac[2],
+                             (double)ab[0] * ac[1] - (double)ab[1] * ac[0]};
+        // The projection's numerators cancel to rounding (6e-8) of edge times distance to the
+        // point, which is a few cells at most.
+        const double thin = 1.0e-5 * longest * std::max(longest, 10.0f * h);
+        if (!(n[0] * n[0] + n[1] * n[1] + n[2] * n[2] > thin * thin)) return false;
         enclose(lo, hi);
         k = nd[1];
     }
@@ -2060,67 +2062,29 @@ static bool walk_finds_closest(const float *vertices4, const uint32_t *indices, 
     return true;
 }
 
-// The trimesh bodies' BVHs in the layout of the grid update: per node its box with the
-// entry link (all ones: a leaf) and the exit link in the spare components, and for a leaf
-// its triangle's vertices with the triangle's index. A leaf's box is that of its triangle (the
-// walk never reads a leaf's own), grown by 1 % of its extent and well above the rounding of
-// its coordinates.
-struct PackedMeshes {
-    std::vector<float4> nodes, leaves;
-    std::vector<uint32_t> base;
-};
-
-static void pack_meshes(const slosh_data *d, const float *vertices4, const uint32_t *indices, PackedMeshes &out) {
-    std::vector<float4> &nodes = out.nodes, &leaves = out.leaves;
-    std::vector<uint32_t> &base = out.base;
+// What the grid update needs to know of the trimesh bodies besides the buffers: per collider
+// its first packed node, how its closest triangles are found (MESH_*) and its largest
+// coordinate; and the number of packed nodes.
+static size_t describe_meshes(const slosh_data *d, const float *vertices4, const uint32_t *indices,
+                              std::vector<uint32_t> &base) {
     base.assign(3 * SLOSH_MAX_COLLIDERS, 0u);
+    size_t nodes = 0;
     for (uint32_t b = 0; b < d->nbodies; b++) {
         const slosh_shape &sh = d->bodies_host[b].shape;
         if (f2u(sh.a[3]) != 6u) continue;
         const size_t vroot = f2u(sh.a[0]), iroot = f2u(sh.a[1]), count = f2u(sh.a[2]);
-        base[b] = (uint32_t)(nodes.size() / 2);
         bool flat = false;
+        base[b] = (uint32_t)nodes;
         base[SLOSH_MAX_COLLIDERS + b] = !walk_finds_closest(vertices4, indices, vroot, iroot, count, d->h, &flat) ? MESH_WALK
                                         : flat && count <= MESH_FLAT_NODES                                    ? MESH_FLAT
                                                                                                               : MESH_LEVELS;
         float largest = 0.0f;  // (the first box holds every triangle)
         for (int c = 0; c < 8; c++) largest = std::max(largest, c % 4 < 3 ? std::fabs(vertices4[4 * vroot + c]) : 0.0f);
         base[2 * SLOSH_MAX_COLLIDERS + b] = f2u(largest);
-        for (size_t k = 0; k < count; k++) {
-            const uint32_t *nd = indices + iroot + 3 * k;
-            const float *mn = vertices4 + 4 * (vroot + 2 * k), *mx = mn + 4;
-            float lo[3] = {mn[0], mn[1], mn[2]}, hi[3] = {mx[0], mx[1], mx[2]};
-            float4 v[3] = {};
-            if (nd[0] == 0xffffffffu) {
-                const uint32_t *t = indices + iroot + 3 * count + 3 * nd[2];
-                for (int j = 0; j < 3; j++) {
-                    const float *p = vertices4 + 4 * (vroot + 2 * count + t[j]);
-                    v[j] = make_float4(p[0], p[1], p[2], u2f(nd[2]));
-                    for (int c = 0; c < 3; c++) {
-                        lo[c] = j == 0 ? p[c] : std::min(lo[c], p[c]);
-                        hi[c] = j == 0 ? p[c] : std::max(hi[c], p[c]);
-                    }
-                }
-                float extent = 0.0f, size = 0.0f;
-                for (int c = 0; c < 3; c++) {
-                    extent = std::max(extent, hi[c] - lo[c]);
-                    size = std::max({size, std::fabs(lo[c]), std::fabs(hi[c])});
-                }
-                const float grow = 0.01f * extent + 1.0e-5f * size;
-                for (int c = 0; c < 3; c++) {
-                    lo[c] -= grow;
-                    hi[c] += grow;
-                }
-            }
-            nodes.push_back(make_float4(lo[0], lo[1], lo[2], u2f(nd[0])));
-            nodes.push_back(make_float4(hi[0], hi[1], hi[2], u2f(nd[1])));
-            leaves.insert(leaves.end(), v, v + 3);
-        }
+        nodes += count;
     }
-    nodes.resize(std::max<size_t>(nodes.size(), 2));
-    leaves.resize(std::max<size_t>(leaves.size(), 3));
+    return nodes;
 }
-
 
 int slosh_data_set_collision_mesh(slosh_data *d, const float *vertices4, size_t num_vertices,
                                   const uint32_t *indices, size_t num_indices) {
@@ -2160,9 +2124,10 @@ int slosh_data_set_collision_mesh(slosh_data *d, const float *vertices4, size_t 
     }
     // All of the new buffers, then the exchange: without memory for them the data keeps the
     // ones it has.
-    PackedMeshes packed;
+    std::vector<uint32_t> described;
+    size_t packed = 0;
     try {
-        pack_meshes(d, vertices4, indices, packed);
+        packed = describe_meshes(d, vertices4, indices, described);
     } catch (const std::bad_alloc &) {
         return fail(SLOSH_E_NO_MEMORY, "collision mesh");
     }
@@ -2171,9 +2136,18 @@ int slosh_data_set_collision_mesh(slosh_data *d, const float *vertices4, size_t 
     float4 *nodes = nullptr, *leaves = nullptr;
     int rc = upload(&vtx, vertices4, 4 * num_vertices);
     if (rc == SLOSH_OK) rc = upload(&idx, indices, num_indices);
-    if (rc == SLOSH_OK) rc = upload(&nodes, packed.nodes.data(), packed.nodes.size());
-    if (rc == SLOSH_OK) rc = upload(&leaves, packed.leaves.data(), packed.leaves.size());
-    if (rc == SLOSH_OK) rc = upload(&base, packed.base.data(), packed.base.size());
+    if (rc == SLOSH_OK) rc = upload(&base, described.data(), described.size());
+    if (rc == SLOSH_OK) rc = dalloc(&nodes, 2 * packed);
+    if (rc == SLOSH_OK) rc = dalloc(&leaves, 3 * packed);
+    for (uint32_t b = 0; b < d->nbodies && rc == SLOSH_OK; b++) {
+        const slosh_shape &sh = d->bodies_host[b].shape;
+        if (f2u(sh.a[3]) != 6u) continue;
+        const size_t vroot = f2u(sh.a[0]), iroot = f2u(sh.a[1]), count = f2u(sh.a[2]), at = described[b];
+        if (launch_pack_mesh((const float4 *)vtx + vroot, idx + iroot, (uint32_t)count, nodes + 2 * at, leaves + 3 * at,
+                             nullptr) != hipSuccess)
+            rc = fail(SLOSH_E_HIP, "packing a collision mesh");
+    }
+    if (rc == SLOSH_OK && hipStreamSynchronize(nullptr) != hipSuccess) rc = fail(SLOSH_E_HIP, "packing a collision mesh");
     if (rc == SLOSH_OK) {
         invalidate_graphs(d);
         std::swap(vtx, d->mesh_vtx);
