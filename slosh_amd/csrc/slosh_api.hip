@@ -1339,6 +1339,19 @@ static int ring_commit(slosh_data *d, size_t off, size_t need, hipStream_t st) {
 }
 
 // ---- readback staging ---------------------------------------------------------
+// The data's GPU as the thread's current one, for as long as this lives: a readback's
+// kernel and staging belong there, and host threads begin with the first GPU.
+struct DeviceScope {
+    int before = -1;
+    explicit DeviceScope(int device) {
+        int now = device;
+        if (hipGetDevice(&now) == hipSuccess && now != device && hipSetDevice(device) == hipSuccess) before = now;
+    }
+    ~DeviceScope() {
+        if (before >= 0) (void)hipSetDevice(before);
+    }
+};
+
 // Records leave the device through pinned memory in pieces, each copied to the
 // caller's (pageable) memory by one of a few host threads while the next is on its
 // way: a direct copy into pageable memory runs at 2.4 GB/s for 2 MiB and page-faults
@@ -1434,7 +1447,7 @@ static int download(slosh_data *d, const void *src, size_t bytes, void *dst, hip
         HIP_TRY(hipMemcpyAsync(stage + o, from + o, len, hipMemcpyDeviceToHost, st));
         HIP_TRY(hipEventRecord(d->read_done[k], st));
     }
-    std::vector<hipError_t> err(T, hipSuccess);
+    hipError_t err[4] = {hipSuccess, hipSuccess, hipSuccess, hipSuccess};
     auto work = [&](size_t t) {
         for (size_t k = t; k < pieces; k += T) {
             const size_t o = k * READ_PIECE, len = std::min(READ_PIECE, bytes - o);
@@ -1447,17 +1460,20 @@ static int download(slosh_data *d, const void *src, size_t bytes, void *dst, hip
             std::memcpy(to + o, stage + o, len);
         }
     };
-    std::vector<std::thread> workers;
-    std::vector<size_t> mine = {0};
+    // (T is 4 at most. What a thread that cannot be started would copy, this one does.)
+    std::thread workers[3];
+    bool started[4] = {};
     for (size_t t = 1; t < T; t++) {
         try {
-            workers.emplace_back(work, t);
+            workers[t - 1] = std::thread(work, t);
+            started[t] = true;
         } catch (...) {
-            mine.push_back(t);
         }
     }
-    for (size_t t : mine) work(t);
-    for (auto &w : workers) w.join();
+    for (size_t t = 0; t < T; t++)
+        if (!started[t]) work(t);
+    for (size_t t = 1; t < T; t++)
+        if (started[t]) workers[t - 1].join();
     HIP_TRY(hipStreamSynchronize(st));
     for (hipError_t e : err) HIP_TRY(e);
     return SLOSH_OK;
@@ -1477,9 +1493,9 @@ static GatherArgs current_particles(slosh_data *d) {
     return a;
 }
 
-// The same assembled on the host from a copy of the state, for a storage that a grid
-// overflow has left inconsistent: the last of an id's slots counts, an id without one
-// reads as zeros.
+// The same assembled on the host from a copy of the state, where no memory can be pinned,
+// and for a storage that a grid overflow has left inconsistent: the last of an id's slots
+// counts, an id without one reads as zeros.
 static int read_records_host(slosh_data *d, uint32_t kind, size_t rec, void *out, hipStream_t st) {
     Snapshot s;
     TRY(download_current(d, st, s));
@@ -1514,9 +1530,9 @@ static int read_records_host(slosh_data *d, uint32_t kind, size_t rec, void *out
 static int read_records(slosh_data *d, uint32_t kind, size_t rec, void *out, hipStream_t st) {
     const size_t n = d->n;
     if (n == 0) return SLOSH_OK;
+    const DeviceScope scope(d->device);
     std::lock_guard<std::mutex> lock(d->read_mu);
-    if (d->lost) return read_records_host(d, kind, rec, out, st);
-    TRY(reserve_read_staging(d, n * rec));
+    if (d->lost || reserve_read_staging(d, n * rec) != SLOSH_OK) return read_records_host(d, kind, rec, out, st);
     uint32_t *bad = nullptr;
     uint8_t *records = nullptr;
     HIP_TRY(hipHostGetDevicePointer((void **)&bad, d->read_host, 0));
@@ -2783,6 +2799,7 @@ int slosh_read_scene(slosh_data *d, slosh_stream stream, uint32_t scene_id, floa
     if (m == 0) return SLOSH_OK;
     if (m > max_count) return fail(SLOSH_E_INVALID, "output smaller than the scene");
     hipStream_t st = (hipStream_t)stream;
+    const DeviceScope scope(d->device);
     std::lock_guard<std::mutex> lock(d->read_mu);
     // Staging: the particle buffer the next substep writes (free between substeps).
     const PBufs &stg = d->pb[d->cur_p ^ 1];
