@@ -1195,8 +1195,10 @@ static int run_step(slosh_pipeline *pl, slosh_data *d, hipStream_t st, const slo
     cb.mesh_base = d->mesh_base;
     // (The launch prepares the fused G2P kernel's items as well, whoever does the rest.)
     const bool combine = K.grid_update || !p2g_by_hook;
-    HIP_TRY(launch_grid_update(P, t, cb, next, p2g_by_hook ? 1u : 0u, K.grid_update ? 1u : 0u,
-                               combine ? pass_events(ts, PASS_GRID_UPDATE, &pe) : nullptr, st));
+    const bool fused = K.builtin_transfers && K.particles_update && !(hooks && hooks->after_g2p);
+    if (combine || fused)
+        HIP_TRY(launch_grid_update(P, t, cb, next, p2g_by_hook ? 1u : 0u, K.grid_update ? 1u : 0u,
+                                   combine ? pass_events(ts, PASS_GRID_UPDATE, &pe) : nullptr, st));
     if (d->coll_cache) d->coll_prev_valid = 1;
     if (hooks && hooks->after_grid_update && hooks->after_grid_update(d, st, hs) != 0)
         return fail(SLOSH_E_HOOK, "after_grid_update hook failed");
